@@ -2303,82 +2303,145 @@ struct TempoEngine {
 // [S][N][2][d2][d2]
 // ---------------------------------------------------------------------------
 
-// w[a][i] = sum_j (P1 v[a])[j] Tin[j][i]   (Tin = identity when null)
+// One step of the dynamics in one launch:
+//   w[a][i]  = sum_j (P1 v[a])[j] Tin[j][i]            (Tin = identity when null)
+//   u[b][i]  = scale sum_a w[a][i] T[a][i][b]
+//   v'[b][o] = sum_p P2[o][p] sum_i u[b][i] Tout[i][p]  (Tout = identity when null)
+// and the readout rho[o] = sum_a cap[a] v[a][o] of the state before the step.
+// Workgroup x < ceil(B / 16) of system y produces 16 values of b: thread
+// (slice, b) sums the rows a = slice (mod 16) of its column, so that a step
+// is a chain of a few loads instead of A d2 of them and a bond of 61 already
+// fills four workgroups; the 16 partial sums meet by wavefront shuffles and
+// LDS. The rows are taken in chunks of kRows: the chunk's site entries are
+// loaded to registers first (16 per thread), then w of the chunk is formed in
+// LDS by the whole workgroup, once per workgroup instead of in a launch of its
+// own. The last workgroup x does the readout. A site entry (a, i, b) lies at
+// a tsa + i tsi + b tsb, so tensors handed over as [a][b][i] are read in place
+// (a thread's d2 entries are then consecutive) and device sites as [a][i][b].
+// D2 is the Liouville dimension (16 with d2 <= 16 for the general case), a
+// compile-time constant so that the accumulators are registers.
+// Bound by the latency of one launch and its chain of loads. 150 steps at bond
+// 61, d2 = 4, from host tensors: 5.9 ms a call, copies included, against
+// 30.7 ms with three launches a step (116 us in the one with a thread per b
+// and all rows in sequence) and the tensors reordered on the host.
+template <int D2>
 __global__ void __launch_bounds__(256)
-dyn_pre_kernel(const double2* v, int A, int d2, long vstride, const double2* P1,
-               long pstride, const double2* tin, double2* w) {
-  const int sys = blockIdx.y;
+dyn_step_kernel(const double2* v, const double2* T, int A, int d2, int B, long tsa, long tsi,
+                long tsb, long vstride, double scale, const double2* tin, const double2* tout,
+                const double2* P1, const double2* P2, long pstride, double2* vout,
+                const double2* cap, double2* rho, long rstride) {
+  constexpr int kPer = D2 <= 4 ? 4 : 1;        // rows per thread and chunk
+  constexpr int kRows = 16 * kPer;
+  __shared__ double2 sv[kRows * D2], sw[kRows * D2];
+  __shared__ double2 sp[D2 * D2];
+  __shared__ double2 red[4][16][D2];
+  const int tid = threadIdx.x, sys = blockIdx.y;
   v += sys * vstride;
-  w += sys * vstride;
-  P1 += sys * pstride;
-  const long total = (long)A * d2;
-  for (long e = blockIdx.x * 256L + threadIdx.x; e < total; e += (long)gridDim.x * 256) {
-    const int i = e % d2;
-    const long a = e / d2;
-    double2 acc = make_double2(0.0, 0.0);
-    for (int j = 0; j < d2; ++j) {
-      double2 pj = make_double2(0.0, 0.0);
-      for (int q = 0; q < d2; ++q) cfma(pj, P1[j * d2 + q], v[a * d2 + q]);
-      if (tin) cfma(acc, pj, tin[j * d2 + i]);
-      else if (j == i) acc = pj;
+  const int tiles = (B + 15) / 16;
+  if ((int)blockIdx.x == tiles) {
+    // readout of the state before the step
+    double2* pr = &red[0][0][0];               // 4 * D2 wavefront sums
+#pragma unroll
+    for (int o = 0; o < D2; ++o) {
+      double2 acc = make_double2(0.0, 0.0);
+      if (o < d2)
+        for (int a = tid; a < A; a += 256) cfma(acc, cap[a], v[(long)a * d2 + o]);
+      acc.x = wave_sum(acc.x);
+      acc.y = wave_sum(acc.y);
+      if ((tid & 63) == 0) pr[(tid >> 6) * D2 + o] = acc;
     }
-    w[e] = acc;
-  }
-}
-
-// u[b][i] = sum_a w[a][i] T[a][i][b] * scale; v'[b][o] = sum_i u[b][i] Tout[i][o]
-// then v''[b][o2] = sum_o P2[o2][o] v'[b][o].  One thread per b; the site is
-// read in its [a][i][b] layout (coalesced over b).
-__global__ void __launch_bounds__(256)
-dyn_mpo_kernel(const double2* w, const double2* T, int A, int d2, int B, long vstride,
-               double scale, const double2* tout, const double2* P2, long pstride,
-               double2* vout) {
-  const int b = blockIdx.x * 256 + threadIdx.x;
-  if (b >= B) return;
-  const int sys = blockIdx.y;
-  w += sys * vstride;
-  vout += sys * vstride;
-  P2 += sys * pstride;
-  double2 u[16];
-  for (int i = 0; i < d2; ++i) u[i] = make_double2(0.0, 0.0);
-  for (int a = 0; a < A; ++a)
-    for (int i = 0; i < d2; ++i)
-      cfma(u[i], w[(long)a * d2 + i], T[((long)a * d2 + i) * B + b]);
-  double2 vp[16];
-  for (int o = 0; o < d2; ++o) {
-    double2 acc = make_double2(0.0, 0.0);
-    for (int i = 0; i < d2; ++i) {
-      if (tout) cfma(acc, u[i], tout[i * d2 + o]);
-      else if (i == o) acc = u[i];
-    }
-    vp[o] = cscale(acc, scale);
-  }
-  for (int o2 = 0; o2 < d2; ++o2) {
-    double2 acc = make_double2(0.0, 0.0);
-    for (int o = 0; o < d2; ++o) cfma(acc, P2[o2 * d2 + o], vp[o]);
-    vout[(long)b * d2 + o2] = acc;
-  }
-}
-
-// rho[o] = sum_a cap[a] v[a][o]   (one workgroup per system)
-__global__ void __launch_bounds__(256)
-dyn_readout_kernel(const double2* v, const double2* cap, int A, int d2, long vstride,
-                   double2* rho, long rstride) {
-  __shared__ double2 red[256];
-  const int sys = blockIdx.y;
-  v += sys * vstride;
-  rho += sys * rstride;
-  for (int o = 0; o < d2; ++o) {
-    double2 acc = make_double2(0.0, 0.0);
-    for (int a = threadIdx.x; a < A; a += 256) cfma(acc, cap[a], v[(long)a * d2 + o]);
-    red[threadIdx.x] = acc;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if (threadIdx.x < s) red[threadIdx.x] = cadd(red[threadIdx.x], red[threadIdx.x + s]);
+    if (tid < d2)
+      rho[sys * rstride + tid] = cadd(cadd(pr[tid], pr[D2 + tid]),
+                                      cadd(pr[2 * D2 + tid], pr[3 * D2 + tid]));
+    return;
+  }
+  vout += sys * vstride;
+  P1 += sys * pstride;
+  P2 += sys * pstride;
+  const int bl = tid & 15, slice = tid >> 4;
+  const int b = blockIdx.x * 16 + bl;
+  const bool on = b < B;
+  const double2 zero = make_double2(0.0, 0.0);
+  double2 u[D2];
+#pragma unroll
+  for (int i = 0; i < D2; ++i) u[i] = zero;
+  if (tid < d2 * d2) sp[tid] = P1[tid];
+  for (int a0 = 0; a0 < A; a0 += kRows) {
+    double2 t[kPer][D2];
+#pragma unroll
+    for (int r = 0; r < kPer; ++r)
+#pragma unroll
+      for (int i = 0; i < D2; ++i) {
+        const int a = a0 + slice + 16 * r;
+        t[r][i] = (on && i < d2 && a < A) ? T[(long)a * tsa + i * tsi + (long)b * tsb] : zero;
+      }
+    const int rows = min(kRows, A - a0);
+    for (int e = tid; e < rows * d2; e += 256) sv[e] = v[(long)a0 * d2 + e];
+    __syncthreads();
+    for (int e = tid; e < rows * d2; e += 256) {
+      const int a = e / d2, j = e - a * d2;
+      double2 acc = zero;
+      for (int q = 0; q < d2; ++q) cfma(acc, sp[j * d2 + q], sv[a * d2 + q]);
+      sw[e] = acc;
+    }
+    __syncthreads();
+    if (tin) {
+      for (int e = tid; e < rows * d2; e += 256) {
+        const int a = e / d2, i = e - a * d2;
+        double2 acc = zero;
+        for (int j = 0; j < d2; ++j) cfma(acc, sw[a * d2 + j], tin[j * d2 + i]);
+        sv[e] = acc;
+      }
       __syncthreads();
     }
-    if (threadIdx.x == 0) rho[o] = red[0];
+    const double2* w = tin ? sv : sw;
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      const int a = slice + 16 * r;
+      if (a < rows) {
+#pragma unroll
+        for (int i = 0; i < D2; ++i)
+          if (i < d2) cfma(u[i], w[a * d2 + i], t[r][i]);
+      }
+    }
     __syncthreads();
+  }
+  // the 16 slices: four per wavefront (lanes 16 apart), then four wavefronts
+#pragma unroll
+  for (int i = 0; i < D2; ++i) {
+    u[i].x += __shfl_xor(u[i].x, 16, 64);
+    u[i].y += __shfl_xor(u[i].y, 16, 64);
+    u[i].x += __shfl_xor(u[i].x, 32, 64);
+    u[i].y += __shfl_xor(u[i].y, 32, 64);
+    if ((tid & 48) == 0) red[tid >> 6][bl][i] = u[i];
+  }
+  if (tid < d2 * d2) sp[tid] = P2[tid];
+  __syncthreads();
+  // sv, sw: [16][d2] (16 <= kRows)
+  if (tid < 16 * d2) {
+    const int bb = tid / d2, i = tid - bb * d2;
+    sv[tid] = cscale(cadd(cadd(red[0][bb][i], red[1][bb][i]),
+                          cadd(red[2][bb][i], red[3][bb][i])), scale);
+  }
+  __syncthreads();
+  if (tout) {
+    if (tid < 16 * d2) {
+      const int bb = tid / d2, o = tid - bb * d2;
+      double2 acc = zero;
+      for (int i = 0; i < d2; ++i) cfma(acc, sv[bb * d2 + i], tout[i * d2 + o]);
+      sw[tid] = acc;
+    }
+    __syncthreads();
+  }
+  const double2* x = tout ? sw : sv;
+  if (tid < 16 * d2) {
+    const int bb = tid / d2, o = tid - bb * d2, gb = blockIdx.x * 16 + bb;
+    if (gb < B) {
+      double2 acc = zero;
+      for (int q = 0; q < d2; ++q) cfma(acc, sp[o * d2 + q], x[bb * d2 + q]);
+      vout[(long)gb * d2 + o] = acc;
+    }
   }
 }
 
@@ -2566,13 +2629,14 @@ static void run_dynamics_multi(hipStream_t st, int d2, int N, const std::vector<
   HIP_CHECK(hipStreamSynchronize(st));
 }
 
-// Runs the dynamics of S systems over device-resident sites [a][i][b]
-// (scaled by `scale`) and caps; props: S x N x 2 x d2 x d2, rho0: S x d2,
-// states_out: S x (N+1) x d2 (interleaved complex).
+// Runs the dynamics of S systems over device-resident sites, [a][i][b] or,
+// when `past_future`, [a][b][i] (scaled by `scale`), and caps; props: S x N x
+// 2 x d2 x d2, rho0: S x d2, states_out: S x (N+1) x d2 (interleaved complex).
 static void run_dynamics(hipStream_t st, int d2, int N, const std::vector<const double2*>& sites,
                          const std::vector<int>& bonds, const std::vector<const double2*>& caps,
                          const double* props, const double* tin_h, const double* tout_h,
-                         const double* rho0, double scale, double* states_out, int S = 1) {
+                         const double* rho0, double scale, double* states_out, int S = 1,
+                         bool past_future = false) {
   require(d2 >= 1 && d2 <= 16, PTE_ERR_ARG, "Liouville dimension must be 1..16");
   require(S >= 1 && S <= 65535, PTE_ERR_ARG, "number of systems must be 1..65535");
   const long pstride = 2L * N * d2 * d2;      // per system, complex entries
@@ -2590,32 +2654,28 @@ static void run_dynamics(hipStream_t st, int d2, int N, const std::vector<const 
   int maxb = 1;
   for (int b : bonds) maxb = std::max(maxb, b);
   const long vstride = (long)maxb * d2, rstride = (long)(N + 1) * d2;
-  double2 *v = nullptr, *v2 = nullptr, *w = nullptr, *rho = nullptr;
+  double2 *v = nullptr, *v2 = nullptr, *rho = nullptr;
   HIP_CHECK(hipMallocAsync((void**)&v, (size_t)S * vstride * sizeof(double2), st));
   HIP_CHECK(hipMallocAsync((void**)&v2, (size_t)S * vstride * sizeof(double2), st));
-  HIP_CHECK(hipMallocAsync((void**)&w, (size_t)S * vstride * sizeof(double2), st));
   HIP_CHECK(hipMallocAsync((void**)&rho, (size_t)S * rstride * sizeof(double2), st));
   HIP_CHECK(hipMemcpy2DAsync(v, vstride * sizeof(double2), rho0, d2 * sizeof(double2),
                              d2 * sizeof(double2), S, hipMemcpyHostToDevice, st));
-  for (int k = 0; k < N; ++k) {
-    const int A = bonds[k], B = bonds[k + 1];
-    dyn_readout_kernel<<<dim3(1, S), 256, 0, st>>>(v, caps[k], A, d2, vstride,
-                                                   rho + (long)k * d2, rstride);
-    const double2* P1 = dprops + (long)k * 2 * d2 * d2;
-    const double2* P2 = P1 + d2 * d2;
-    dyn_pre_kernel<<<dim3(grid_for((long)A * d2), S), 256, 0, st>>>(v, A, d2, vstride, P1,
-                                                                    pstride, tin, w);
-    dyn_mpo_kernel<<<dim3((B + 255) / 256, S), 256, 0, st>>>(w, sites[k], A, d2, B, vstride,
-                                                             scale, tout, P2, pstride, v2);
+  auto step = d2 == 4 ? dyn_step_kernel<4> : d2 <= 9 ? dyn_step_kernel<9> : dyn_step_kernel<16>;
+  for (int k = 0; k <= N; ++k) {
+    // k = N: the readout alone (no b)
+    const int A = bonds[k], B = k < N ? bonds[k + 1] : 0;
+    const double2* P1 = dprops + (long)std::min(k, N - 1) * 2 * d2 * d2;
+    const long tsi = past_future ? 1 : B, tsb = past_future ? d2 : 1;
+    step<<<dim3((B + 15) / 16 + 1, S), 256, 0, st>>>(
+        v, k < N ? sites[k] : nullptr, A, d2, B, (long)B * d2, tsi, tsb, vstride, scale, tin,
+        tout, P1, P1 + d2 * d2, pstride, v2, caps[k], rho + (long)k * d2, rstride);
     std::swap(v, v2);
   }
-  dyn_readout_kernel<<<dim3(1, S), 256, 0, st>>>(v, caps[N], bonds[N], d2, vstride,
-                                                 rho + (long)N * d2, rstride);
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipMemcpyAsync(states_out, rho, (size_t)S * rstride * sizeof(double2),
                            hipMemcpyDeviceToHost, st));
   HIP_CHECK(hipStreamSynchronize(st));
-  (void)hipFreeAsync(v, st); (void)hipFreeAsync(v2, st); (void)hipFreeAsync(w, st); (void)hipFreeAsync(rho, st);
+  (void)hipFreeAsync(v, st); (void)hipFreeAsync(v2, st); (void)hipFreeAsync(rho, st);
   (void)hipFreeAsync(dprops, st);
   if (tin) (void)hipFreeAsync(tin, st);
   if (tout) (void)hipFreeAsync(tout, st);
@@ -3438,42 +3498,40 @@ int pte_dynamics_run(int d2, int num_steps, const int* bonds, const double* tens
             "null argument");
     require(num_steps >= 1, PTE_ERR_ARG, "num_steps must be >= 1");
     require(bonds[0] == 1, PTE_ERR_ARG, "the first bond must be 1");
+    std::vector<int> b(bonds, bonds + num_steps + 1);
+    for (int x : b) require(x >= 1, PTE_ERR_ARG, "bond dims must be positive");
+    require(d2 >= 1 && d2 <= 16, PTE_ERR_ARG, "Liouville dimension must be 1..16");
+    // tensors ([a][b][i], read in place by the kernel) and caps in one
+    // allocation and one copy each
+    std::vector<long> off(num_steps + 1, 0), coff(num_steps + 2, 0);
+    for (int k = 0; k < num_steps; ++k) off[k + 1] = off[k] + (long)b[k] * b[k + 1] * d2;
+    for (int k = 0; k <= num_steps; ++k) coff[k + 1] = coff[k] + b[k];
     hipStream_t st;
     HIP_CHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    std::vector<int> b(bonds, bonds + num_steps + 1);
-    std::vector<double2*> dsites(num_steps), dcaps(num_steps + 1);
-    long off = 0, coff = 0;
-    for (int k = 0; k < num_steps; ++k) {
-      require(b[k] >= 1 && b[k + 1] >= 1, PTE_ERR_ARG, "bond dims must be positive");
-      // tensors come as [a][b][i]; the kernel reads [a][i][b]
-      const long cnt = (long)b[k] * b[k + 1] * d2;
-      std::vector<cplx> h(cnt);
-      for (int a = 0; a < b[k]; ++a)
-        for (int bb = 0; bb < b[k + 1]; ++bb)
-          for (int i = 0; i < d2; ++i) {
-            const long src = off + ((long)a * b[k + 1] + bb) * d2 + i;
-            h[((long)a * d2 + i) * b[k + 1] + bb] = cplx(tensors[2 * src], tensors[2 * src + 1]);
-          }
-      HIP_CHECK(hipMallocAsync((void**)&dsites[k], cnt * sizeof(double2), st));
-      HIP_CHECK(hipMemcpyAsync(dsites[k], h.data(), cnt * sizeof(double2),
+    double2* dev = nullptr;
+    auto release = [&] {
+      (void)hipStreamSynchronize(st);
+      if (dev) (void)hipFreeAsync(dev, st);
+      (void)hipStreamSynchronize(st);
+      (void)hipStreamDestroy(st);
+    };
+    try {
+      const long nt = off[num_steps], nc = coff[num_steps + 1];
+      HIP_CHECK(hipMallocAsync((void**)&dev, (size_t)(nt + nc) * sizeof(double2), st));
+      HIP_CHECK(hipMemcpyAsync(dev, tensors, (size_t)nt * sizeof(double2),
                                hipMemcpyHostToDevice, st));
-      HIP_CHECK(hipStreamSynchronize(st));
-      off += cnt;
-    }
-    require(b[num_steps] >= 1, PTE_ERR_ARG, "bond dims must be positive");
-    for (int k = 0; k <= num_steps; ++k) {
-      HIP_CHECK(hipMallocAsync((void**)&dcaps[k], b[k] * sizeof(double2), st));
-      HIP_CHECK(hipMemcpyAsync(dcaps[k], caps + 2 * coff, b[k] * sizeof(double2),
+      HIP_CHECK(hipMemcpyAsync(dev + nt, caps, (size_t)nc * sizeof(double2),
                                hipMemcpyHostToDevice, st));
-      coff += b[k];
+      std::vector<const double2*> cs(num_steps), cc(num_steps + 1);
+      for (int k = 0; k < num_steps; ++k) cs[k] = dev + off[k];
+      for (int k = 0; k <= num_steps; ++k) cc[k] = dev + nt + coff[k];
+      run_dynamics(st, d2, num_steps, cs, b, cc, props, tin, tout, rho0, 1.0, states_out, 1,
+                   true);
+    } catch (...) {
+      release();
+      throw;
     }
-    std::vector<const double2*> cs(dsites.begin(), dsites.end());
-    std::vector<const double2*> cc(dcaps.begin(), dcaps.end());
-    run_dynamics(st, d2, num_steps, cs, b, cc, props, tin, tout, rho0, 1.0, states_out);
-    for (auto p : dsites) (void)hipFreeAsync(p, st);
-    for (auto p : dcaps) (void)hipFreeAsync(p, st);
-    HIP_CHECK(hipStreamSynchronize(st));
-    (void)hipStreamDestroy(st);
+    release();
   });
 }
 
