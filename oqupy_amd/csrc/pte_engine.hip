@@ -532,6 +532,10 @@ struct Workspace {
         &per_cu, reinterpret_cast<const void*>(jacobi_tile_kernel), 256,
         tile_lds_bytes(kTileMaxRows)));
     tile_coop_blocks = per_cu * num_cus;
+    for (const void* f : {reinterpret_cast<const void*>(gram_svd_kernel),
+                          reinterpret_cast<const void*>(gram_svd_batch_kernel)})
+      HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)gram_lds(kGramMaxRank)));
     if (const char* v = std::getenv("PTE_JACOBI_TILE")) tile_enabled = std::atoi(v) != 0;
     if (const char* v = std::getenv("PTE_JACOBI_TILE_ROWS"))
       tile_rows = std::max(32, std::min(kTileMaxRows, std::atoi(v)));
@@ -783,7 +787,7 @@ struct Workspace {
     trunc_extra2 = folded ? rank->out_d : nullptr;
     int k;
     try {
-      k = svd(n, r);
+      k = gram_ok(r) ? svd_gram(n, r) : svd(n, r);
     } catch (...) {
       trunc_extra2 = nullptr;
       throw;
@@ -838,21 +842,42 @@ struct Workspace {
     return *qr_rank_h;
   }
 
-  // ---- small SVDs: one workgroup, LDS resident (small_svd_kernel) ----
-  // dynamic LDS of small_svd_kernel: 160 KiB less 1 KiB for its static part
+  // ---- SVDs whose Jacobi runs on the Gram matrix in one workgroup ----
+  // dynamic LDS of small_svd_kernel and gram_svd_kernel: 160 KiB less 1 KiB
+  // for their static part
   static constexpr size_t kSmallLdsMax = 159 * 1024;
-  // the QR phase needs M and 64 bytes per column; the Jacobi phase Y
-  // (n x r) and, when it fits, W (r x r), r <= min(m, n); the epilogue Y and
-  // two r-vectors
+  // the Gram Jacobi needs the 2 x 2 blocks of the Hermitian half, 64 rotations
+  // and three r-vectors
+  static size_t gram_lds(int r) {
+    const size_t pairs = (size_t)(r + 1) / 2;
+    return pairs * (pairs + 1) / 2 * 64 + 64 * 24 + (size_t)r * 24;
+  }
+  // small_svd_kernel's QR phase needs M and 64 bytes per column; then Y (n x r
+  // with an odd leading dimension), then the Gram Jacobi, r <= min(m, n)
   static size_t small_qr_lds(int m, int n) { return (size_t)m * n * 16 + (size_t)n * 64; }
   static size_t small_lds(int m, int n) {
-    const size_t r = (size_t)std::min(m, n);
-    return std::max({small_qr_lds(m, n), (size_t)n * r * 16 + r * 16,
-                     std::min(kSmallLdsMax, ((size_t)n * r + r * r) * 16)});
+    const int r = std::min(m, n);
+    return std::max({small_qr_lds(m, n), (size_t)(n | 1) * r * 16, gram_lds(r)});
   }
   bool small_ok(int m, int n) const {
     return small_enabled && n <= kSmallMaxCols && small_qr_lds(m, n) <= kSmallLdsMax;
   }
+
+  // Rotation log of a Gram Jacobi of rank at most r (in gpart, which the
+  // blocked Jacobi uses otherwise): 64 complex and 64 real entries per round.
+  void gram_log(int r, double2** logs, double** logc) {
+    const size_t rounds = (size_t)kGramMaxSweeps * std::max(1, r + (r & 1) - 1);
+    gpart.ensure(rounds * 96, svd_stream);
+    *logs = gpart.p;
+    *logc = reinterpret_cast<double*>(gpart.p + rounds * 64);
+  }
+
+  GramReplayArgs replay_args(int n, const double* logc, const double2* logs) const {
+    GramReplayArgs ra;
+    ra.Y = X.p; ra.n = n; ra.W = V.p; ra.info = info_d; ra.logc = logc; ra.logs = logs;
+    return ra;
+  }
+  static unsigned replay_grid(int n, int r) { return (unsigned)((n + r + 3) / 4); }
 
   // buffers and arguments of small_svd_kernel on Q (m x n)
   SmallSvdArgs small_prepare(int m, int n, SvdInfo* copy) {
@@ -866,41 +891,104 @@ struct Workspace {
     sa.A = Q.p; sa.m = m; sa.n = n;
     sa.tau = qr_tau; sa.vscale = qr_vscale; sa.beta = qr_beta; sa.piv = qr_piv;
     sa.qrank = qr_rank_d;
-    sa.Y = X.p; sa.W = V.p;
+    sa.Y = X.p;
     sa.sigma = sigma; sa.perm = perm; sa.sorted = sorted; sa.info = info_d;
-    sa.epsrel = epsrel; sa.max_rank = chi_cap; sa.max_sweeps = max_sweeps;
+    sa.epsrel = epsrel; sa.max_rank = chi_cap;
+    sa.max_sweeps = std::min(max_sweeps, kGramMaxSweeps);
     sa.copy = copy;
     sa.stop_rel = 0.0;
-    sa.lds_bytes = (long)small_lds(m, n);
+    sa.folded = nullptr;
+    gram_log(rmax, &sa.logs, &sa.logc);
     return sa;
   }
 
   // after synchronisation (summary in info_h): the same checks, statistics
   // and state as the pivoted-QR + Jacobi path
   int small_finish(int m, int n, float ms) {
+    small_state(m, n);
+    return jacobi_check(n, qr_r, ms, true);
+  }
+  void small_state(int m, int n) {
     const int r = info_h->pad;
     require(r >= 1, PTE_ERR_NUMERIC, "SVD of a zero matrix");
     qr_count += 1;
     tr_m = m; tr_n = n; tr_r = r; tr_qr_ms = 0.f;
     qr_m = m; qr_n = n; qr_r = r;
-    return jacobi_check(n, r, ms, true);
   }
 
   // `adaptive`: the learned form's adaptive stop of the QR (its residual
   // counted in the cut)
   int svd_small(int m, int n, bool adaptive = false) {
     SmallSvdArgs sa = small_prepare(m, n, nullptr);
-    if (adaptive) sa.stop_rel = rank->theta * epsrel;
+    if (adaptive) {
+      sa.stop_rel = rank->theta * epsrel;
+      sa.folded = rank->out_d;
+    }
     // timed (two event records on the stream) only for the SVD trace
     const bool timed = trace != nullptr;
     if (timed) mark(evj0);
     small_svd_kernel<<<1, kSmallThreads, small_lds(m, n), svd_stream>>>(sa);
+    gram_replay_kernel<<<replay_grid(n, std::min(m, n)), 256, 0, svd_stream>>>(
+        replay_args(n, sa.logc, sa.logs));
     if (timed) mark(evj1);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipMemcpyAsync(info_h, info_d, sizeof(SvdInfo), hipMemcpyDeviceToHost,
                              svd_stream));
     HIP_CHECK(hipStreamSynchronize(svd_stream));
+    if (info_h->sweeps < 0) {
+      // not converged within the log: Y is untouched, the blocked Jacobi
+      // takes it
+      small_state(m, n);
+      trunc_extra2 = adaptive ? rank->out_d : nullptr;
+      int k;
+      try {
+        k = svd(n, qr_r);
+      } catch (...) {
+        trunc_extra2 = nullptr;
+        throw;
+      }
+      trunc_extra2 = nullptr;
+      return k;
+    }
     return small_finish(m, n, timed ? elapsed(evj0, evj1) : 0.f);
+  }
+
+  // Y of at most kGramMaxRank columns, from a pivoted QR (the method relies
+  // on its graded rows); beyond, G does not fit one workgroup. Both sides at
+  // ranks 64 to 126 of the TEMPO and PT-TEMPO runs: 0.41 ms on average here,
+  // 0.9 ms in the blocked Jacobi.
+  bool gram_ok(int r) const { return small_enabled && r <= kGramMaxRank; }
+
+  GramSvdArgs gram_prepare(int n, int r, SvdInfo* copy) {
+    ensure_sv((size_t)r);
+    V.ensure((size_t)r * r, svd_stream);
+    GramSvdArgs ga;
+    ga.Y = X.p; ga.n = n; ga.r = r;
+    ga.sigma = sigma; ga.perm = perm; ga.sorted = sorted; ga.info = info_d;
+    ga.epsrel = epsrel; ga.max_rank = chi_cap;
+    ga.max_sweeps = std::min(max_sweeps, kGramMaxSweeps);
+    ga.copy = copy;
+    ga.extra2 = trunc_extra2;
+    gram_log(r, &ga.logs, &ga.logc);
+    return ga;
+  }
+
+  // Jacobi SVD of Y = R^H (n x r, in X) after the pivoted QR, as svd(n, r)
+  int svd_gram(int n, int r) {
+    GramSvdArgs ga = gram_prepare(n, r, nullptr);
+    const bool timed = trace != nullptr;
+    if (timed) mark(evj0);
+    gram_svd_kernel<<<1, 1024, gram_lds(r), svd_stream>>>(ga);
+    gram_replay_kernel<<<replay_grid(n, r), 256, 0, svd_stream>>>(
+        replay_args(n, ga.logc, ga.logs));
+    if (timed) mark(evj1);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipMemcpyAsync(info_h, info_d, sizeof(SvdInfo), hipMemcpyDeviceToHost,
+                             svd_stream));
+    HIP_CHECK(hipStreamSynchronize(svd_stream));
+    // not converged within the log: Y is untouched
+    if (info_h->sweeps < 0) return svd(n, r);
+    return jacobi_check(n, r, timed ? elapsed(evj0, evj1) : 0.f, true);
   }
 
   int qr_natural_grid(int n) const { return std::max(1, std::min({n, qr_blocks, num_cus})); }
@@ -1038,10 +1126,12 @@ struct Workspace {
 // Batched truncated SVDs for many engines stepped together (one host thread
 // per engine). An engine thread that reaches an SVD posts a request and
 // waits; when every running thread has posted (or left), the last one to
-// arrive serves all requests at once on the batch stream: one cooperative
-// launch of qrcp_batch_kernel for the pivoted QRs, one of
-// jacobi_batch_kernel for the Jacobi SVDs, each workgroup working on one
-// request with that request's own barrier counter. Requests that do not fit
+// arrive serves all requests at once on the batch stream: one launch for the
+// SVDs done by one workgroup each (small_svd_batch_kernel), one cooperative
+// launch of qrcp_batch_kernel for the pivoted QRs of the others, one launch
+// for the Gram Jacobi of those of rank up to kGramMaxRank and one of
+// jacobi_batch_kernel for the rest, each workgroup of a cooperative launch
+// working on one request with that request's own barrier counter. Requests that do not fit
 // the co-resident grid together go into several launches.
 // ---------------------------------------------------------------------------
 struct SvdRequest {
@@ -1267,29 +1357,83 @@ struct Batcher {
     gather_cap = c;
   }
 
-  // small SVDs: one workgroup each, all in one launch
-  void run_small(std::vector<SvdRequest*>& rs) {
+  // small SVDs: one workgroup each, all in one launch, and their replays in
+  // another; a request that did not converge goes to `blocked`
+  void run_small(std::vector<SvdRequest*>& rs, std::vector<SvdRequest*>* blocked) {
     ensure_gather(rs.size());
     std::vector<SmallSvdArgs> args;
+    std::vector<GramReplayArgs> reps;
     std::vector<SvdRequest*> in;
     size_t lds = 0;
+    unsigned gx = 1;
     for (auto* r : rs) {
       try {
         args.push_back(r->ws->small_prepare(r->m, r->n, infos_d + in.size()));
+        reps.push_back(r->ws->replay_args(r->n, args.back().logc, args.back().logs));
         lds = std::max(lds, Workspace::small_lds(r->m, r->n));
+        gx = std::max(gx, Workspace::replay_grid(r->n, std::min(r->m, r->n)));
         in.push_back(r);
       } catch (...) {
         fail(r);
       }
     }
     if (in.empty()) return;
-    for (auto& sa : args) sa.lds_bytes = (long)lds;
     Pack pk;
     const size_t oa = pk.add(args.data(), args.size() * sizeof(SmallSvdArgs));
+    const size_t orp = pk.add(reps.data(), reps.size() * sizeof(GramReplayArgs));
     char* base = upload(pk);
     HIP_CHECK(hipEventRecord(ev0, stream));
     small_svd_batch_kernel<<<(unsigned)in.size(), kSmallBatchThreads, lds, stream>>>(
         reinterpret_cast<const SmallSvdArgs*>(base + oa));
+    gram_replay_batch_kernel<<<dim3(gx, (unsigned)in.size()), 256, 0, stream>>>(
+        reinterpret_cast<const GramReplayArgs*>(base + orp));
+    gather(in, [](SvdRequest* r, float ms) { return r->ws->small_finish(r->m, r->n, ms); },
+           [&](SvdRequest* r) {
+             r->ws->small_state(r->m, r->n);
+             r->jm = r->n;
+             r->jn = r->ws->qr_r;
+             blocked->push_back(r);
+           });
+  }
+
+  // Y of at most kGramMaxRank columns: as run_small, after run_qr
+  void run_gram(std::vector<SvdRequest*>& rs, std::vector<SvdRequest*>* blocked) {
+    ensure_gather(rs.size());
+    std::vector<GramSvdArgs> args;
+    std::vector<GramReplayArgs> reps;
+    std::vector<SvdRequest*> in;
+    size_t lds = 0;
+    unsigned gx = 1;
+    for (auto* r : rs) {
+      try {
+        args.push_back(r->ws->gram_prepare(r->jm, r->jn, infos_d + in.size()));
+        reps.push_back(r->ws->replay_args(r->jm, args.back().logc, args.back().logs));
+        lds = std::max(lds, Workspace::gram_lds(r->jn));
+        gx = std::max(gx, Workspace::replay_grid(r->jm, r->jn));
+        in.push_back(r);
+      } catch (...) {
+        fail(r);
+      }
+    }
+    if (in.empty()) return;
+    Pack pk;
+    const size_t oa = pk.add(args.data(), args.size() * sizeof(GramSvdArgs));
+    const size_t orp = pk.add(reps.data(), reps.size() * sizeof(GramReplayArgs));
+    char* base = upload(pk);
+    HIP_CHECK(hipEventRecord(ev0, stream));
+    gram_svd_batch_kernel<<<(unsigned)in.size(), 1024, lds, stream>>>(
+        reinterpret_cast<const GramSvdArgs*>(base + oa));
+    gram_replay_batch_kernel<<<dim3(gx, (unsigned)in.size()), 256, 0, stream>>>(
+        reinterpret_cast<const GramReplayArgs*>(base + orp));
+    gather(in, [](SvdRequest* r, float ms) {
+      return r->ws->jacobi_check(r->jm, r->jn, ms, true);
+    }, [&](SvdRequest* r) { blocked->push_back(r); });
+  }
+
+  // after the launches of run_small / run_gram: summaries to the host, then
+  // `finish` per request, or `retry` where the Gram Jacobi did not converge
+  template <class Finish, class Retry>
+  void gather(std::vector<SvdRequest*>& in, Finish finish, Retry retry) {
     HIP_CHECK(hipEventRecord(ev1, stream));
     HIP_CHECK(hipGetLastError());
     n_launches += 1;
@@ -1303,7 +1447,8 @@ struct Batcher {
       SvdRequest* r = in[i];
       try {
         *r->ws->info_h = infos_h[i];
-        r->k = r->ws->small_finish(r->m, r->n, ms);
+        if (infos_h[i].sweeps < 0) retry(r);
+        else r->k = finish(r, ms);
       } catch (...) {
         fail(r);
       }
@@ -1506,11 +1651,15 @@ struct Batcher {
       else if (r->qr) qrs.push_back(r);
       else { r->jm = r->m; r->jn = r->n; }
     }
-    if (!smalls.empty()) run_small(smalls);
+    std::vector<SvdRequest*> jr, gr;
+    if (!smalls.empty()) run_small(smalls, &jr);
     if (!qrs.empty()) run_qr(qrs);
-    std::vector<SvdRequest*> jr;
-    for (auto* r : batch)
-      if (!r->failed && !(r->qr && r->ws->small_ok(r->m, r->n))) jr.push_back(r);
+    for (auto* r : batch) {
+      if (r->failed || (r->qr && r->ws->small_ok(r->m, r->n))) continue;
+      if (r->qr && r->ws->gram_ok(r->jn)) gr.push_back(r);
+      else jr.push_back(r);
+    }
+    if (!gr.empty()) run_gram(gr, &jr);
     if (!jr.empty()) run_jacobi(jr);
     for (auto* r : batch) r->ws->svd_stream = r->ws->stream;
   }

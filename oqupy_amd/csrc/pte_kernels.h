@@ -36,6 +36,8 @@ struct SvdInfo {
   int pad;
   double s0;       // largest singular value
   double discarded;  // 2-norm of the discarded singular values
+  int rounds;      // rotation rounds logged (Gram Jacobi)
+  int unused;
 };
 
 struct JacobiArgs {
@@ -128,21 +130,45 @@ struct RhArgs {
   double2* Y;
 };
 
-// One small truncated SVD done by one workgroup (small_svd_kernel): the same
-// outputs as the pivoted QR + Jacobi path (reflectors in A, tau, vscale,
-// beta, piv, *qrank; Z = Y W in Y (n x r, ld n); W (r x r, ld r); sigma,
-// perm, sorted; info with info->pad = r).
+// One small truncated SVD (small_svd_kernel): the pivoted QR's outputs
+// (reflectors in A, tau, vscale, beta, piv, *qrank), Y = R^H in Y (n x r,
+// ld n), sigma, perm, sorted, info (info->pad = r) and the rotation log, from
+// which gram_replay_kernel forms Z = Y W in Y and W.
 struct SmallSvdArgs {
   double2* A; int m, n;
   double2* tau; double2* vscale; double* beta; int* piv; int* qrank;
-  double2* Y; double2* W;
+  double2* Y;
   double* sigma; int* perm; double* sorted; SvdInfo* info;
   double epsrel; int max_rank; int max_sweeps;
   SvdInfo* copy;    // optional second copy of the summary (batched gather)
   double stop_rel;  // > 0: stop the QR at residual <= stop_rel * |beta_0|
-  long lds_bytes;   // dynamic LDS of the launch (W stays in LDS when it fits)
+  double* folded;   // optional: the squared residual of that stop
+  double* logc; double2* logs;
 };
 
+// Jacobi SVD of Y = R^H (n x r, ld n) of a pivoted QR on its Gram matrix, in
+// one workgroup (gram_svd_kernel): sigma, perm, sorted, info and the rotation
+// log (64 rotations per round).
+struct GramSvdArgs {
+  const double2* Y; int n, r;
+  double* sigma; int* perm; double* sorted; SvdInfo* info;
+  double epsrel; int max_rank; int max_sweeps;
+  SvdInfo* copy;
+  const double* extra2;     // optional squared weight counted in every tail
+  double* logc; double2* logs;
+};
+
+// Z = Y W in place and W (r x r, ld r, r = info->pad) from the rotation log;
+// nothing when info->sweeps < 0.
+struct GramReplayArgs {
+  double2* Y; int n;
+  double2* W;
+  const SvdInfo* info;
+  const double* logc; const double2* logs;
+};
+
+constexpr int kGramMaxRank = 126;           // G in LDS, two blocks of it per thread
+constexpr int kGramMaxSweeps = 20;          // sweeps the rotation log holds
 constexpr int kSmallMaxCols = 96;           // columns of M in small_svd_kernel
 constexpr int kSmallThreads = 1024;         // workgroup of small_svd_kernel
 constexpr int kSmallBatchThreads = 512;     // workgroup of small_svd_batch_kernel
@@ -163,6 +189,10 @@ __global__ void truncate_batch_kernel(const SvdPostArgs* pa, SvdInfo* out);
 __global__ void zero_items_kernel(const ZeroItem* items);
 __global__ void small_svd_kernel(SmallSvdArgs a);
 __global__ void small_svd_batch_kernel(const SmallSvdArgs* probs);
+__global__ void gram_svd_kernel(GramSvdArgs a);
+__global__ void gram_svd_batch_kernel(const GramSvdArgs* probs);
+__global__ void gram_replay_kernel(GramReplayArgs a);
+__global__ void gram_replay_batch_kernel(const GramReplayArgs* probs);   // problem = blockIdx.y
 __global__ void gather_qr_rank_kernel(const QrcpArgs* probs, int n, int* out);
 __global__ void apply_q_kernel(ApplyQArgs a);
 __global__ void apply_q_wave_kernel(ApplyQArgs a);   // Q of at most kApplyQWaveRows rows

@@ -1958,13 +1958,10 @@ build_rh_batch_kernel(const RhArgs* pa) {
 // ---------------------------------------------------------------------------
 // Small truncated SVD in one workgroup of NT threads (M with at most
 // kSmallMaxCols columns, staged in LDS): the pivoted QR of qrcp_kernel (same
-// reflectors, pivoting, norm downdating and eps-rank stop), then the
-// one-sided Jacobi of Y = R^H (n x r) with scalar column pairs in the
-// round-robin order (the rotation and stopping rule of jacobi_kernel), then
-// singular values, order and cut. Barriers are workgroup barriers only;
-// column pairs (and QR columns) are reduced by lane groups with wavefront
-// shuffles. Y stays in LDS; the accumulated rotation W (r x r) is kept in LDS
-// when Y and W fit in the dynamic LDS (a.lds_bytes), else in a.W.
+// reflectors, pivoting, norm downdating and eps-rank stop), then the Jacobi
+// of Y = R^H (n x r) on its Gram matrix in the same LDS (below), singular
+// values, order and cut. Barriers are workgroup barriers only; the QR's
+// columns are reduced by lane groups with wavefront shuffles.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double group_sum(double v, int G) { return group_sum1(v, G); }
 
@@ -1974,177 +1971,493 @@ __device__ __forceinline__ int pow2_ceil(int x) {
   return p;
 }
 
-// Sum over an NT-thread workgroup with one __syncthreads (wavefront sums in
-// slot[parity][wave], parity alternating between calls); every thread gets
-// the same bits.
-template <int NT>
-__device__ __forceinline__ double block_sum_nt(double v, double (*slot)[NT / 64], int& parity) {
-  v = wave_sum(v);
-  if ((threadIdx.x & 63) == 0) slot[parity][threadIdx.x >> 6] = v;
-  __syncthreads();
-  double r = 0.0;
-#pragma unroll
-  for (int w = 0; w < NT / 64; ++w) r += slot[parity][w];
-  parity ^= 1;
-  return r;
+// ---------------------------------------------------------------------------
+// Jacobi SVD of Y = R^H (n x r, r <= kGramMaxRank) of a pivoted QR in one
+// workgroup, on the Gram matrix.
+//
+// One-sided Jacobi rotates columns of Y, and of the accumulated W, and takes
+// three inner products of length n per pair and round to find each rotation.
+// Here the rotations are found on G = Y^H Y (computed once, on the FP64 matrix
+// cores) by two-sided rotations in LDS: a pair's three entries are read, not
+// summed. The rows of R fall off with the pivots, G = D A D with D their norms
+// and A well conditioned, and Jacobi keeps the small entries of such a matrix
+// to high relative accuracy (Demmel and Veselic, 1992), so the singular values
+// are the square roots of the final diagonal and the rotations orthogonalise
+// Y itself to the stopping rule of jacobi_kernel; they are applied to the rows
+// of Y and of the identity afterwards, by as many wavefronts as there are rows
+// (gram_replay_kernel), from a log of every round's rotations.
+//
+// The order is the round-robin of P = ceil(r / 2) pairs: position 2q holds the
+// pair's first column a_q, position 2q + 1 its second, b_q; position 0 keeps
+// its column and the others move on by one position a round (gram_next), so
+// that after re - 1 rounds (re = 2P) every two columns have met and all are
+// back. G is kept by positions, as the P (P + 1) / 2 blocks (q1, q2), q1 <= q2,
+// of 2 x 2 entries (the Hermitian half; 129 KB of LDS at r = 126), entry e of
+// every block in a plane of its own. A round is
+//   (1) every thread reads the blocks it owns; wavefront 0, one pair per lane,
+//       computes the rotations from the diagonal blocks, to LDS and to the log;
+//   (2) every thread rotates its blocks from both sides, J_q1^H B J_q2, and
+//       writes each entry where its columns are in the next round,
+// with a barrier after each. Reads and writes go to addresses that are the same
+// in every round: no index arithmetic, and reads without bank conflicts. (By
+// columns, with the packed triangle's indices computed every round, that
+// arithmetic alone took longer than the rotations: 1.5 us a round at r = 83.)
+// The padding column of an odd r is zero and stays so. A sweep starts with a
+// test of all pairs, so the last, idle sweep of the one-sided form is not run.
+// Rotation: (x_a, x_b) <- (c x_a - conj(s) x_b, s x_a + c x_b), s carrying the
+// phase of g_ab.
+// Bound by the chain of a round in one compute unit: LDS reads, about 60
+// dependent FP64 operations of a rotation, the blocks' 48 each, LDS writes.
+// Y of 100 columns on average (TEMPO, bonds of about a hundred): 0.41 ms
+// against 0.9 ms of jacobi_tile_kernel; 88 x 83 matrix in small_svd_kernel:
+// 0.82 ms against 1.83 ms with the one-sided sweeps in LDS, QR included.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int gram_block(int q1, int q2) { return q2 * (q2 + 1) / 2 + q1; }
+
+// position of column c in round 0 (P pairs) and a position's next one
+__device__ __forceinline__ int gram_pos(int c, int P) {
+  const int L = 2 * P - 1;
+  return c == L ? 0 : c == 0 ? 1 : c < P ? 2 * c : 2 * (L - c) + 1;
+}
+__device__ __forceinline__ int gram_next(int x, int P) {
+  if (x == 0 || P == 1) return x;
+  if (x == 2) return 1;
+  if ((x & 1) == 0) return x - 2;
+  return x == 2 * P - 1 ? x - 1 : x + 2;
 }
 
-// Lanes per pair (a power of two, NT/64..64, all pairs in one pass): the
-// count that minimises the issue slots of the most loaded SIMD, busy
-// wavefronts per SIMD x instructions per wavefront (rows per lane of the two
-// Y and two W columns, plus the reduction and the rotation); ties go to more
-// lanes (shorter chains).
-template <int NT>
-__device__ __forceinline__ int small_pair_lanes(int P, int n, int r) {
-  int best = NT / 64, best_cost = 1 << 30;
-  for (int gj = NT / 64; gj <= 64; gj *= 2) {
-    if (P * gj > NT || (gj > NT / 64 && gj > pow2_ceil(n))) break;
-    const int waves = (P * gj + 63) / 64;
-    const int per_simd = (waves + 3) / 4;
-    const int instr = ((n + gj - 1) / gj) * 35 + ((r + gj - 1) / gj) * 15 + 150;
-    const int cost = per_simd * instr;
-    if (cost <= best_cost) { best_cost = cost; best = gj; }
+// where the entry of positions (x, y) is kept (T: entries of a plane), and
+// whether conjugated
+__device__ __forceinline__ int gram_place(int x, int y, int T, bool& conj) {
+  const int qx = x >> 1, qy = y >> 1;
+  conj = qx > qy || (qx == qy && x > y);
+  if (conj) return (2 * (y & 1) + (x & 1)) * T + gram_block(qy, qx);
+  return (2 * (x & 1) + (y & 1)) * T + gram_block(qx, qy);
+}
+
+// 16 x 16 tile t of the upper triangle of Y^H Y (list (0,0), (0,1), (1,1),
+// (0,2), ...) by one wavefront, 3M on the FP64 matrix cores; Y is n x r with
+// leading dimension ld. Lane l gets rows 4 q + l / 16 of column l % 16.
+__device__ __forceinline__ void gram_tile_index(int t, int& I, int& J) {
+  J = 0;
+  while ((J + 1) * (J + 2) / 2 <= t) ++J;
+  I = t - J * (J + 1) / 2;
+}
+
+__device__ __forceinline__ void gram_tile(const double2* Y, long ld, int n, int r, int t,
+                                          double2 (&g)[4]) {
+  const int lane = threadIdx.x & 63;
+  const int lr = lane & 15, lk = lane >> 4;
+  int I, J;
+  gram_tile_index(t, I, J);
+  const int ci = 16 * I + lr, cj = 16 * J + lr;
+  const double2* yi = Y + (long)min(ci, r - 1) * ld;
+  const double2* yj = Y + (long)min(cj, r - 1) * ld;
+  doublex4 p1 = {0.0, 0.0, 0.0, 0.0}, p2 = p1, p3 = p1;
+#pragma unroll 4
+  for (int k4 = 0; k4 < n; k4 += 4) {
+    const int k = k4 + lk;
+    double2 x = yi[min(k, n - 1)], y = yj[min(k, n - 1)];
+    if (k >= n || ci >= r) x = make_double2(0.0, 0.0);
+    if (k >= n || cj >= r) y = make_double2(0.0, 0.0);
+    p1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, y.x, p1, 0, 0, 0);
+    p2 = __builtin_amdgcn_mfma_f64_16x16x4f64(-x.y, y.y, p2, 0, 0, 0);
+    p3 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x - x.y, y.x + y.y, p3, 0, 0, 0);
   }
-  return best;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) g[q] = make_double2(p1[q] - p2[q], p3[q] - p1[q] - p2[q]);
 }
 
-// Cyclic one-sided Jacobi sweeps on the columns of Ys (n x r, ld n, LDS),
-// rotations accumulated in W (r x r, ld r): in LDS after Y when WL, else Wg.
-// Lane group q (GJ lanes) owns pair q of each round; a lane holds rows
-// gj, gj + GJ, ... (at most RP) of the pair's two columns in registers. The
-// row loops are branch-free: a block of GJ rows is skipped when it starts
-// past the end (a test uniform over the workgroup), and inside the last block
-// a lane past the end works on the last row instead, masked out of the inner
-// products; it then stores the same bits as the lane that owns that row.
-// A pair is skipped when neither column has been rotated since the round
-// one sweep earlier (the order repeats every sweep, so that round checked
-// this pair and found it converged): recomputing it would give the same bits.
-// last_rot[c] (LDS) is the round of column c's last rotation; a wavefront
-// whose pairs are all skipped only takes part in the barrier.
-// Returns the sweep count; `converged` when the last sweep rotated nothing.
-template <int NT, bool WL>
-__device__ __forceinline__ int small_jacobi(double2* Ys, double2* Wg, int n, int r,
-                                            double tol2, double abs_tol2, int max_sweeps,
-                                            int* last_rot, bool& converged) {
-  constexpr int RP = kSmallMaxCols * 64 / NT;   // GJ >= NT / 64 lanes per pair
-  double2* const Wp = WL ? Ys + (long)n * r : Wg;
-  const int tid = threadIdx.x;
-  const int re = r + (r & 1);
-  const int P = re / 2;
-  const int GJ = small_pair_lanes<NT>(P, n, r);
-  const int q = tid / GJ, gj = tid % GJ;
-  const int L = re > 1 ? re - 1 : 1;
-  // a wavefront whose lane groups all lie beyond the last pair only takes
-  // part in the barriers
-  const bool wave_busy = (tid & ~63) / GJ < P;
-  const double2 zero = make_double2(0.0, 0.0);
-  int sweeps = 0;
-  converged = false;
-  SEG_INIT();
-  for (; sweeps < max_sweeps; ++sweeps) {
-    int any = 0;
-    for (int round = 0; round < L; ++round) {
-      const int gr = sweeps * L + round;   // global round index
-      if (!wave_busy) {
-        __syncthreads();
-        continue;
-      }
-      int ci = 0, cj = 0;
-      bool valid = false;
-      if (q < P && re > 1) {
-        // round-robin pairing of tournament_pair without integer division
-        const int Lr = re - 1;
-        if (q == 0) {
-          ci = Lr;
-          cj = round;
-        } else {
-          ci = round + q;
-          if (ci >= Lr) ci -= Lr;
-          cj = round - q;
-          if (cj < 0) cj += Lr;
-        }
-        if (ci > cj) { const int tt = ci; ci = cj; cj = tt; }
-        valid = cj < r;
-        if (valid && gr >= L && last_rot[ci] < gr - L && last_rot[cj] < gr - L)
-          valid = false;   // converged at its last check, columns unchanged
-      }
-      // a wavefront whose pairs are all skipped only takes part in the barrier
-      if (__ballot(valid) != 0) {
-        if (!valid) { ci = 0; cj = 0; }   // harmless addresses; no rotation
-        double2* y0 = Ys + (long)ci * n;
-        double2* y1 = Ys + (long)cj * n;
-        double2 yi[RP], yj[RP];
-        double al = 0.0, be = 0.0;
-        double2 ga = zero;
+// that tile into G (zeroed before: the padding column has no entries)
+__device__ __forceinline__ void gram_store(double2* G, int r, int t, const double2 (&g)[4]) {
+  const int lane = threadIdx.x & 63;
+  const int lr = lane & 15, lk = lane >> 4;
+  const int P = (r + 1) / 2, T = P * (P + 1) / 2;
+  int I, J;
+  gram_tile_index(t, I, J);
+  const int j = 16 * J + lr;
 #pragma unroll
-        for (int t = 0; t < RP; ++t) {
-          if (t * GJ < n) {
-            const int i0 = gj + t * GJ;
-            const int i = min(i0, n - 1);
-            yi[t] = y0[i];
-            yj[t] = y1[i];
-            const double2 u = i0 < n ? yi[t] : zero;
-            const double2 v = i0 < n ? yj[t] : zero;
-            al += cabs2(u);
-            be += cabs2(v);
-            cfmac(ga, u, v);
-          }
-        }
-        SEG(0);
-        group_sum4(al, be, ga.x, ga.y, GJ);
-        SEG(1);
-        double rot[4];
-        const bool rotate = jacobi_rotation_fast(valid, al, be, ga, tol2, abs_tol2, rot);
-        SEG(2);
-        if (rotate) {
-          any = 1;
-          const double c = rot[0], sn = rot[1];
-          const double2 cph = make_double2(rot[2], -rot[3]);
+  for (int q = 0; q < 4; ++q) {
+    const int i = 16 * I + 4 * q + lk;
+    if (i > j || j >= r) continue;
+    bool conj;
+    const int at = gram_place(gram_pos(i, P), gram_pos(j, P), T, conj);
+    const double im = i == j ? 0.0 : g[q].y;
+    G[at] = make_double2(g[q].x, conj ? -im : im);
+  }
+}
+
+// Two-sided Jacobi sweeps on G (rank r) in LDS; rc, rs: LDS scratch of 64
+// rotations; NB: blocks per thread, at least T / NT. Returns the sweeps done.
+template <int NT, int NB>
+__device__ __forceinline__ int gram_jacobi(double2* G, int r, double tol2, double abs_tol2,
+                                           int max_sweeps, double* rc, double2* rs,
+                                           double* logc, double2* logs, bool& converged) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int P = (r + 1) / 2, L = 2 * P - 1;
+  const int T = P * (P + 1) / 2;
+  int q1[NB], q2[NB];      // own blocks tid, tid + NT, ... (q1 = -1: none)
+  // places of the entries in the next round, 15 bits each, and in bit 15 the
+  // conjugation: entries 0 and 1 in dst[u][0], 2 and 3 in dst[u][1]
+  unsigned dst[NB][2];
 #pragma unroll
-          for (int t = 0; t < RP; ++t) {
-            if (t * GJ < n) {
-              const int i = min(gj + t * GJ, n - 1);
-              const double2 xp = yi[t];
-              const double2 xq = cmul(yj[t], cph);
-              y0[i] = make_double2(c * xp.x - sn * xq.x, c * xp.y - sn * xq.y);
-              y1[i] = make_double2(sn * xp.x + c * xq.x, sn * xp.y + c * xq.y);
-            }
-          }
-          SEG(3);
-          double2* w0 = Wp + (long)ci * r;
-          double2* w1 = Wp + (long)cj * r;
-#pragma unroll
-          for (int t = 0; t < RP; ++t) {
-            if (t * GJ < r) {
-              const int i = min(gj + t * GJ, r - 1);
-              const double2 xp = w0[i];
-              const double2 xq = cmul(w1[i], cph);
-              w0[i] = make_double2(c * xp.x - sn * xq.x, c * xp.y - sn * xq.y);
-              w1[i] = make_double2(sn * xp.x + c * xq.x, sn * xp.y + c * xq.y);
-            }
-          }
-          if (gj == 0) { last_rot[ci] = gr; last_rot[cj] = gr; }
-          SEG(4);
-        }
-      }
-      __syncthreads();
-      SEG(5);
+  for (int u = 0; u < NB; ++u) {
+    const int b = tid + u * NT;
+    int c = 0;
+    if (b < T) {
+      c = (int)((sqrtf(8.0f * (float)b + 1.0f) - 1.0f) * 0.5f);
+      while ((c + 1) * (c + 2) / 2 <= b) ++c;
+      while (c * (c + 1) / 2 > b) --c;
     }
-    if (!__syncthreads_or(any)) {
+    q2[u] = c;
+    q1[u] = b < T ? b - c * (c + 1) / 2 : -1;
+    dst[u][0] = dst[u][1] = 0;
+    if (q1[u] >= 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        bool conj = false;
+        const int at = gram_place(gram_next(2 * q1[u] + (e >> 1), P),
+                                  gram_next(2 * q2[u] + (e & 1), P), T, conj);
+        dst[u][e >> 1] |= ((unsigned)at | (conj ? 0x8000u : 0u)) << (16 * (e & 1));
+      }
+    }
+  }
+  auto put = [&](unsigned place, double2 v) {   // place in the upper 16 bits
+    v.y = __hiloint2double(__double2hiint(v.y) ^ (int)(place & 0x80000000u),
+                           __double2loint(v.y));
+    G[(place >> 16) & 0x7fffu] = v;
+  };
+  converged = false;
+  int sweeps = 0;
+  for (;;) {
+    int mine = 0;
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      if (q1[u] < 0) continue;
+      const int b = tid + u * NT, b1 = gram_block(q1[u], q1[u]), b2 = gram_block(q2[u], q2[u]);
+      const double da1 = G[b1].x, db1 = G[3 * T + b1].x;
+      const double da2 = G[b2].x, db2 = G[3 * T + b2].x;
+      bool any = needs_rotation(da1, db2, cabs2(G[T + b]), tol2, abs_tol2);
+      if (q1[u] != q2[u]) {
+        any |= needs_rotation(da1, da2, cabs2(G[b]), tol2, abs_tol2);
+        any |= needs_rotation(db1, da2, cabs2(G[2 * T + b]), tol2, abs_tol2);
+        any |= needs_rotation(db1, db2, cabs2(G[3 * T + b]), tol2, abs_tol2);
+      }
+      if (any) mine = 1;
+    }
+    if (!__syncthreads_or(mine)) {
       converged = true;
       break;
     }
+    if (sweeps == max_sweeps) break;
+    for (int t = 0; t < L; ++t) {
+      double2 b00[NB], b01[NB], b10[NB], b11[NB];
+#pragma unroll
+      for (int u = 0; u < NB; ++u) {
+        const int b = q1[u] >= 0 ? tid + u * NT : 0;
+        b00[u] = G[b];
+        b01[u] = G[T + b];
+        b10[u] = G[2 * T + b];
+        b11[u] = G[3 * T + b];
+      }
+      if (wave == 0) {
+        const bool valid = lane < P;
+        const int d = gram_block(min(lane, P - 1), min(lane, P - 1));
+        double rot[4];
+        (void)jacobi_rotation_fast(valid, G[d].x, G[3 * T + d].x, G[T + d], tol2, abs_tol2,
+                                   rot);
+        const double2 s = make_double2(rot[1] * rot[2], rot[1] * rot[3]);
+        if (valid) {
+          rc[lane] = rot[0];
+          rs[lane] = s;
+          const long e = (long)(sweeps * L + t) * 64 + lane;
+          logc[e] = rot[0];
+          logs[e] = s;
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < NB; ++u) {
+        if (q1[u] >= 0) {
+          const double c1 = rc[q1[u]], c2 = rc[q2[u]];
+          const double2 s1 = rs[q1[u]], s2 = rs[q2[u]];
+          const double2 s1c = cconj(s1), s2c = cconj(s2);
+          const bool diag = q1[u] == q2[u];
+          if (diag) b10[u] = cconj(b01[u]);
+          const double2 n00 = csub(cscale(b00[u], c2), cmul(s2c, b01[u]));
+          const double2 n01 = cadd(cmul(s2, b00[u]), cscale(b01[u], c2));
+          const double2 n10 = csub(cscale(b10[u], c2), cmul(s2c, b11[u]));
+          const double2 n11 = cadd(cmul(s2, b10[u]), cscale(b11[u], c2));
+          double2 m00 = csub(cscale(n00, c1), cmul(s1, n10));
+          double2 m01 = csub(cscale(n01, c1), cmul(s1, n11));
+          const double2 m10 = cadd(cmul(s1c, n00), cscale(n10, c1));
+          double2 m11 = cadd(cmul(s1c, n01), cscale(n11, c1));
+          if (diag) {
+            m00.y = 0.0;
+            m11.y = 0.0;
+            // a rotated pair is diagonal
+            if (s1.x != 0.0 || s1.y != 0.0) m01 = make_double2(0.0, 0.0);
+          } else {
+            put(dst[u][1] << 16, m10);
+          }
+          put(dst[u][0] << 16, m00);
+          put(dst[u][0], m01);
+          put(dst[u][1], m11);
+        }
+      }
+      __syncthreads();
+    }
+    ++sweeps;
   }
-  SEG_FLUSH(0, 6);
   return sweeps;
+}
+
+// squared norm of column c (after whole sweeps)
+__device__ __forceinline__ double gram_diag(const double2* G, int c, int r) {
+  const int P = (r + 1) / 2, T = P * (P + 1) / 2;
+  const int x = gram_pos(c, P), q = x >> 1;
+  return G[((x & 1) ? 3 * T : 0) + gram_block(q, q)].x;
+}
+
+// Scales G by an even power of two that brings its trace to [1, 4), so that
+// the squares of its entries in the rotations' tests stay in range; returns the
+// scaled trace, and in *half half the exponent taken out (sigma = sqrt(g_cc)
+// 2^half). Called by the whole workgroup after a barrier; ends with one.
+template <int NT>
+__device__ __forceinline__ double gram_scale(double2* G, int r, int* half) {
+  double tr = 0.0;
+  for (int i = threadIdx.x & 63; i < r; i += 64) tr += gram_diag(G, i, r);
+  tr = wave_sum(tr);          // the same bits in every wavefront
+  *half = 0;
+  if (!(tr > 0.0 && tr < 1.7e308)) return tr;
+  *half = ilogb(tr) >> 1;
+  const int P = (r + 1) / 2;
+  __syncthreads();
+  for (int e = threadIdx.x; e < 2 * P * (P + 1); e += NT) {
+    const double2 v = G[e];
+    G[e] = make_double2(ldexp(v.x, -2 * *half), ldexp(v.y, -2 * *half));
+  }
+  __syncthreads();
+  return ldexp(tr, -2 * *half);
+}
+
+// LDS of the Gram Jacobi: G, 64 rotations, three r-vectors
+__device__ __host__ constexpr int gram_entries(int r) {
+  return 4 * (((r + 1) / 2) * ((r + 1) / 2 + 1) / 2);
+}
+
+// Singular values (roots of G's diagonal), descending order and cut, by the
+// whole workgroup; s_sig, s_sorted, s_tail: LDS, r entries each, outside G.
+// extra2: squared weight left out of G, counted in every tail (valid in every
+// thread of wavefront 0).
+template <int NT>
+__device__ __forceinline__ void gram_finish(const double2* G, int r, double epsrel,
+                                            int max_rank, double extra2, int sweeps,
+                                            int rounds, bool converged, int half,
+                                            double* s_sig,
+                                            double* s_sorted, double* s_tail, double* sigma,
+                                            int* perm, double* sorted, SvdInfo* info,
+                                            SvdInfo* copy) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  int bad = 0;
+  if (tid < r) {
+    const double d = gram_diag(G, tid, r);
+    bad = !(d < 1.7e308);                     // not a number, or overflowed
+    const double sg = ldexp(sqrt(fmax(d, 0.0)), half);
+    s_sig[tid] = sg;
+    sigma[tid] = sg;
+  }
+  bad = __syncthreads_or(bad);
+  if (tid < r && !bad) {
+    const double sj = s_sig[tid];
+    int rank = 0;
+    for (int i = 0; i < r; ++i) {
+      const double si = s_sig[i];
+      rank += (si > sj) || (si == sj && i < tid);
+    }
+    perm[rank] = tid;
+    sorted[rank] = sj;
+    s_sorted[rank] = sj;
+  }
+  __syncthreads();
+  if (tid >= 64) return;
+  // tails sum_{i >= j} s_i^2 of the two values of each lane: suffix scan of
+  // the lane sums; k = #{j: sqrt(tail_j) > epsrel s_0}
+  const int i0 = 2 * lane, i1 = i0 + 1;
+  const double v0 = i0 < r && !bad ? s_sorted[i0] * s_sorted[i0] : 0.0;
+  const double v1 = i1 < r && !bad ? s_sorted[i1] * s_sorted[i1] : 0.0;
+  double x = v0 + v1;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const double o = __shfl_down(x, off, 64);
+    if (lane + off < 64) x += o;
+  }
+  double after = __shfl_down(x, 1, 64);
+  if (lane == 63) after = 0.0;
+  const double t1 = after + v1 + extra2, t0 = after + (v0 + v1) + extra2;
+  const double s0 = bad ? 0.0 : s_sorted[0];
+  const double thr = epsrel * s0;
+  const int k = bad ? 0 : __popcll(__ballot(i0 < r && sqrt(t0) > thr)) +
+                          __popcll(__ballot(i1 < r && sqrt(t1) > thr));
+  if (i0 < r) s_tail[i0] = t0;
+  if (i1 < r) s_tail[i1] = t1;
+  __builtin_amdgcn_wave_barrier();
+  if (lane == 0) {
+    SvdInfo inf;
+    inf.rank = k;
+    inf.overflow = k > max_rank ? 1 : 0;
+    inf.sweeps = converged ? sweeps + 1 : -1;
+    inf.pad = r;
+    inf.s0 = s0;
+    inf.discarded = sqrt(k < r ? s_tail[k] : extra2);
+    inf.rounds = rounds;
+    inf.unused = 0;
+    *info = inf;
+    if (copy) *copy = inf;
+  }
+}
+
+constexpr int kGramThreads = 1024;
+// pair blocks per thread: 2016 at r = 126, two for each of 1024 threads (a third
+// does not fit the 128 registers of a thread)
+constexpr int kGramBlocks = 2;
+
+__device__ __forceinline__ void gram_svd_body(const GramSvdArgs& a) {
+  extern __shared__ double2 lds_gram[];
+  const int r = a.r;
+  double2* G = lds_gram;
+  double2* rs = G + gram_entries(r);
+  double* rc = reinterpret_cast<double*>(rs + 64);
+  double* s_sig = rc + 64;
+  for (int e = threadIdx.x; e < gram_entries(r); e += kGramThreads)
+    G[e] = make_double2(0.0, 0.0);
+  __syncthreads();
+  const int nb = (r + 15) / 16;
+  for (int t = threadIdx.x >> 6; t < nb * (nb + 1) / 2; t += kGramThreads / 64) {
+    double2 g[4];
+    gram_tile(a.Y, a.n, a.n, r, t, g);
+    gram_store(G, r, t, g);
+  }
+  __syncthreads();
+  int half;
+  const double tr = gram_scale<kGramThreads>(G, r, &half);
+  const double eps = 2.220446049250313e-16;
+  const double tol = (a.n > 16 ? a.n : 16) * eps;
+  bool converged = false;
+  const int sweeps = gram_jacobi<kGramThreads, kGramBlocks>(
+      G, r, tol * tol, eps * eps * tr, a.max_sweeps, rc, rs, a.logc, a.logs, converged);
+  const int L = max(2, r + (r & 1)) - 1;
+  gram_finish<kGramThreads>(G, r, a.epsrel, a.max_rank, a.extra2 ? *a.extra2 : 0.0, sweeps,
+                            sweeps * L, converged, half, s_sig, s_sig + r, s_sig + 2 * r, a.sigma,
+                            a.perm, a.sorted, a.info, a.copy);
+}
+
+__global__ void __launch_bounds__(kGramThreads)
+gram_svd_kernel(GramSvdArgs a) {
+  gram_svd_body(a);
+}
+
+__global__ void __launch_bounds__(kGramThreads)
+gram_svd_batch_kernel(const GramSvdArgs* probs) {
+  const GramSvdArgs a = probs[blockIdx.x];
+  gram_svd_body(a);
+}
+
+// wavefront shifts by one lane: lane i reads lane i + 1 (down) or i - 1 (up)
+constexpr int kDppWaveShl1 = 0x130, kDppWaveShr1 = 0x138;
+template <int CTRL>
+__device__ __forceinline__ double2 dpp_d2(double2 v) {
+  return make_double2(dpp_d<CTRL>(v.x), dpp_d<CTRL>(v.y));
+}
+
+// Applies the logged rotations to the rows of Y (in place: Z = Y W) and of
+// the identity (W, r x r), one wavefront per row. Lane q holds the entries of
+// the row in columns a_q and b_q; going to the next round of the round-robin
+// moves every a one lane down and every b one lane up (a_0 stays, b of the
+// last lane turns into its a, a_1 into b_0), so that a round is 12 FMAs and
+// register moves, with no LDS, no barrier and no column index; after whole
+// sweeps every entry is back in its column. The rounds' rotations are the
+// same for all rows (L2) and are loaded four rounds ahead. 0.05 us a round.
+__device__ __forceinline__ void gram_replay_body(const GramReplayArgs& a, int row) {
+  const SvdInfo inf = *a.info;
+  const int r = inf.pad, n = a.n;
+  if (inf.sweeps < 0 || r < 1 || row >= n + r) return;
+  const int lane = threadIdx.x & 63;
+  const int re = max(2, r + (r & 1)), P = re / 2, L = re - 1;
+  const double2 zero = make_double2(0.0, 0.0);
+  const int ca = lane == 0 ? L : lane, cb = lane == 0 ? 0 : L - lane;
+  const bool oa = lane < P && ca < r, ob = lane < P && cb < r;
+  const bool isy = row < n;
+  double2 xa = zero, xb = zero;
+  if (isy) {
+    if (oa) xa = a.Y[row + (long)ca * n];
+    if (ob) xb = a.Y[row + (long)cb * n];
+  } else {
+    if (oa && ca == row - n) xa.x = 1.0;
+    if (ob && cb == row - n) xb.x = 1.0;
+  }
+  const int rounds = inf.rounds;
+  const int le = min(lane, P - 1);
+  constexpr int PFR = 4;
+  double nc[PFR];
+  double2 ns[PFR];
+  auto fetch = [&](int t0) {
+#pragma unroll
+    for (int u = 0; u < PFR; ++u) {
+      const long e = (long)min(t0 + u, rounds - 1) * 64 + le;
+      nc[u] = a.logc[e];
+      ns[u] = a.logs[e];
+    }
+  };
+  if (rounds > 0) fetch(0);
+  for (int t0 = 0; t0 < rounds; t0 += PFR) {
+    double c[PFR];
+    double2 s[PFR];
+#pragma unroll
+    for (int u = 0; u < PFR; ++u) { c[u] = nc[u]; s[u] = ns[u]; }
+    if (t0 + PFR < rounds) fetch(t0 + PFR);
+#pragma unroll
+    for (int u = 0; u < PFR; ++u) {
+      if (t0 + u < rounds) {
+        double2 ya = cscale(xa, c[u]), yb = cscale(xb, c[u]);
+        cfmac(ya, make_double2(-s[u].x, -s[u].y), xb);
+        cfma(yb, s[u], xa);
+        if (P > 1) {
+          const double2 down = dpp_d2<kDppWaveShl1>(ya), up = dpp_d2<kDppWaveShr1>(yb);
+          xa = lane == 0 ? ya : (lane == P - 1 ? yb : down);
+          xb = lane == 0 ? down : up;
+        } else {
+          xa = ya;
+          xb = yb;
+        }
+      }
+    }
+  }
+  if (isy) {
+    if (oa) a.Y[row + (long)ca * n] = xa;
+    if (ob) a.Y[row + (long)cb * n] = xb;
+  } else {
+    if (oa) a.W[row - n + (long)ca * r] = xa;
+    if (ob) a.W[row - n + (long)cb * r] = xb;
+  }
+}
+
+__global__ void __launch_bounds__(256)
+gram_replay_kernel(GramReplayArgs a) {
+  gram_replay_body(a, blockIdx.x * 4 + (threadIdx.x >> 6));
+}
+
+__global__ void __launch_bounds__(256)
+gram_replay_batch_kernel(const GramReplayArgs* probs) {
+  const GramReplayArgs a = probs[blockIdx.y];
+  gram_replay_body(a, blockIdx.x * 4 + (threadIdx.x >> 6));
 }
 
 template <int NT>
 __device__ void small_svd_body(const SmallSvdArgs& a) {
-  static_assert(NT % 64 == 0 && (kSmallMaxCols * 64) % NT == 0, "workgroup size");
+  static_assert(NT % 64 == 0, "workgroup size");
   extern __shared__ double2 lds_small[];
-  __shared__ double slot[2][NT / 64];
-  int parity = 0;
+  __shared__ double s_folded;       // residual of an adaptive stop (folded2)
   const int m = a.m, n = a.n, tid = threadIdx.x, lane = tid & 63;
   // QR phase: M (m x n, ld m), then the per-column scalars (64 n bytes)
   double2* As = lds_small;
@@ -2338,93 +2651,63 @@ __device__ void small_svd_body(const SmallSvdArgs& a) {
       SvdInfo inf;
       inf.rank = 0; inf.overflow = 0; inf.sweeps = 1; inf.pad = 0;
       inf.s0 = 0.0; inf.discarded = 0.0;
+      inf.rounds = 0; inf.unused = 0;
       *a.info = inf;
       if (a.copy) *a.copy = inf;
     }
     return;
   }
-  // ---- Y = R^H (n x r, ld n) in LDS; W = I (r x r) in LDS or a.W ----
-  // Y lies inside the space of M (r <= m), below the scalars it reads; W
-  // (when it fits) follows Y and may cover the scalars, so it is set after
-  // a barrier.
+  // ---- Y = R^H (n x r) to global memory and to LDS (odd leading dimension:
+  // the tile loads of the Gram matrix step over columns), G from it on the
+  // matrix cores, then G over Y in LDS ----
+  const int ldy = n | 1;
   double2* Ys = lds_small;
-  const bool wl = (long)(n + r) * r * (long)sizeof(double2) <= a.lds_bytes;
-  double2* Wp = wl ? Ys + (long)n * r : a.W;
   for (long e = tid; e < (long)n * r; e += NT) {
     const int sidx = e % n, t = e / n;
     const int ps = q_piv[sidx];
     double2 v = make_double2(0.0, 0.0);
     if (t < sidx) v = cconj(a.A[t + (long)ps * m]);   // As is being overwritten
-    else if (t == sidx) v = make_double2(q_beta[sidx], 0.0);
-    Ys[e] = v;
+    else if (t == sidx) v = make_double2(a.beta[sidx], 0.0);
+    a.Y[e] = v;
   }
   __syncthreads();
-  for (long e = tid; e < (long)r * r; e += NT)
-    Wp[e] = make_double2((e % r) == (e / r) ? 1.0 : 0.0, 0.0);
+  for (long e = tid; e < (long)n * r; e += NT) Ys[e % n + (e / n) * ldy] = a.Y[e];
   __syncthreads();
-  double fpart = 0.0;
-  for (long e = tid; e < (long)n * r; e += NT) fpart += cabs2(Ys[e]);
-  const double fro = sqrt(block_sum_nt<NT>(fpart, slot, parity));
-  const double tol = (n > 16 ? n : 16) * eps, abs_tol = eps * fro;
-  // ---- one-sided Jacobi on the columns of Y ----
-  __shared__ int last_rot[kSmallMaxCols];
-  for (int c = tid; c < r; c += NT) last_rot[c] = -(1 << 30);
+  double2* Gm = lds_small;
+  double2* rs = Gm + gram_entries(r);
+  double* rc = reinterpret_cast<double*>(rs + 64);
+  double* s_sig = rc + 64;
+  {
+    constexpr int kTiles = (21 + NT / 64 - 1) / (NT / 64);   // of 21 at 96 columns
+    const int nb = (r + 15) / 16, tiles = nb * (nb + 1) / 2;
+    double2 g[kTiles][4];
+#pragma unroll
+    for (int u = 0; u < kTiles; ++u)
+      if (wave + u * (NT / 64) < tiles) gram_tile(Ys, ldy, n, r, wave + u * (NT / 64), g[u]);
+    __syncthreads();
+    for (int e = tid; e < gram_entries(r); e += NT) Gm[e] = make_double2(0.0, 0.0);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kTiles; ++u)
+      if (wave + u * (NT / 64) < tiles) gram_store(Gm, r, wave + u * (NT / 64), g[u]);
+  }
   __syncthreads();
+  int half;
+  const double tr = gram_scale<NT>(Gm, r, &half);
+  const double tol = (n > 16 ? n : 16) * eps;
   bool converged = false;
-  const int sweeps = wl ? small_jacobi<NT, true>(Ys, a.W, n, r, tol * tol, abs_tol * abs_tol,
-                                                 a.max_sweeps, last_rot, converged)
-                        : small_jacobi<NT, false>(Ys, a.W, n, r, tol * tol, abs_tol * abs_tol,
-                                                  a.max_sweeps, last_rot, converged);
+  constexpr int kBlocks = (1176 + NT - 1) / NT;              // of 1176 at 96 columns
+  const int sweeps = gram_jacobi<NT, kBlocks>(Gm, r, tol * tol, eps * eps * tr, a.max_sweeps,
+                                              rc, rs, a.logc, a.logs, converged);
   PHASE(14);
-  // ---- singular values, order, cut; Z and W to global memory ----
-  for (long e = tid; e < (long)n * r; e += NT) a.Y[e] = Ys[e];
-  if (wl)
-    for (long e = tid; e < (long)r * r; e += NT) a.W[e] = Wp[e];
-  __syncthreads();
-  // two r-vectors after Y (over W, which is in global memory now)
-  double* s_sig = reinterpret_cast<double*>(Ys + (long)n * r);
-  double* s_sorted = s_sig + r;
-  for (int c = tid / 64; c < r; c += NT / 64) {
-    double part2 = 0.0;
-    for (int i = lane; i < n; i += 64) part2 += cabs2(Ys[i + (long)c * n]);
-    const double sg = sqrt(wave_sum(part2));
-    if (lane == 0) { s_sig[c] = sg; a.sigma[c] = sg; }
-  }
-  __syncthreads();
-  if (tid < r) {
-    const double sj = s_sig[tid];
-    int rank = 0;
-    for (int i = 0; i < r; ++i) {
-      const double si = s_sig[i];
-      rank += (si > sj) || (si == sj && i < tid);
-    }
-    a.perm[rank] = tid;
-    a.sorted[rank] = sj;
-    s_sorted[rank] = sj;
-  }
-  __syncthreads();
   if (tid == 0) {
-    // smallest k with sqrt(sum_{i>=k} s_i^2) <= epsrel s_0 (suffix sums)
-    const double s0 = s_sorted[0];
-    const double thr = a.epsrel * s0;
-    double tail = folded2;
-    int k = 0;
-    for (int i = r - 1; i >= 0; --i) {
-      tail += s_sorted[i] * s_sorted[i];
-      if (sqrt(tail) > thr) { k = i + 1; break; }
-    }
-    double d = folded2;
-    for (int i = r - 1; i >= k; --i) d += s_sorted[i] * s_sorted[i];
-    SvdInfo inf;
-    inf.rank = k;
-    inf.overflow = k > a.max_rank ? 1 : 0;
-    inf.sweeps = converged ? sweeps + 1 : -1;
-    inf.pad = r;
-    inf.s0 = s0;
-    inf.discarded = sqrt(d);
-    *a.info = inf;
-    if (a.copy) *a.copy = inf;
+    s_folded = folded2;
+    if (a.folded) *a.folded = folded2;
   }
+  __syncthreads();
+  gram_finish<NT>(Gm, r, a.epsrel, a.max_rank, s_folded, sweeps,
+                  sweeps * (max(2, r + (r & 1)) - 1), converged, half, s_sig, s_sig + r,
+                  s_sig + 2 * r, a.sigma, a.perm, a.sorted, a.info, a.copy);
   PHASE(15);
 }
 
