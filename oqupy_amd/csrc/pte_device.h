@@ -52,13 +52,47 @@ template <int CTRL>
 __device__ __forceinline__ double dpp_d(double v) {
   const long long b = __double_as_longlong(v);
   int lo = (int)(b & 0xffffffffll), hi = (int)(b >> 32);
-  lo = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xF, 0xF, false);
-  hi = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xF, 0xF, false);
+  lo = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xF, 0xF, true);
+  hi = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xF, 0xF, true);
   return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
 }
 template <int CTRL>
 __device__ __forceinline__ int dpp_i(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
+}
+
+// Both halves of a double's exchange across rows of 16 lanes (HALF 16: with the
+// neighbouring row; HALF 32: with the other half of the wavefront): lo is the
+// value of the lower partner, hi of the upper one, on both partners. Two VALU
+// moves (gfx950 lane swaps) instead of two LDS-routed shuffles.
+template <int HALF>
+__device__ __forceinline__ void swap_d(double v, double& lo, double& hi) {
+  const unsigned a = (unsigned)__double2loint(v), b = (unsigned)__double2hiint(v);
+  typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+  uint2v x, y;
+  if constexpr (HALF == 16) {
+    x = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+    y = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  } else {
+    x = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+    y = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  }
+  lo = __hiloint2double((int)y[0], (int)x[0]);
+  hi = __hiloint2double((int)y[1], (int)x[1]);
+}
+template <int HALF>
+__device__ __forceinline__ double swap_sum(double v) {
+  double lo, hi;
+  swap_d<HALF>(v, lo, hi);
+  return lo + hi;
+}
+template <int HALF>
+__device__ __forceinline__ unsigned swap_max(unsigned v) {
+  typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+  uint2v x;
+  if constexpr (HALF == 16) x = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  else x = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return max(x[0], x[1]);
 }
 
 // Sums over aligned groups of G lanes (G a power of two <= 64) of four
@@ -83,12 +117,12 @@ __device__ __forceinline__ void group_sum4(double& a, double& b, double& c, doub
     c += dpp_d<kDppMirror>(c); d += dpp_d<kDppMirror>(d);
   }
   if (G >= 32) {
-    a += __shfl_xor(a, 16, 64); b += __shfl_xor(b, 16, 64);
-    c += __shfl_xor(c, 16, 64); d += __shfl_xor(d, 16, 64);
+    a = swap_sum<16>(a); b = swap_sum<16>(b);
+    c = swap_sum<16>(c); d = swap_sum<16>(d);
   }
   if (G >= 64) {
-    a += __shfl_xor(a, 32, 64); b += __shfl_xor(b, 32, 64);
-    c += __shfl_xor(c, 32, 64); d += __shfl_xor(d, 32, 64);
+    a = swap_sum<32>(a); b = swap_sum<32>(b);
+    c = swap_sum<32>(c); d = swap_sum<32>(d);
   }
 }
 

@@ -852,15 +852,18 @@ struct Workspace {
     const size_t pairs = (size_t)(r + 1) / 2;
     return pairs * (pairs + 1) / 2 * 64 + 64 * 24 + (size_t)r * 24;
   }
-  // small_svd_kernel's QR phase needs M and 64 bytes per column; then Y (n x r
-  // with an odd leading dimension), then the Gram Jacobi, r <= min(m, n)
-  static size_t small_qr_lds(int m, int n) { return (size_t)m * n * 16 + (size_t)n * 64; }
+  // small_svd_kernel needs the pivot column and the QR's scalars, then Y
+  // (n x r with an odd leading dimension) where that fits, then the Gram
+  // Jacobi, r <= min(m, n)
   static size_t small_lds(int m, int n) {
     const int r = std::min(m, n);
-    return std::max({small_qr_lds(m, n), (size_t)(n | 1) * r * 16, gram_lds(r)});
+    const size_t y = (size_t)(n | 1) * r * 16;
+    return std::max({kSmallQrLds, y <= kSmallLdsMax ? y : 0, gram_lds(r)});
   }
+  // M fits the registers of one workgroup: 2.8 us a step at 88 x 83 and 6.1 at
+  // 128 x 126, where qrcp_kernel takes 7 to 9 us, so the limit is what fits.
   bool small_ok(int m, int n) const {
-    return small_enabled && n <= kSmallMaxCols && small_qr_lds(m, n) <= kSmallLdsMax;
+    return small_enabled && n <= kSmallMaxCols && m <= kSmallRows * small_lanes(n);
   }
 
   // Rotation log of a Gram Jacobi of rank at most r (in gpart, which the
@@ -898,8 +901,21 @@ struct Workspace {
     sa.copy = copy;
     sa.stop_rel = 0.0;
     sa.folded = nullptr;
+    sa.lds_bytes = (long)small_lds(m, n);
     gram_log(rmax, &sa.logs, &sa.logc);
     return sa;
+  }
+
+  // the Jacobi of a rank above kGramSmallRank after small_svd_kernel's QR
+  GramSvdArgs small_rest(const SmallSvdArgs& sa) const {
+    GramSvdArgs ga;
+    ga.Y = sa.Y; ga.n = sa.n; ga.r = std::min(sa.m, sa.n); ga.pending = 1;
+    ga.sigma = sa.sigma; ga.perm = sa.perm; ga.sorted = sa.sorted; ga.info = sa.info;
+    ga.epsrel = sa.epsrel; ga.max_rank = sa.max_rank; ga.max_sweeps = sa.max_sweeps;
+    ga.copy = sa.copy;
+    ga.extra2 = sa.folded;
+    ga.logc = sa.logc; ga.logs = sa.logs;
+    return ga;
   }
 
   // after synchronisation (summary in info_h): the same checks, statistics
@@ -928,6 +944,9 @@ struct Workspace {
     const bool timed = trace != nullptr;
     if (timed) mark(evj0);
     small_svd_kernel<<<1, kSmallThreads, small_lds(m, n), svd_stream>>>(sa);
+    if (std::min(m, n) > kGramSmallRank)
+      gram_svd_kernel<<<1, kGramThreads, gram_lds(std::min(m, n)), svd_stream>>>(
+          small_rest(sa));
     gram_replay_kernel<<<replay_grid(n, std::min(m, n)), 256, 0, svd_stream>>>(
         replay_args(n, sa.logc, sa.logs));
     if (timed) mark(evj1);
@@ -963,7 +982,7 @@ struct Workspace {
     ensure_sv((size_t)r);
     V.ensure((size_t)r * r, svd_stream);
     GramSvdArgs ga;
-    ga.Y = X.p; ga.n = n; ga.r = r;
+    ga.Y = X.p; ga.n = n; ga.r = r; ga.pending = 0;
     ga.sigma = sigma; ga.perm = perm; ga.sorted = sorted; ga.info = info_d;
     ga.epsrel = epsrel; ga.max_rank = chi_cap;
     ga.max_sweeps = std::min(max_sweeps, kGramMaxSweeps);
@@ -978,7 +997,7 @@ struct Workspace {
     GramSvdArgs ga = gram_prepare(n, r, nullptr);
     const bool timed = trace != nullptr;
     if (timed) mark(evj0);
-    gram_svd_kernel<<<1, 1024, gram_lds(r), svd_stream>>>(ga);
+    gram_svd_kernel<<<1, kGramThreads, gram_lds(r), svd_stream>>>(ga);
     gram_replay_kernel<<<replay_grid(n, r), 256, 0, svd_stream>>>(
         replay_args(n, ga.logc, ga.logs));
     if (timed) mark(evj1);
@@ -1362,15 +1381,20 @@ struct Batcher {
   void run_small(std::vector<SvdRequest*>& rs, std::vector<SvdRequest*>* blocked) {
     ensure_gather(rs.size());
     std::vector<SmallSvdArgs> args;
+    std::vector<GramSvdArgs> rest;
     std::vector<GramReplayArgs> reps;
     std::vector<SvdRequest*> in;
-    size_t lds = 0;
+    size_t lds = 0, rest_lds = 0;
     unsigned gx = 1;
     for (auto* r : rs) {
       try {
         args.push_back(r->ws->small_prepare(r->m, r->n, infos_d + in.size()));
         reps.push_back(r->ws->replay_args(r->n, args.back().logc, args.back().logs));
         lds = std::max(lds, Workspace::small_lds(r->m, r->n));
+        if (std::min(r->m, r->n) > kGramSmallRank) {
+          rest.push_back(r->ws->small_rest(args.back()));
+          rest_lds = std::max(rest_lds, Workspace::gram_lds(rest.back().r));
+        }
         gx = std::max(gx, Workspace::replay_grid(r->n, std::min(r->m, r->n)));
         in.push_back(r);
       } catch (...) {
@@ -1378,13 +1402,18 @@ struct Batcher {
       }
     }
     if (in.empty()) return;
+    for (auto& sa : args) sa.lds_bytes = (long)lds;
     Pack pk;
     const size_t oa = pk.add(args.data(), args.size() * sizeof(SmallSvdArgs));
     const size_t orp = pk.add(reps.data(), reps.size() * sizeof(GramReplayArgs));
+    const size_t ore = pk.add(rest.data(), rest.size() * sizeof(GramSvdArgs));
     char* base = upload(pk);
     HIP_CHECK(hipEventRecord(ev0, stream));
-    small_svd_batch_kernel<<<(unsigned)in.size(), kSmallBatchThreads, lds, stream>>>(
+    small_svd_batch_kernel<<<(unsigned)in.size(), kSmallThreads, lds, stream>>>(
         reinterpret_cast<const SmallSvdArgs*>(base + oa));
+    if (!rest.empty())
+      gram_svd_batch_kernel<<<(unsigned)rest.size(), kGramThreads, rest_lds, stream>>>(
+          reinterpret_cast<const GramSvdArgs*>(base + ore));
     gram_replay_batch_kernel<<<dim3(gx, (unsigned)in.size()), 256, 0, stream>>>(
         reinterpret_cast<const GramReplayArgs*>(base + orp));
     gather(in, [](SvdRequest* r, float ms) { return r->ws->small_finish(r->m, r->n, ms); },
@@ -1421,7 +1450,7 @@ struct Batcher {
     const size_t orp = pk.add(reps.data(), reps.size() * sizeof(GramReplayArgs));
     char* base = upload(pk);
     HIP_CHECK(hipEventRecord(ev0, stream));
-    gram_svd_batch_kernel<<<(unsigned)in.size(), 1024, lds, stream>>>(
+    gram_svd_batch_kernel<<<(unsigned)in.size(), kGramThreads, lds, stream>>>(
         reinterpret_cast<const GramSvdArgs*>(base + oa));
     gram_replay_batch_kernel<<<dim3(gx, (unsigned)in.size()), 256, 0, stream>>>(
         reinterpret_cast<const GramReplayArgs*>(base + orp));

@@ -143,14 +143,17 @@ struct SmallSvdArgs {
   SvdInfo* copy;    // optional second copy of the summary (batched gather)
   double stop_rel;  // > 0: stop the QR at residual <= stop_rel * |beta_0|
   double* folded;   // optional: the squared residual of that stop
+  long lds_bytes;   // dynamic LDS of the launch (Y goes through it when it fits)
   double* logc; double2* logs;
 };
 
 // Jacobi SVD of Y = R^H (n x r, ld n) of a pivoted QR on its Gram matrix, in
 // one workgroup (gram_svd_kernel): sigma, perm, sorted, info and the rotation
-// log (64 rotations per round).
+// log (64 rotations per round). With `pending`, r is an upper bound: the rank
+// is info->pad, and there is nothing to do unless info->sweeps is 0.
 struct GramSvdArgs {
   const double2* Y; int n, r;
+  int pending;
   double* sigma; int* perm; double* sorted; SvdInfo* info;
   double epsrel; int max_rank; int max_sweeps;
   SvdInfo* copy;
@@ -169,9 +172,16 @@ struct GramReplayArgs {
 
 constexpr int kGramMaxRank = 126;           // G in LDS, two blocks of it per thread
 constexpr int kGramMaxSweeps = 20;          // sweeps the rotation log holds
-constexpr int kSmallMaxCols = 96;           // columns of M in small_svd_kernel
-constexpr int kSmallThreads = 1024;         // workgroup of small_svd_kernel
-constexpr int kSmallBatchThreads = 512;     // workgroup of small_svd_batch_kernel
+constexpr int kSmallMaxCols = kGramMaxRank; // columns of M in small_svd_kernel
+constexpr int kSmallThreads = 512;          // its workgroup
+constexpr int kGramThreads = 1024;          // workgroup of gram_svd_kernel
+constexpr int kGramSmallRank = 88;          // ranks small_svd_kernel finishes itself
+constexpr int kSmallRows = 40;              // rows of M a lane holds at most
+constexpr size_t kSmallQrLds = 64 * kSmallRows * 16 + 2048;   // LDS of its QR
+// lanes per column of small_svd_kernel's QR
+__host__ __device__ constexpr int small_lanes(int n) {
+  return n > 64 ? 4 : n > 32 ? 8 : n > 16 ? 16 : n > 8 ? 32 : 64;
+}
 
 struct ZeroItem {
   unsigned* p; int words; int pad;

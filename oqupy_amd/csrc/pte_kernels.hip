@@ -31,9 +31,10 @@ __device__ unsigned long long g_phase[16];
       ph_t_ = t_;                                                      \
     }                                                                  \
   } while (0)
-// Segment cycle counts of the one-workgroup SVD (thread 0, s_memtime), in
-// the same build: SEG_INIT() starts, SEG(k) adds the cycles since the last
+// Segment cycle counts of the one-workgroup SVD (thread 0, s_memtime), with
+// -DPTE_SEG_TIMING besides (their reads of the clock lengthen the steps): SEG_INIT() starts, SEG(k) adds the cycles since the last
 // mark to slot k, SEG_FLUSH(k0, n) adds slots k0.. to g_phase.
+#ifdef PTE_SEG_TIMING
 #define SEG_INIT()                                 \
   unsigned long long sg_[6] = {0, 0, 0, 0, 0, 0}; \
   unsigned long long sg_t_ = clock64()
@@ -48,6 +49,11 @@ __device__ unsigned long long g_phase[16];
     if (threadIdx.x == 0)                                                  \
       for (int k_ = 0; k_ < (cnt); ++k_) atomicAdd(&g_phase[(k0) + k_], sg_[k_]); \
   } while (0)
+#else
+#define SEG_INIT() (void)0
+#define SEG(k) (void)0
+#define SEG_FLUSH(k0, cnt) (void)0
+#endif
 #else
 #define PHASE_INIT() (void)0
 #define PHASE(k) (void)0
@@ -481,19 +487,17 @@ __device__ __forceinline__ bool needs_rotation(double app, double aqq, double ma
          mag2 > 0.0;
 }
 
-// 1/sqrt(x) and 1/x for normal positive x: the hardware estimates refined
-// by Newton steps (quadratic convergence) to full double precision.
+// 1/sqrt(x) and 1/x for normal positive x: the hardware estimates (measured
+// relative error 2^-24) refined by one cubic step to full double precision.
 __device__ __forceinline__ double rsqrt_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  y = y * fma(-0.5 * x * y, y, 1.5);
-  y = y * fma(-0.5 * x * y, y, 1.5);
-  return y;
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
 }
 __device__ __forceinline__ double rcp_nr(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = y * fma(-x, y, 2.0);
-  y = y * fma(-x, y, 2.0);
-  return y;
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(fma(e, e, e), y, y);
 }
 
 // Rotation of that block: J = [[cs, sn], [-sn conj(ph), cs conj(ph)]],
@@ -543,17 +547,9 @@ __device__ __forceinline__ bool jacobi_rotation_fast(bool valid, double app, dou
   const double m2 = need ? cabs2(c) : 1.0;
   const double d = (aqq - app) * sc;
   const double h2 = fma(d, d, 4.0 * m2);
-  // 1 / |apq| and 1 / h: hardware estimates and two Newton steps each
-  double inv = __builtin_amdgcn_rsq(m2), rh = __builtin_amdgcn_rsq(h2);
-#pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    inv = inv * fma(-0.5 * m2 * inv, inv, 1.5);
-    rh = rh * fma(-0.5 * h2 * rh, rh, 1.5);
-  }
-  const double cos2 = fma(0.5 * fabs(d), rh, 0.5);   // cos^2(theta)
-  double rc = __builtin_amdgcn_rsq(cos2);             // 1 / cos(theta)
-#pragma unroll
-  for (int it = 0; it < 2; ++it) rc = rc * fma(-0.5 * cos2 * rc, rc, 1.5);
+  const double inv = rsqrt_nr(m2), rh = rsqrt_nr(h2);   // 1 / |apq|, 1 / h
+  const double cos2 = fma(0.5 * fabs(d), rh, 0.5);      // cos^2(theta)
+  const double rc = rsqrt_nr(cos2);                     // 1 / cos(theta)
   const double sn = copysign(m2 * inv * rh * rc, d < 0.0 ? -1.0 : 1.0);
   r[0] = need ? cos2 * rc : 1.0;
   r[1] = need ? sn : 0.0;
@@ -1956,20 +1952,11 @@ build_rh_batch_kernel(const RhArgs* pa) {
 }
 
 // ---------------------------------------------------------------------------
-// Small truncated SVD in one workgroup of NT threads (M with at most
-// kSmallMaxCols columns, staged in LDS): the pivoted QR of qrcp_kernel (same
-// reflectors, pivoting, norm downdating and eps-rank stop), then the Jacobi
-// of Y = R^H (n x r) on its Gram matrix in the same LDS (below), singular
-// values, order and cut. Barriers are workgroup barriers only; the QR's
-// columns are reduced by lane groups with wavefront shuffles.
+// Small truncated SVD in one workgroup (M with at most kSmallMaxCols columns and
+// kSmallRows rows per lane of a column, see small_lanes): the pivoted QR with
+// M in registers (small_qr), then the Jacobi of Y = R^H (n x r) on its Gram
+// matrix in LDS (below), singular values, order and cut.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double group_sum(double v, int G) { return group_sum1(v, G); }
-
-__device__ __forceinline__ int pow2_ceil(int x) {
-  int p = 1;
-  while (p < x) p <<= 1;
-  return p;
-}
 
 // ---------------------------------------------------------------------------
 // Jacobi SVD of Y = R^H (n x r, r <= kGramMaxRank) of a pivoted QR in one
@@ -2054,15 +2041,23 @@ __device__ __forceinline__ void gram_tile(const double2* Y, long ld, int n, int 
   const double2* yi = Y + (long)min(ci, r - 1) * ld;
   const double2* yj = Y + (long)min(cj, r - 1) * ld;
   doublex4 p1 = {0.0, 0.0, 0.0, 0.0}, p2 = p1, p3 = p1;
-#pragma unroll 4
-  for (int k4 = 0; k4 < n; k4 += 4) {
-    const int k = k4 + lk;
-    double2 x = yi[min(k, n - 1)], y = yj[min(k, n - 1)];
-    if (k >= n || ci >= r) x = make_double2(0.0, 0.0);
-    if (k >= n || cj >= r) y = make_double2(0.0, 0.0);
-    p1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, y.x, p1, 0, 0, 0);
-    p2 = __builtin_amdgcn_mfma_f64_16x16x4f64(-x.y, y.y, p2, 0, 0, 0);
-    p3 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x - x.y, y.x + y.y, p3, 0, 0, 0);
+  // four slices of four rows loaded together
+  for (int k4 = 0; k4 < n; k4 += 16) {
+    double2 x[4], y[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int k = k4 + 4 * q + lk;
+      x[q] = yi[min(k, n - 1)];
+      y[q] = yj[min(k, n - 1)];
+      if (k >= n || ci >= r) x[q] = make_double2(0.0, 0.0);
+      if (k >= n || cj >= r) y[q] = make_double2(0.0, 0.0);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      p1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x[q].x, y[q].x, p1, 0, 0, 0);
+      p2 = __builtin_amdgcn_mfma_f64_16x16x4f64(-x[q].y, y[q].y, p2, 0, 0, 0);
+      p3 = __builtin_amdgcn_mfma_f64_16x16x4f64(x[q].x - x[q].y, y[q].x + y[q].y, p3, 0, 0, 0);
+    }
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) g[q] = make_double2(p1[q] - p2[q], p3[q] - p1[q] - p2[q]);
@@ -2085,6 +2080,27 @@ __device__ __forceinline__ void gram_store(double2* G, int r, int t, const doubl
     const double im = i == j ? 0.0 : g[q].y;
     G[at] = make_double2(g[q].x, conj ? -im : im);
   }
+}
+
+// Rotation of the 2 x 2 block [[app, apq], [conj(apq), aqq]]: with
+// d = aqq - app and h = sqrt(d^2 + 4 |apq|^2), c = cos(theta) =
+// sqrt((h + |d|) / 2h) and s = sign(d) apq / (h c) (jacobi_rotation_fast's
+// formulas; the phase of apq stays in s, so its modulus is not needed, and G is
+// scaled, so the block is not). The identity where no rotation is needed.
+__device__ __forceinline__ void gram_rotation(bool valid, double app, double aqq, double2 apq,
+                                              double tol2, double abs_tol2, double& c,
+                                              double2& s) {
+  const double mag2 = cabs2(apq);
+  const bool need = valid & (mag2 > tol2 * fabs(app * aqq)) &
+                    (mag2 > abs_tol2 * fmax(fmax(app, aqq), 0.0)) & (mag2 > 0.0);
+  const double d = aqq - app;
+  const double h2 = need ? fma(d, d, 4.0 * mag2) : 1.0;
+  const double rh = rsqrt_nr(h2);
+  const double cos2 = fma(0.5 * fabs(d), rh, 0.5);
+  const double rc = rsqrt_nr(cos2);
+  const double f = copysign(rh * rc, d < 0.0 ? -1.0 : 1.0);
+  c = need ? cos2 * rc : 1.0;
+  s = make_double2(need ? apq.x * f : 0.0, need ? apq.y * f : 0.0);
 }
 
 // Two-sided Jacobi sweeps on G (rank r) in LDS; rc, rs: LDS scratch of 64
@@ -2163,16 +2179,15 @@ __device__ __forceinline__ int gram_jacobi(double2* G, int r, double tol2, doubl
       if (wave == 0) {
         const bool valid = lane < P;
         const int d = gram_block(min(lane, P - 1), min(lane, P - 1));
-        double rot[4];
-        (void)jacobi_rotation_fast(valid, G[d].x, G[3 * T + d].x, G[T + d], tol2, abs_tol2,
-                                   rot);
-        const double2 s = make_double2(rot[1] * rot[2], rot[1] * rot[3]);
+        double c;
+        double2 sn;
+        gram_rotation(valid, G[d].x, G[3 * T + d].x, G[T + d], tol2, abs_tol2, c, sn);
         if (valid) {
-          rc[lane] = rot[0];
-          rs[lane] = s;
+          rc[lane] = c;
+          rs[lane] = sn;
           const long e = (long)(sweeps * L + t) * 64 + lane;
-          logc[e] = rot[0];
-          logs[e] = s;
+          logc[e] = c;
+          logs[e] = sn;
         }
       }
       __syncthreads();
@@ -2317,18 +2332,35 @@ __device__ __forceinline__ void gram_finish(const double2* G, int r, double epsr
   }
 }
 
-constexpr int kGramThreads = 1024;
-// pair blocks per thread: 2016 at r = 126, two for each of 1024 threads (a third
-// does not fit the 128 registers of a thread)
-constexpr int kGramBlocks = 2;
-
-__device__ __forceinline__ void gram_svd_body(const GramSvdArgs& a) {
-  extern __shared__ double2 lds_gram[];
-  const int r = a.r;
-  double2* G = lds_gram;
+// Rest of the SVD after the Gram matrix: the whole workgroup of NT threads, NB
+// blocks of G per thread at most.
+template <int NT, int NB, class Args>
+__device__ __forceinline__ void gram_run(const Args& a, double2* G, int n, int r,
+                                         double extra2) {
   double2* rs = G + gram_entries(r);
   double* rc = reinterpret_cast<double*>(rs + 64);
   double* s_sig = rc + 64;
+  int half;
+  const double tr = gram_scale<NT>(G, r, &half);
+  const double eps = 2.220446049250313e-16;
+  const double tol = (n > 16 ? n : 16) * eps;
+  bool converged = false;
+  const int sweeps = gram_jacobi<NT, NB>(G, r, tol * tol, eps * eps * tr, a.max_sweeps, rc, rs,
+                                         a.logc, a.logs, converged);
+  gram_finish<NT>(G, r, a.epsrel, a.max_rank, extra2, sweeps,
+                  sweeps * (max(2, r + (r & 1)) - 1), converged, half, s_sig, s_sig + r,
+                  s_sig + 2 * r, a.sigma, a.perm, a.sorted, a.info, a.copy);
+}
+
+// 1024 threads: at ranks above kGramSmallRank the rotations' FP64 issue and the
+// LDS traffic of G set the time of a round, not its barriers (112: 1.35 us a
+// round, 1.7 us with 512 threads; 74: 0.92 us and 0.96; 35: 0.68 us and 0.64).
+__device__ __forceinline__ void gram_svd_body(const GramSvdArgs& a) {
+  extern __shared__ double2 lds_gram[];
+  // the rank and the matrix of the one-workgroup QR, if that left them here
+  if (a.info->sweeps != 0 && a.pending) return;
+  const int r = __builtin_amdgcn_readfirstlane(a.pending ? a.info->pad : a.r);
+  double2* G = lds_gram;
   for (int e = threadIdx.x; e < gram_entries(r); e += kGramThreads)
     G[e] = make_double2(0.0, 0.0);
   __syncthreads();
@@ -2339,17 +2371,8 @@ __device__ __forceinline__ void gram_svd_body(const GramSvdArgs& a) {
     gram_store(G, r, t, g);
   }
   __syncthreads();
-  int half;
-  const double tr = gram_scale<kGramThreads>(G, r, &half);
-  const double eps = 2.220446049250313e-16;
-  const double tol = (a.n > 16 ? a.n : 16) * eps;
-  bool converged = false;
-  const int sweeps = gram_jacobi<kGramThreads, kGramBlocks>(
-      G, r, tol * tol, eps * eps * tr, a.max_sweeps, rc, rs, a.logc, a.logs, converged);
-  const int L = max(2, r + (r & 1)) - 1;
-  gram_finish<kGramThreads>(G, r, a.epsrel, a.max_rank, a.extra2 ? *a.extra2 : 0.0, sweeps,
-                            sweeps * L, converged, half, s_sig, s_sig + r, s_sig + 2 * r, a.sigma,
-                            a.perm, a.sorted, a.info, a.copy);
+  // 2016 blocks at rank 126
+  gram_run<kGramThreads, 2>(a, G, a.n, r, a.extra2 ? *a.extra2 : 0.0);
 }
 
 __global__ void __launch_bounds__(kGramThreads)
@@ -2453,199 +2476,265 @@ gram_replay_batch_kernel(const GramReplayArgs* probs) {
   gram_replay_body(a, blockIdx.x * 4 + (threadIdx.x >> 6));
 }
 
-template <int NT>
-__device__ void small_svd_body(const SmallSvdArgs& a) {
-  static_assert(NT % 64 == 0, "workgroup size");
-  extern __shared__ double2 lds_small[];
-  __shared__ double s_folded;       // residual of an adaptive stop (folded2)
-  const int m = a.m, n = a.n, tid = threadIdx.x, lane = tid & 63;
-  // QR phase: M (m x n, ld m), then the per-column scalars (64 n bytes)
-  double2* As = lds_small;
-  double2* q_tau = As + (long)m * n;
-  double2* q_vscale = q_tau + n;
-  double* vn1 = reinterpret_cast<double*>(q_vscale + n);
-  double* vn2 = vn1 + n;
-  double* q_beta = vn2 + n;
-  int* done = reinterpret_cast<int*>(q_beta + n);
-  int* q_piv = done + n;
-  const double eps = 2.220446049250313e-16;
+// ---------------------------------------------------------------------------
+// Pivoted Householder QR of M (m x n) with M in registers: G = 2^lg lanes per
+// column (small_lanes), lane g of a group holding rows g + G u, u < RP. The
+// reflectors (zlarfg) and the eps-rank stop are qrcp_kernel's; the residual
+// norms are summed anew in every step (two FMAs a row, in place of the
+// downdate's square root and division and of a pass over the pivot column), and
+// the pivot is the first column whose squared norm has the largest upper word
+// (within 1e-6 of the largest). A step:
+//   (1) each group has the norm, first entry and reflector scalars of its
+//       remaining rows; each wavefront posts its largest column to LDS; barrier;
+//   (2) every wavefront picks the winner of the posts; the winner's group
+//       writes its column to LDS; barrier;
+//   (3) every group applies the reflector to its column.
+// Row j (row u = j / G of lane j % G) is taken out of the registers before step
+// j and stored as R's when the step is done, so registers of finished rows are
+// zero: the inner product, the update and the norm run over all RP rows without
+// masks or branches, and the pivot column is copied to LDS whole, as
+// [u][64 lanes]. (Skipping the finished rows took 1550 instructions a step at
+// 12 rows a lane, two thirds of them branches, masks and register copies.) The
+// reflector is used unscaled, its scale (vscale, as in the factors of
+// qrcp_kernel) folded into the scalars.
+// 512 threads: a workgroup barrier costs 86 cycles with 8 wavefronts, 326 with
+// 16 and 11 with 4, and 256 threads would not hold M.
+// Bound by the chain of a step (two barriers, two passes through LDS, the
+// reductions and the reflector's scalars): 1.7 us a step at 24 x 24, 1.9 at
+// 40 x 44, 2.8 at 88 x 83, where M in LDS took 3.0, 3.2 and 4.4.
+// ---------------------------------------------------------------------------
+struct SmallCand {
+  double2 tau, scale;
+  double sum, beta;
+  unsigned key;      // upper word of the squared norm
+  int col;
+  int pad[2];
+};
+constexpr int kSmallWaves = kSmallThreads / 64;
+static_assert(kSmallWaves == 8, "the posts are reduced over groups of 8 lanes");
+static_assert(64 * kSmallRows * 16 + kSmallWaves * (int)sizeof(SmallCand) +
+                  2 * 128 * (int)sizeof(int) <= (int)kSmallQrLds, "LDS of the QR");
 
-  PHASE_INIT();
-  for (long e = tid; e < (long)m * n; e += NT) As[e] = a.A[e];
-  __syncthreads();
-  PHASE(6);
-  // ---- pivoted QR in LDS ----
-  const int NP = pow2_ceil(n);
-  // threads per column: at most 64, at most NT / NP, no more than the rows
-  const int G = min(min(NP >= NT / 64 ? NT / NP : 64, pow2_ceil(m)), 64);
-  const int myc = tid / G, g = tid % G;
-  {
-    double part = 0.0;
-    if (myc < n)
-      for (int i = g; i < m; i += G) part += cabs2(As[i + (long)myc * m]);
-    const double nrm = sqrt(group_sum(part, G));
-    if (myc < n && g == 0) { vn1[myc] = nrm; vn2[myc] = nrm; done[myc] = 0; }
+// 1/x and 1/sqrt(x): refined estimates where they are safe, else the division
+__device__ __forceinline__ double rcp_safe(double x) {
+  return (x > 1e-290 && x < 1e290) ? rcp_nr(x) : 1.0 / x;
+}
+__device__ __forceinline__ double rsqrt_safe(double x) {
+  return (x > 1e-290 && x < 1e290) ? rsqrt_nr(x) : 1.0 / sqrt(x);
+}
+
+template <int RP>
+__device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, double2* vcol,
+                                        SmallCand* cand, int* s_piv, int* s_done,
+                                        double& folded2) {
+  // up to 24 rows the reflector's rows stay in registers between the inner
+  // product and the update, else they are read again
+  constexpr bool kKeep = RP <= 24;
+  const int m = a.m, n = a.n, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int G = 1 << lg;
+  const int myc = tid >> lg, g = tid & (G - 1);
+  const double eps = 2.220446049250313e-16;
+  const int kmax = min(m, n);
+  bool alive = myc < n;
+  int myt = -1;                       // step at which the own column was pivoted
+  double2 col[RP];
+#pragma unroll
+  for (int u = 0; u < RP; ++u) {
+    const int i = g + G * u;
+    col[u] = make_double2(0.0, 0.0);
+    if (alive && i < m) col[u] = a.A[i + (long)myc * m];
   }
-  __syncthreads();
-  // Each step takes two barriers: after the first, every wavefront reads the
-  // step's pivot and reflector from LDS and the group of each remaining
-  // column applies the reflector to it and downdates its norm; after the
-  // second, wavefront 0 alone chooses the next pivot (largest residual norm,
-  // ties to the smaller column), decides whether to stop, computes the next
-  // reflector and stores it into the pivot column already scaled (v_i =
-  // M_ij * scale below the diagonal, so vscale is 1), so the scalar work is
-  // not repeated by every wavefront.
-  __shared__ int s_ctl[2];          // pivot column, 1 while the QR continues
-  __shared__ double2 s_tau;
-  const int wave = tid >> 6;
-  int j = 0;
-  // adaptive stop (stop_rel > 0): once the residual is at most
-  // stop_rel * |beta_0|; the residual is then counted in the cut (folded2,
-  // used by thread 0 only)
-  double drop2 = 0.0, stop2 = -1.0, folded2 = 0.0;
-  const double tol3z = 1.4901161193847656e-08;
-  const int kmax = m < n ? m : n;
-  // wavefront 0: pivot and reflector of step j, or the stop
-  auto pivot_step = [&]() {
-    double bv = -1.0, sv = 0.0;
-    int bc = -1;
-    for (int c = lane; c < n; c += 64)
-      if (!done[c]) { sv += vn1[c] * vn1[c]; better(bv, bc, vn1[c], c); }
-    better(bv, bc, dpp_d<kDppXor1>(bv), dpp_i<kDppXor1>(bc));
-    better(bv, bc, dpp_d<kDppXor2>(bv), dpp_i<kDppXor2>(bc));
-    better(bv, bc, dpp_d<kDppHalfMirror>(bv), dpp_i<kDppHalfMirror>(bc));
-    better(bv, bc, dpp_d<kDppMirror>(bv), dpp_i<kDppMirror>(bc));
-    better(bv, bc, __shfl_xor(bv, 16, 64), __shfl_xor(bc, 16, 64));
-    better(bv, bc, __shfl_xor(bv, 32, 64), __shfl_xor(bc, 32, 64));
-    const int p = bc;
-    const double total = wave_sum(sv);
-    if (j == 0) drop2 = eps * eps * total;
-    bool go;
-    if (a.stop_rel > 0.0 && j >= 1) {
-      if (j == 1) stop2 = (a.stop_rel * q_beta[0]) * (a.stop_rel * q_beta[0]);
-      if (total <= stop2) {
-        folded2 = (p >= 0 && j < kmax) ? total : 0.0;
-        go = false;
-      } else {
-        go = j < kmax && p >= 0 && total > drop2;
-      }
-    } else {
-      go = j < kmax && p >= 0 && total > drop2;
-    }
-    if (go) {
-      double2* pc = As + (long)p * m;
-      double part = 0.0;
-      for (int i = j + 1 + lane; i < m; i += 64) part += cabs2(pc[i]);
-      const double xnorm2 = wave_sum(part);
-      const double2 alpha = pc[j];
-      double2 tau, scale;
-      double beta;
-      if (xnorm2 == 0.0 && alpha.y == 0.0) {
-        tau = make_double2(0.0, 0.0);
-        scale = make_double2(0.0, 0.0);
-        beta = alpha.x;
-      } else {
-        beta = -copysign(sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xnorm2), alpha.x);
-        const double dr = alpha.x - beta, di = alpha.y;
-        const double den = dr * dr + di * di;
-        scale = make_double2(dr / den, -di / den);
-        tau = make_double2((beta - alpha.x) / beta, -alpha.y / beta);
-      }
-      for (int i = j + 1 + lane; i < m; i += 64) pc[i] = cmul(pc[i], scale);
-      if (lane == 0) {
-        q_piv[j] = p;
-        q_tau[j] = tau;
-        q_vscale[j] = make_double2(1.0, 0.0);
-        q_beta[j] = beta;
-        s_tau = tau;
-        s_ctl[0] = p;
+  for (int c = tid; c < n; c += kSmallThreads) s_done[c] = 0;
+  // takes row jn out (cj: its entry, in the lane that held it), then the norm,
+  // reflector scalars and post of step jn
+  double2 cj = make_double2(0.0, 0.0);
+  auto post = [&](int jn) __attribute__((always_inline)) {
+    const int uj = jn >> lg;
+    const bool here = alive && g == (jn & (G - 1));
+    cj = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int u = 0; u < RP; ++u) {
+      if (u == uj) {
+        cj = make_double2(here ? col[u].x : 0.0, here ? col[u].y : 0.0);
+        col[u] = make_double2(here ? 0.0 : col[u].x, here ? 0.0 : col[u].y);
       }
     }
-    if (lane == 0) s_ctl[1] = go ? 1 : 0;
+    double tail = 0.0, tail1 = 0.0, ax = cj.x, ay = cj.y;
+#pragma unroll
+    for (int u = 0; u < RP; ++u) {
+      tail = fma(col[u].x, col[u].x, tail);
+      tail1 = fma(col[u].y, col[u].y, tail1);
+    }
+    tail += tail1;
+    double z = 0.0;
+    group_sum4(tail, ax, ay, z, G);
+    const double norm2 = alive ? tail + fma(ax, ax, ay * ay) : 0.0;
+    // largest column of the wavefront: its norms are the same bits in all lanes
+    // of a group, so the first lane with the largest key is lane 0 of a group
+    unsigned key = (unsigned)__double2hiint(norm2);
+    const unsigned mykey = key;
+    double sv = norm2;
+    if (G <= 4) { key = max(key, (unsigned)dpp_i<kDppHalfMirror>((int)key)); sv += dpp_d<kDppHalfMirror>(sv); }
+    if (G <= 8) { key = max(key, (unsigned)dpp_i<kDppMirror>((int)key)); sv += dpp_d<kDppMirror>(sv); }
+    if (G <= 16) { key = swap_max<16>(key); sv = swap_sum<16>(sv); }
+    if (G <= 32) { key = swap_max<32>(key); sv = swap_sum<32>(sv); }
+    const unsigned long long at = __ballot(alive && mykey == key);
+    double beta = ax;
+    double2 tau = make_double2(0.0, 0.0), scale = make_double2(0.0, 0.0);
+    if (tail != 0.0 || ay != 0.0) {
+      const double inv = rsqrt_safe(norm2);
+      const double ib = -copysign(inv, ax);        // 1 / beta
+      beta = -copysign(norm2 * inv, ax);
+      const double dr = ax - beta;
+      const double id = rcp_safe(fma(dr, dr, ay * ay));
+      scale = make_double2(dr * id, -ay * id);
+      tau = make_double2(-dr * ib, -ay * ib);
+    }
+    if (lane == (at ? __ffsll(at) - 1 : 0)) {
+      SmallCand* cd = cand + wave;
+      cd->tau = tau;
+      cd->scale = scale;
+      cd->sum = sv;
+      cd->beta = beta;
+      cd->key = key;
+      cd->col = at ? myc : -1;
+    }
   };
+  post(0);
   SEG_INIT();
-  if (wave == 0) pivot_step();
-  SEG(0);
+  double drop2 = 0.0, stop2 = -1.0;
+  folded2 = 0.0;
+  int j = 0;
   for (;;) {
     __syncthreads();
-    SEG(1);
-    if (!s_ctl[1]) break;
-    const int p = s_ctl[0];
-    const double2 tau = s_tau;
-    const double2* pv = As + (long)p * m;   // reflector, v_j = 1 implicit
-    const bool reflect = (tau.x != 0.0 || tau.y != 0.0);
-    // the group of column myc applies H_j^H and downdates the column norm;
-    // only that group touches the column, its norms and its done flag
-    if (myc < n && !done[myc]) {
-      if (myc == p) {
-        if (g == 0) done[myc] = 1;
-      } else {
-        double2* col = As + (long)myc * m;
-        double2 rj2 = col[j];
-        if (reflect) {
-          double2 w = make_double2(0.0, 0.0);
-#pragma unroll 4
-          for (int i = j + g; i < m; i += G) {
-            const double2 vi = (i == j) ? make_double2(1.0, 0.0) : pv[i];
-            cfmac(w, vi, col[i]);
-          }
-          {
-            double z0 = 0.0, z1 = 0.0;
-            group_sum4(w.x, w.y, z0, z1, G);
-          }
-          const double2 tw = cmul(make_double2(tau.x, -tau.y), w);
-#pragma unroll 4
-          for (int i = j + g; i < m; i += G) {
-            const double2 vi = (i == j) ? make_double2(1.0, 0.0) : pv[i];
-            col[i] = csub(col[i], cmul(vi, tw));
-          }
-          // row j of the column after the reflection (held by lane g = 0)
-          rj2 = csub(rj2, tw);
-        }
-        double nv = vn1[myc];
-        if (nv != 0.0) {
-          const double rj = sqrt(cabs2(rj2));
-          double temp = 1.0 - (rj / nv) * (rj / nv);
-          temp = temp > 0.0 ? temp : 0.0;
-          const double ratio = nv / vn2[myc];
-          if (temp * ratio * ratio <= tol3z) {
-            double pp = 0.0;
-            for (int i = j + 1 + g; i < m; i += G) pp += cabs2(col[i]);
-            nv = (j + 1 < m) ? sqrt(group_sum(pp, G)) : 0.0;
-            if (g == 0) { vn1[myc] = nv; vn2[myc] = nv; }
-          } else if (g == 0) {
-            vn1[myc] = nv * sqrt(temp);
-          }
-        }
+    SEG(0);
+    // the posts, replicated in every group of 8 lanes; ties go to the first
+    // wavefront, whose columns are the smaller ones
+    const SmallCand* cl = cand + (lane & (kSmallWaves - 1));
+    const int mcol = cl->col;
+    unsigned key = cl->key;
+    double total = cl->sum;
+    const unsigned mykey = key;
+    key = max(key, (unsigned)dpp_i<kDppXor1>((int)key));
+    total += dpp_d<kDppXor1>(total);
+    key = max(key, (unsigned)dpp_i<kDppXor2>((int)key));
+    total += dpp_d<kDppXor2>(total);
+    key = max(key, (unsigned)dpp_i<kDppHalfMirror>((int)key));
+    total += dpp_d<kDppHalfMirror>(total);
+    const unsigned long long at = __ballot(mcol >= 0 && mykey == key);
+    const int ws = at ? __ffsll(at) - 1 : 0;          // wavefront of the winner
+    const int p = at ? __builtin_amdgcn_readlane(mcol, ws) : -1;
+    // residual test; an adaptive stop (stop_rel > 0) ends at a residual of
+    // stop_rel * |beta_0| and counts it in the cut
+    if (j == 0) drop2 = eps * eps * total;
+    bool go = j < kmax && p >= 0 && total > drop2;
+    if (a.stop_rel > 0.0 && j >= 1 && total <= stop2) {
+      folded2 = (p >= 0 && j < kmax) ? total : 0.0;
+      go = false;
+    }
+    // (the same in every lane; said so, so that the loop, its step and all that
+    // hangs on them stay in scalar registers and scalar branches)
+    if (!__builtin_amdgcn_readfirstlane((int)go)) break;
+    const SmallCand* cw = cand + ws;
+    const double2 tau = cw->tau, scale = cw->scale;
+    if (j == 0) stop2 = (a.stop_rel * cw->beta) * (a.stop_rel * cw->beta);
+    if (alive && myc == p) {
+#pragma unroll
+      for (int u = 0; u < RP; ++u) vcol[64 * u + g] = col[u];
+      alive = false;
+      myt = j;
+      if (g == 0) {
+        s_piv[j] = p;
+        s_done[p] = 1;
+        a.tau[j] = tau;
+        a.vscale[j] = scale;
+        a.beta[j] = cw->beta;
       }
     }
-    SEG(2);
+    SEG(1);
     __syncthreads();
+    SEG(2);
+    if (alive) {
+      double2 pv[kKeep ? RP : 1];
+      double2 S = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int u = 0; u < RP; ++u) {
+        const double2 v = vcol[64 * u + g];
+        if constexpr (kKeep) pv[u] = v;
+        cfmac(S, v, col[u]);
+        // at most eight rows of the reflector in flight beside M's registers
+        if (!kKeep && u % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+      }
+      double2 w = cadd(cj, cmulc(scale, S));
+      double z0 = 0.0, z1 = 0.0;
+      group_sum4(w.x, w.y, z0, z1, G);
+      const double2 tw = cmulc(tau, w);
+      const double2 sv2 = cmul(scale, tw);
+      SEG(3);
+      if (!kKeep) asm volatile("" ::: "memory");
+#pragma unroll
+      for (int u = 0; u < RP; ++u) {
+        double2 v;
+        if constexpr (kKeep) v = pv[u];
+        else v = vcol[64 * u + g];
+        cfma(col[u], make_double2(-v.x, -v.y), sv2);
+        if (!kKeep && u % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+      }
+      if (g == (j & (G - 1))) a.A[j + (long)myc * m] = csub(cj, tw);
+    }
     ++j;
-    if (wave == 0) pivot_step();
-    SEG(3);
+    SEG(4);
+    post(j);
+    SEG(5);
   }
-  SEG_FLUSH(8, 4);
-  const int r = j;
-  PHASE(13);
-  if (tid == 0) {
-    int t = r;
-    for (int c = 0; c < n; ++c)
-      if (!done[c]) q_piv[t++] = c;
-    *a.qrank = r;
-  }
-  __syncthreads();
-  for (int t = tid; t < n; t += NT) {
-    a.piv[t] = q_piv[t];
-    if (t < r) {
-      a.tau[t] = q_tau[t];
-      a.vscale[t] = q_vscale[t];
-      a.beta[t] = q_beta[t];
+  SEG_FLUSH(0, 6);
+  // reflectors to global memory (apply_q_kernel reads them)
+  if (myt >= 0) {
+    // (opaque copy: the indices and masks of the loads above would otherwise be
+    // kept in registers through the loop for reuse here)
+    int g2 = g;
+    asm volatile("" : "+v"(g2));
+#pragma unroll
+    for (int u = 0; u < RP; ++u) {
+      const int i = g2 + G * u;
+      if (i > myt && i < m) a.A[i + (long)myc * m] = col[u];
     }
   }
-  // reflectors and R back to global memory (apply_q_kernel reads them)
-  for (long e = tid; e < (long)m * n; e += NT) a.A[e] = As[e];
+  // remaining columns in ascending order after the pivots
+  if (wave == 0) {
+    const bool r0 = lane < n && !s_done[lane], r1 = lane + 64 < n && !s_done[lane + 64];
+    const unsigned long long b0 = __ballot(r0), b1 = __ballot(r1);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    if (r0) s_piv[j + __popcll(b0 & below)] = lane;
+    if (r1) s_piv[j + __popcll(b0) + __popcll(b1 & below)] = lane + 64;
+  }
+  if (tid == 0) *a.qrank = j;
   __syncthreads();
+  for (int t = tid; t < n; t += kSmallThreads) a.piv[t] = s_piv[t];
+  return j;
+}
+
+__device__ __forceinline__ void small_svd_body(const SmallSvdArgs& a) {
+  constexpr int NT = kSmallThreads;
+  extern __shared__ double2 lds_small[];
+  const int m = a.m, n = a.n, tid = threadIdx.x, wave = tid >> 6;
+  // QR phase: the pivot column, the posts, pivots and done flags
+  double2* vcol = lds_small;
+  SmallCand* cand = reinterpret_cast<SmallCand*>(vcol + 64 * kSmallRows);
+  int* s_piv = reinterpret_cast<int*>(cand + kSmallWaves);
+  int* s_done = s_piv + 128;
+  PHASE_INIT();
+  const int lg = __builtin_amdgcn_readfirstlane(31 - __clz(small_lanes(n)));
+  const int rows = (m + (1 << lg) - 1) >> lg;
+  double folded2;
+  const int steps = rows <= 4 ? small_qr<4>(a, lg, vcol, cand, s_piv, s_done, folded2)
+                : rows <= 8  ? small_qr<8>(a, lg, vcol, cand, s_piv, s_done, folded2)
+                : rows <= 16 ? small_qr<16>(a, lg, vcol, cand, s_piv, s_done, folded2)
+                : rows <= 24 ? small_qr<24>(a, lg, vcol, cand, s_piv, s_done, folded2)
+                : rows <= 32 ? small_qr<32>(a, lg, vcol, cand, s_piv, s_done, folded2)
+                             : small_qr<kSmallRows>(a, lg, vcol, cand, s_piv, s_done, folded2);
+  PHASE(13);
+  const int r = __builtin_amdgcn_readfirstlane(steps);
   if (r == 0) {
     if (tid == 0) {
       SvdInfo inf;
@@ -2657,29 +2746,34 @@ __device__ void small_svd_body(const SmallSvdArgs& a) {
     }
     return;
   }
-  // ---- Y = R^H (n x r) to global memory and to LDS (odd leading dimension:
-  // the tile loads of the Gram matrix step over columns), G from it on the
-  // matrix cores, then G over Y in LDS ----
-  const int ldy = n | 1;
-  double2* Ys = lds_small;
+  // ---- Y = R^H (n x r) to global memory; G from it on the matrix cores, by
+  // way of LDS where Y fits it (odd leading dimension: the tile loads step
+  // over columns), else from global memory; G replaces Y in LDS ----
   for (long e = tid; e < (long)n * r; e += NT) {
     const int sidx = e % n, t = e / n;
-    const int ps = q_piv[sidx];
     double2 v = make_double2(0.0, 0.0);
-    if (t < sidx) v = cconj(a.A[t + (long)ps * m]);   // As is being overwritten
+    if (t < sidx) v = cconj(a.A[t + (long)s_piv[sidx] * m]);
     else if (t == sidx) v = make_double2(a.beta[sidx], 0.0);
     a.Y[e] = v;
   }
   __syncthreads();
-  for (long e = tid; e < (long)n * r; e += NT) Ys[e % n + (e / n) * ldy] = a.Y[e];
-  __syncthreads();
+  if (tid == 0 && a.folded) *a.folded = folded2;
+  if (r > kGramSmallRank) {
+    // gram_svd_kernel goes on from Y
+    if (tid == 0) {
+      a.info->sweeps = 0;
+      a.info->pad = r;
+    }
+    return;
+  }
   double2* Gm = lds_small;
-  double2* rs = Gm + gram_entries(r);
-  double* rc = reinterpret_cast<double*>(rs + 64);
-  double* s_sig = rc + 64;
-  {
-    constexpr int kTiles = (21 + NT / 64 - 1) / (NT / 64);   // of 21 at 96 columns
-    const int nb = (r + 15) / 16, tiles = nb * (nb + 1) / 2;
+  const int nb = (r + 15) / 16, tiles = nb * (nb + 1) / 2;
+  const int ldy = n | 1;
+  if ((long)ldy * r * (long)sizeof(double2) <= a.lds_bytes) {
+    double2* Ys = lds_small;
+    for (long e = tid; e < (long)n * r; e += NT) Ys[e % n + (e / n) * ldy] = a.Y[e];
+    __syncthreads();
+    constexpr int kTiles = 3;                 // of the 21 at rank 88, 8 wavefronts
     double2 g[kTiles][4];
 #pragma unroll
     for (int u = 0; u < kTiles; ++u)
@@ -2690,36 +2784,31 @@ __device__ void small_svd_body(const SmallSvdArgs& a) {
 #pragma unroll
     for (int u = 0; u < kTiles; ++u)
       if (wave + u * (NT / 64) < tiles) gram_store(Gm, r, wave + u * (NT / 64), g[u]);
+  } else {
+    for (int e = tid; e < gram_entries(r); e += NT) Gm[e] = make_double2(0.0, 0.0);
+    __syncthreads();
+    for (int t = wave; t < tiles; t += NT / 64) {
+      double2 g[4];
+      gram_tile(a.Y, n, n, r, t, g);
+      gram_store(Gm, r, t, g);
+    }
   }
   __syncthreads();
-  int half;
-  const double tr = gram_scale<NT>(Gm, r, &half);
-  const double tol = (n > 16 ? n : 16) * eps;
-  bool converged = false;
-  constexpr int kBlocks = (1176 + NT - 1) / NT;              // of 1176 at 96 columns
-  const int sweeps = gram_jacobi<NT, kBlocks>(Gm, r, tol * tol, eps * eps * tr, a.max_sweeps,
-                                              rc, rs, a.logc, a.logs, converged);
+  // one block per thread up to rank 62 (496 blocks), two at 88 (990)
+  if (r <= 62) gram_run<NT, 1>(a, Gm, n, r, folded2);
+  else gram_run<NT, 2>(a, Gm, n, r, folded2);
   PHASE(14);
-  if (tid == 0) {
-    s_folded = folded2;
-    if (a.folded) *a.folded = folded2;
-  }
-  __syncthreads();
-  gram_finish<NT>(Gm, r, a.epsrel, a.max_rank, s_folded, sweeps,
-                  sweeps * (max(2, r + (r & 1)) - 1), converged, half, s_sig, s_sig + r,
-                  s_sig + 2 * r, a.sigma, a.perm, a.sorted, a.info, a.copy);
-  PHASE(15);
 }
 
 __global__ void __launch_bounds__(kSmallThreads)
 small_svd_kernel(SmallSvdArgs a) {
-  small_svd_body<kSmallThreads>(a);
+  small_svd_body(a);
 }
 
-__global__ void __launch_bounds__(kSmallBatchThreads)
+__global__ void __launch_bounds__(kSmallThreads)
 small_svd_batch_kernel(const SmallSvdArgs* probs) {
   const SmallSvdArgs a = probs[blockIdx.x];
-  small_svd_body<kSmallBatchThreads>(a);
+  small_svd_body(a);
 }
 
 // Left singular vectors Q W[:, perm[j]] (j < k) of the pivoted QR, the

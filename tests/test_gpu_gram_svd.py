@@ -67,3 +67,16 @@ def test_scale_limits(n, scale):
     s = 10.0 ** (-8.0 * np.arange(n) / (n - 1))
     mat = (_unitary(rng, n, n) * s) @ _unitary(rng, n, n).conj().T
     _check(mat * scale, f"scale {scale:g}")
+
+
+@pytest.mark.parametrize("m,n", [
+    (1, 9), (64, 1), (1280, 1), (1281, 2), (1024, 16), (640, 17), (641, 17),
+    (320, 33), (321, 40), (160, 65), (161, 66), (128, 126), (160, 126),
+    (257, 64), (129, 80), (31, 126), (5, 120)])
+def test_register_qr_edges(m, n):
+    """Rows per lane of the one-workgroup QR at the limits of its variants
+    (4, 8, 12, 16 and 20) for 8 to 64 lanes a column, and just beyond."""
+    rng = np.random.default_rng([m, n, 1])
+    r = min(m, n)
+    s = 10.0 ** (-8.0 * np.arange(r) / max(r - 1, 1))
+    _check((_unitary(rng, m, r) * s) @ _unitary(rng, n, r).conj().T, "qr")
