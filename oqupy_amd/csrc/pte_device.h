@@ -132,6 +132,16 @@ __device__ __forceinline__ double group_sum1(double a, int G) {
   return a;
 }
 
+// Largest / smallest value of a wavefront, in every lane.
+__device__ __forceinline__ unsigned wave_max(unsigned v) {
+  v = max(v, (unsigned)dpp_i<kDppXor1>((int)v));
+  v = max(v, (unsigned)dpp_i<kDppXor2>((int)v));
+  v = max(v, (unsigned)dpp_i<kDppHalfMirror>((int)v));
+  v = max(v, (unsigned)dpp_i<kDppMirror>((int)v));
+  return swap_max<32>(swap_max<16>(v));
+}
+__device__ __forceinline__ unsigned wave_min(unsigned v) { return ~wave_max(~v); }
+
 // Sum over one 64-lane wavefront; every lane gets the same bits.
 __device__ __forceinline__ double wave_sum(double v) { return group_sum1(v, 64); }
 
@@ -186,6 +196,13 @@ __device__ __forceinline__ unsigned ld_agent(const unsigned* p) {
                            __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void st_agent(unsigned* p, unsigned v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long ld_agent(const unsigned long long* p) {
+  return __hip_atomic_load(const_cast<unsigned long long*>(p), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent(unsigned long long* p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ double2 ld_agent(const double2* p) {

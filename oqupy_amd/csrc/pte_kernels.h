@@ -73,12 +73,10 @@ struct EmitArgs {
   double2* dst;
 };
 
-// Pivoted QR of a column-major matrix (see qrcp_kernel).
+// Pivoted QR of a column-major matrix (see qrcp_kernel): a workgroup's post of
+// one step (see qrcp_post).
 struct QrcpCand {
-  double vmax;   // largest residual column norm of a workgroup
-  double vsum;   // sum of squared residual norms of a workgroup
-  int col;       // column of vmax (-1: none)
-  int pad;
+  unsigned long long w0, w1;
 };
 
 struct QrcpArgs {
@@ -87,9 +85,8 @@ struct QrcpArgs {
   double2* tau; double2* vscale; double* beta;
   int* piv;                   // [n] physical column of each step, then the rest
   int* done;                  // [n] scratch
-  QrcpCand* cand;             // [2 * gridDim.x] scratch
+  QrcpCand* cand;             // [2 * gridDim.x] posts, zeroed before the launch
   int* rank;                  // steps taken
-  unsigned* bar;
   const int* max_steps;       // optional cap on the steps (device int)
   double* out;                // optional: [0] squared residual norm at the stop,
                               // [1] ||A||_F^2 (first run), [2] |beta_0|, [3] the

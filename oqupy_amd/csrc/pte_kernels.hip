@@ -1470,52 +1470,39 @@ emit_kernel(EmitArgs a) {
 // the Frobenius norm of the unfactored block is at most drop * ||A||_F; the
 // rows below r of R are dropped (a perturbation of that size).
 // Column c belongs to workgroup c % gridDim.x; every workgroup forms the
-// step's reflector from the pivot column itself, so one grid barrier per
-// step suffices: candidates (largest residual norm per workgroup) are posted
-// before it and reduced identically by every workgroup after it.
+// step's reflector from the pivot column itself, so workgroups wait for each
+// other once per step: each posts its candidate (largest residual norm) and
+// every one waits for all posts of the step and reduces them identically.
+// A post is two 8-byte words that each carry the step's tag, so reading the
+// posts is the waiting: no arrival counter stands between them (two dependent
+// atomics and a separate read of the candidates less). A step at 380 x 108 takes
+// 7.0 us on 27 workgroups (8.8 with the counters; 1.5 forming the reflector, 1.3
+// updating the columns, 2.3 until their stores are acknowledged, 1.7 waiting for
+// the posts), at 996 x 860 8.8 us on 215 (10.1). The posts are double-buffered by step parity: a workgroup
+// posts step j + 2 after reading all posts of step j + 1, which were made after
+// their workgroups had read step j's. They are zeroed before the launch (no
+// step has tag 0).
 // ---------------------------------------------------------------------------
 // (value, column) maximum with ties to the smaller column; -1 = none
 __device__ __forceinline__ void better(double& v, int& c, double ov, int oc) {
   if (oc >= 0 && (c < 0 || ov > v || (ov == v && oc < c))) { v = ov; c = oc; }
 }
 
-// global winner and residual total among the posted candidates; every
-// thread of the workgroup gets identical results
-__device__ void qrcp_reduce(const QrcpCand* cand, int nblk, double (*slot)[4],
-                            double (*slotv)[4], int (*slotc)[4], int& parity,
-                            int* bestc, double* total) {
-  double bv = -1.0, sv = 0.0;
-  int bc = -1;
-  for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-    sv += ld_agent(&cand[b].vsum);
-    better(bv, bc, ld_agent(&cand[b].vmax), ld_agent(&cand[b].col));
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const double ov = __shfl_xor(bv, off, 64);
-    const int oc = __shfl_xor(bc, off, 64);
-    better(bv, bc, ov, oc);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    slotv[parity][threadIdx.x >> 6] = bv;
-    slotc[parity][threadIdx.x >> 6] = bc;
-  }
-  // block_sum256 synchronises before reading, which also publishes the slots
-  *total = block_sum256(sv, slot, parity);
-  double v = -1.0;
-  int c = -1;
-  const int par = parity ^ 1;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) better(v, c, slotv[par][w], slotc[par][w]);
-  *bestc = c;
+constexpr unsigned long long kQrTagMask = 0xfffull;
+__device__ __forceinline__ unsigned long long qrcp_tag(int j) {
+  return (unsigned long long)(1 + j % 4095);
 }
 
-// wavefront-level column work of qrcp_kernel: the four wavefronts of a
-// workgroup take its columns in turn
-__device__ __forceinline__ void qrcp_post(QrcpCand* dst, double wmax, int wcol, double wsum,
-                                          double* cw_max, int* cw_col, double* cw_sum) {
+// Posts the workgroup's candidate of step j: word 0 holds the upper word of the
+// largest residual norm, its column (20 bits; all ones: none) and the tag, word
+// 1 the sum of the squared residual norms with the tag in its lowest 12 bits.
+// Every wavefront waits for its own column stores first.
+__device__ __forceinline__ void qrcp_post(QrcpCand* dst, int j, double wmax, int wcol,
+                                          double wsum, double* cw_max, int* cw_col,
+                                          double* cw_sum) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (lane == 0) { cw_max[wave] = wmax; cw_col[wave] = wcol; cw_sum[wave] = wsum; }
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (threadIdx.x == 0) {
     double v = -1.0, sm = 0.0;
@@ -1524,10 +1511,56 @@ __device__ __forceinline__ void qrcp_post(QrcpCand* dst, double wmax, int wcol, 
       sm += cw_sum[w];
       better(v, c, cw_max[w], cw_col[w]);
     }
-    st_agent(&dst->vmax, v);
-    st_agent(&dst->vsum, sm);
-    st_agent(&dst->col, c);
+    const unsigned long long tag = qrcp_tag(j);
+    const unsigned long long key = c >= 0 ? (unsigned)__double2hiint(v) : 0u;
+    const unsigned long long col = c >= 0 ? (unsigned)c : 0xfffffu;
+    st_agent(&dst->w1, ((unsigned long long)__double_as_longlong(sm) & ~kQrTagMask) | tag);
+    st_agent(&dst->w0, (key << 32) | (col << 12) | tag);
   }
+}
+
+// Waits for the posts of step j and reduces them: the column of the largest
+// norm (by the upper word, ties to the smaller column; -1: none) and the
+// residual total, the same bits in every thread of the grid.
+__device__ __forceinline__ void qrcp_reduce(const QrcpCand* cand, int nblk, int j,
+                                            double (*slot)[4], unsigned (*slotk)[4],
+                                            unsigned (*slotc)[4], int& parity, int* bestc,
+                                            double* total) {
+  const unsigned long long tag = qrcp_tag(j);
+  double sv = 0.0;
+  unsigned key = 0, col = 0xfffffu;
+  if ((int)threadIdx.x < nblk) {
+    // both words in one 16-byte load (each has its own tag)
+    const __amdgpu_buffer_rsrc_t rs = agent_rsrc(cand, (unsigned)nblk * 16u);
+    unsigned long long w0, w1;
+    for (;;) {
+      const double2 v = ld_agent16(rs, threadIdx.x * 16u);
+      w0 = (unsigned long long)__double_as_longlong(v.x);
+      w1 = (unsigned long long)__double_as_longlong(v.y);
+      if ((w0 & kQrTagMask) == tag && (w1 & kQrTagMask) == tag) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    key = (unsigned)(w0 >> 32);
+    col = (unsigned)(w0 >> 12) & 0xfffffu;
+    sv = __longlong_as_double((long long)(w1 & ~kQrTagMask));
+  }
+  // a workgroup without columns left has key 0 and the largest column number
+  const unsigned wkey = wave_max(key);
+  const unsigned wcol = wave_min(key == wkey ? col : 0xfffffu);
+  if ((threadIdx.x & 63) == 0) {
+    slotk[parity][threadIdx.x >> 6] = wkey;
+    slotc[parity][threadIdx.x >> 6] = wcol;
+  }
+  // block_sum256 synchronises before reading, which also publishes the slots
+  *total = block_sum256(sv, slot, parity);
+  const int par = parity ^ 1;
+  unsigned k = slotk[par][0], c = slotc[par][0];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) {
+    const unsigned ok = slotk[par][w], oc = slotc[par][w];
+    if (ok > k || (ok == k && oc < c)) { k = ok; c = oc; }
+  }
+  *bestc = __builtin_amdgcn_readfirstlane(c == 0xfffffu ? -1 : (int)c);
 }
 
 // loads of the pivoted QR issued together (per thread), and the rows of a
@@ -1538,8 +1571,8 @@ constexpr int kQrCache = 16;
 
 __device__ __forceinline__ void qrcp_body(const QrcpArgs& a, const int blk, const int nblk) {
   extern __shared__ double2 vcol[];            // reflector of the step (m)
-  __shared__ double slot[2][4], slotv[2][4];
-  __shared__ int slotc[2][4];
+  __shared__ double slot[2][4];
+  __shared__ unsigned slotk[2][4], slotc[2][4];
   __shared__ double vn1[kQrcpMaxLocal], vn2[kQrcpMaxLocal];
   __shared__ int done[kQrcpMaxLocal];
   __shared__ double cw_max[4], cw_sum[4];
@@ -1551,7 +1584,6 @@ __device__ __forceinline__ void qrcp_body(const QrcpArgs& a, const int blk, cons
   const long lda = a.lda;
   const int kmax = m < n ? m : n;
   const int nloc = (n - blk + nblk - 1) / nblk;   // own columns blk, blk+nblk, ...
-  unsigned epoch = 0;
 
   // initial column norms (one wavefront per column); when resuming, the
   // norms of the unfactored rows start..m-1 of the columns not yet pivoted
@@ -1604,15 +1636,15 @@ __device__ __forceinline__ void qrcp_body(const QrcpArgs& a, const int blk, cons
     wsum += nrm * nrm;
     better(wmax, wcol, nrm, c);
   }
-  qrcp_post(a.cand + blk, wmax, wcol, wsum, cw_max, cw_col, cw_sum);
-  grid_barrier_all(a.bar, nblk, blk, epoch);
+  qrcp_post(a.cand + (j0 & 1) * nblk + blk, j0, wmax, wcol, wsum, cw_max, cw_col, cw_sum);
   double total;
   int p;
-  qrcp_reduce(a.cand, nblk, slot, slotv, slotc, parity, &p, &total);
+  qrcp_reduce(a.cand + (j0 & 1) * nblk, nblk, j0, slot, slotk, slotc, parity, &p, &total);
   const double total0 = total;
   const double drop2 = j0 > 0 ? a.drop_abs2 : a.drop * a.drop * total;
   const double tol3z = 1.4901161193847656e-08;   // sqrt(eps), zlaqp2
-  const int jmax = a.max_steps ? min(kmax, max(1, *a.max_steps)) : kmax;
+  const int jmax =
+      __builtin_amdgcn_readfirstlane(a.max_steps ? min(kmax, max(1, *a.max_steps)) : kmax);
   int j = j0;
   // mark: the first step count with residual^2 <= (mark_rel |beta_0|)^2;
   // every workgroup reduces the same candidates in the same order, so the
@@ -1624,7 +1656,10 @@ __device__ __forceinline__ void qrcp_body(const QrcpArgs& a, const int blk, cons
     mark2 = b0 * b0;
   }
   PHASE_INIT();
-  while (j < jmax && p >= 0 && total > drop2) {
+  // p, the step and the exit are the same in every lane, and scalar for the
+  // compiler by the readfirstlanes (else the buffer descriptors of the columns
+  // would be assembled lane by lane)
+  while (j < jmax && p >= 0 && __builtin_amdgcn_readfirstlane((int)(total > drop2))) {
     // reflector j from the pivot column p (rows j..m-1), whole workgroup: the
     // column is read once into vcol (loads issued in batches, so that their
     // latencies overlap), then scaled in LDS
@@ -1872,21 +1907,17 @@ __device__ __forceinline__ void qrcp_body(const QrcpArgs& a, const int blk, cons
       better(wmax, wcol, nv, c);
     }
     PHASE(9);
-    qrcp_post(a.cand + ((j + 1) & 1) * nblk + blk, wmax, wcol, wsum, cw_max, cw_col,
-              cw_sum);
-    PHASE(10);
-    grid_barrier_all(a.bar, nblk, blk, epoch);
-    PHASE(11);
-    qrcp_reduce(a.cand + ((j + 1) & 1) * nblk, nblk, slot, slotv, slotc, parity, &p,
-                &total);
-    PHASE(12);
     ++j;
+    qrcp_post(a.cand + (j & 1) * nblk + blk, j, wmax, wcol, wsum, cw_max, cw_col, cw_sum);
+    PHASE(10);
+    qrcp_reduce(a.cand + (j & 1) * nblk, nblk, j, slot, slotk, slotc, parity, &p, &total);
+    PHASE(12);
     if (a.mark_rel > 0.0) {
       if (j == 1) {
         const double b0 = a.mark_rel * fabs(beta);
         mark2 = b0 * b0;
       }
-      if (mark < 0 && total <= mark2) {
+      if (mark < 0 && __builtin_amdgcn_readfirstlane((int)(total <= mark2))) {
         mark = j;
         if (a.stop_at_mark) break;
       }
