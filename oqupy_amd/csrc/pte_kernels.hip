@@ -473,11 +473,6 @@ __device__ __forceinline__ void tournament_pair(int nplayers, int round, int slo
   }
 }
 
-__device__ __forceinline__ void ordered_pair(int sub, int slot, int& p, int& q) {
-  tournament_pair(JP, sub, slot, p, q);
-  if (p > q) { const int t = p; p = q; q = t; }
-}
-
 // Does the Hermitian 2x2 block [[app, apq], [conj(apq), aqq]] need a rotation:
 // |apq| > tol * sqrt(|app aqq|) and |apq| > abs_tol * sqrt(max(app, aqq)),
 // compared in squares.
@@ -500,149 +495,298 @@ __device__ __forceinline__ double rcp_nr(double x) {
   return fma(fma(e, e, e), y, y);
 }
 
-// Rotation of that block: J = [[cs, sn], [-sn conj(ph), cs conj(ph)]],
-// ph = apq / |apq|, chosen so that J^H [[app, apq], [conj(apq), aqq]] J is
-// diagonal (Rutishauser's formulas). r = {cs, sn, Re ph, Im ph}.
-__device__ __forceinline__ bool jacobi_rotation(double app, double aqq, double2 apq,
-                                                double tol2, double abs_tol2, double* r) {
+// Rotation of the 2 x 2 block [[app, apq], [conj(apq), aqq]]: with
+// d = aqq - app and h = sqrt(d^2 + 4 |apq|^2), c = cos(theta) =
+// sqrt((h + |d|) / 2h) and s = sign(d) apq / (h c) (theta = pi/4 for d = 0); no
+// sum in it cancels, and the phase of apq stays in s, so its modulus is not
+// needed. The identity where no rotation is needed. The Gram matrices are
+// scaled to a trace near one, so the squares stay in range.
+// Returns whether one is; the rotated diagonal is app - shift, aqq + shift.
+__device__ __forceinline__ bool gram_rotation(bool valid, double app, double aqq, double2 apq,
+                                              double tol2, double abs_tol2, double& c,
+                                              double2& s, double& shift) {
   const double mag2 = cabs2(apq);
-  r[0] = 1.0; r[1] = 0.0; r[2] = 1.0; r[3] = 0.0;
-  if (!needs_rotation(app, aqq, mag2, tol2, abs_tol2)) return false;
-  const double inv = rsqrt_nr(mag2);
-  const double zeta = (aqq - app) * 0.5 * inv;
-  double t;
-  if (zeta == 0.0) {
-    t = 1.0;
-  } else if (fabs(zeta) > 1e150) {
-    t = copysign(0.5, zeta) * rcp_nr(fabs(zeta));
-  } else {
-    const double q = fma(zeta, zeta, 1.0);
-    const double root = q * rsqrt_nr(q);             // sqrt(1 + zeta^2)
-    t = copysign(1.0, zeta) * rcp_nr(fabs(zeta) + root);
-  }
-  const double cs = rsqrt_nr(fma(t, t, 1.0));
-  r[0] = cs; r[1] = cs * t; r[2] = apq.x * inv; r[3] = apq.y * inv;
-  return true;
-}
-
-// The same rotation with two dependent square-root chains instead of four:
-// with d = aqq - app and h = sqrt(d^2 + 4|apq|^2), cos(theta) =
-// sqrt((h + |d|) / (2h)) and sin(theta) = sign(d) |apq| / (h cos(theta))
-// (theta = pi/4 for d = 0); no sum in it cancels. The phase apq / |apq| is an
-// independent chain. The 2x2 block is first scaled by a power of two that
-// brings max(app, aqq) into [1, 2) (the rotation is scale-invariant and
-// |apq|^2 <= app aqq keeps every square finite), and everything is evaluated
-// without branches (a pair that needs no rotation runs the formula on
-// harmless operands and keeps the identity). r is the same
-// {cs, sn, Re ph, Im ph} as jacobi_rotation's up to rounding.
-__device__ __forceinline__ bool jacobi_rotation_fast(bool valid, double app, double aqq,
-                                                     double2 apq, double tol2, double abs_tol2,
-                                                     double* r) {
-  const double mag2 = cabs2(apq);
-  // needs_rotation, without short-circuit branches
-  const bool need = valid & (mag2 > tol2 * fabs(app * aqq)) &
-                    (mag2 > abs_tol2 * fmax(fmax(app, aqq), 0.0)) & (mag2 > 0.0);
-  const double sc = need ? ldexp(1.0, -ilogb(fmax(fmax(app, aqq), 1e-300))) : 0.0;
-  const double2 c = make_double2(apq.x * sc, apq.y * sc);
-  const double m2 = need ? cabs2(c) : 1.0;
-  const double d = (aqq - app) * sc;
-  const double h2 = fma(d, d, 4.0 * m2);
-  const double inv = rsqrt_nr(m2), rh = rsqrt_nr(h2);   // 1 / |apq|, 1 / h
-  const double cos2 = fma(0.5 * fabs(d), rh, 0.5);      // cos^2(theta)
-  const double rc = rsqrt_nr(cos2);                     // 1 / cos(theta)
-  const double sn = copysign(m2 * inv * rh * rc, d < 0.0 ? -1.0 : 1.0);
-  r[0] = need ? cos2 * rc : 1.0;
-  r[1] = need ? sn : 0.0;
-  r[2] = need ? c.x * inv : 1.0;
-  r[3] = need ? c.y * inv : 0.0;
+  const bool need = valid & (mag2 > tol2 * fabs(app * aqq)) & (mag2 > abs_tol2 * app) &
+                    (mag2 > abs_tol2 * aqq) & (mag2 > 0.0);
+  const double d = aqq - app;
+  const double h2 = need ? fma(d, d, 4.0 * mag2) : 1.0;
+  const double rh = rsqrt_nr(h2);
+  const double cos2 = fma(0.5 * fabs(d), rh, 0.5);
+  const double rc = rsqrt_nr(cos2);
+  const double f = copysign(rh * rc, d < 0.0 ? -1.0 : 1.0);
+  c = need ? cos2 * rc : 1.0;
+  s = make_double2(need ? apq.x * f : 0.0, need ? apq.y * f : 0.0);
+  shift = need ? f * rc * mag2 : 0.0;
   return need;
 }
-
-// Valid columns of the block pair (bi, bj) as a 32-bit mask (the last block
-// may be partial).
-__device__ __forceinline__ unsigned pair_valid_mask(int bi, int bj, int n) {
-  const unsigned mi = bi * JB + JB <= n ? 0xffffu : (bi * JB < n ? (1u << (n - bi * JB)) - 1u : 0u);
-  const unsigned mj = bj * JB + JB <= n ? 0xffffu : (bj * JB < n ? (1u << (n - bj * JB)) - 1u : 0u);
-  return mi | (mj << JB);
+__device__ __forceinline__ bool gram_rotation(bool valid, double app, double aqq, double2 apq,
+                                              double tol2, double abs_tol2, double& c,
+                                              double2& s) {
+  double shift;
+  return gram_rotation(valid, app, aqq, apq, tol2, abs_tol2, c, s, shift);
 }
 
-// Cyclic two-sided Jacobi sweeps on the pair's 2JB x 2JB Gram Gs[0],
-// accumulating the rotations in Ws (identity on entry). Gs is
-// double-buffered: a sub-step reads Gs[cur] and writes every entry of
-// Gs[cur ^ 1], so one barrier per sub-step suffices. Each thread owns the
-// 2x2 block (P1, P2) of the sub-step's pairing (ptab); each lane computes the
-// rotation of pair P2 = lane & 15 and takes the one of pair P1 from lane P1
-// of its wavefront; it also rotates rows P1 and P1+16 of Ws for pair P2.
-__device__ __forceinline__ void pair_inner_sweeps(double2 (*Gs)[JP][JP + 2],
-                                                  double2 (*Ws)[JP + 2],
-                                                  const int (*ptab)[JB], unsigned vmask,
-                                                  double tol2, double abs_tol2,
-                                                  int inner_sweeps) {
-  const int tid = threadIdx.x;
-  const int P1 = tid >> 4, P2 = tid & 15;
-  int cur = 0;
-  for (int isw = 0; isw < inner_sweeps; ++isw) {
-    int any = 0;
-    for (int sub = 0; sub < JP - 1; ++sub) {
-      const int e1 = ptab[sub][P1], e2 = ptab[sub][P2];
-      const int p1 = e1 & 255, q1 = e1 >> 8, p2 = e2 & 255, q2 = e2 >> 8;
-      // every LDS operand of the sub-step is read at once
-      const double2 g22 = Gs[cur][p2][q2];
-      const double d2p = Gs[cur][p2][p2].x, d2q = Gs[cur][q2][q2].x;
-      double2 b00 = Gs[cur][p1][p2], b01 = Gs[cur][p1][q2];
-      double2 b10 = Gs[cur][q1][p2], b11 = Gs[cur][q1][q2];
-      double2 w0p = Ws[P1][p2], w0q = Ws[P1][q2];
-      double2 w1p = Ws[P1 + 16][p2], w1q = Ws[P1 + 16][q2];
-      // keep every read above issued before the rotation's arithmetic
-      __builtin_amdgcn_sched_barrier(0);
-      double r1[4], r2[4];
-      const bool on2 = jacobi_rotation_fast(((vmask >> p2) & (vmask >> q2) & 1u) != 0u, d2p,
-                                            d2q, g22, tol2, abs_tol2, r2);
+// Places of a Hermitian matrix kept by round-robin position (gram_jacobi and
+// the pair sweeps below): position 2q holds the first column a_q of pair q,
+// position 2q + 1 its second, b_q; position 0 keeps its column and the others
+// move on by one position a round (gram_next), so that after 2P - 1 rounds (P
+// pairs) every two columns have met and all are back. The matrix is stored as
+// the P (P + 1) / 2 blocks (q1, q2), q1 <= q2, of 2 x 2 entries, entry e of every
+// block in a plane of its own.
+__device__ __forceinline__ int gram_block(int q1, int q2) { return q2 * (q2 + 1) / 2 + q1; }
+
+// position of column c in round 0 (P pairs) and a position's next one
+__device__ __forceinline__ int gram_pos(int c, int P) {
+  const int L = 2 * P - 1;
+  return c == L ? 0 : c == 0 ? 1 : c < P ? 2 * c : 2 * (L - c) + 1;
+}
+__device__ __forceinline__ int gram_next(int x, int P) {
+  if (x == 0 || P == 1) return x;
+  if (x == 2) return 1;
+  if ((x & 1) == 0) return x - 2;
+  return x == 2 * P - 1 ? x - 1 : x + 2;
+}
+
+// where the entry of positions (x, y) is kept (T: entries of a plane), and
+// whether conjugated
+__device__ __forceinline__ int gram_place(int x, int y, int T, bool& conj) {
+  const int qx = x >> 1, qy = y >> 1;
+  conj = qx > qy || (qx == qy && x > y);
+  if (conj) return (2 * (y & 1) + (x & 1)) * T + gram_block(qy, qx);
+  return (2 * (x & 1) + (y & 1)) * T + gram_block(qx, qy);
+}
+
+// ---- cyclic two-sided Jacobi sweeps on a block pair's 2JB x 2JB Gram matrix,
+// by 256 threads ----
+// The matrix is kept by position (PT blocks, four planes) in two buffers: a
+// round reads one and writes the other with the entries where their columns are
+// in the next round. What a round takes is the chain from one round's rotations
+// to the next's, so wavefront 0 does nothing else: lane q has pair q's diagonal
+// in registers, transforms the one entry of another block that will be its
+// next pair's off-diagonal one, and computes the next rotation while wavefronts
+// 1 and 2 rotate the 120 off-diagonal blocks from both sides (a thread each) and
+// 1 to 3 accumulate the rotations in W, whose rows are in registers: lane q (mod
+// 16) of a row of lanes has the entries of columns a_q and b_q, which move on by
+// one lane a round. One barrier a round (11 cycles with four wavefronts).
+// A round takes 0.39 us; 0.75 us with every wavefront computing the rotations
+// from a column-indexed matrix and W in LDS, and 0.65 us with the matrix by
+// position but the rotations and the updates one after the other.
+constexpr int PP = JB;                      // pairs of a block pair's columns
+constexpr int PT = PP * (PP + 1) / 2;       // blocks of its Gram matrix
+constexpr int kPairOwners = PT - PP;        // off-diagonal ones, a thread each
+static_assert(PP == 16 && kPairOwners <= 128, "a DPP row of pairs; owners in wavefronts 1 and 2");
+constexpr int kDppRowShl1 = 0x101, kDppRowShr1 = 0x111;
+
+// A thread's constants: its block (wavefront 0: pair lane % 16's diagonal one),
+// the places of the entries in the next round (as in gram_jacobi) and the places
+// at which it stores the Gram matrix.
+struct PairThread {
+  int q1, q2;
+  unsigned dst[2];
+  int store[4];       // -1: not stored (lower triangle); bit 30: conjugated
+};
+
+__device__ __forceinline__ PairThread pair_thread(int slices) {
+  PairThread t;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int b = min(max(tid - 64, 0), kPairOwners - 1);
+  int c = 1;
+  while (c * (c + 1) / 2 <= b) ++c;
+  t.q2 = wave == 0 ? lane & 15 : c;
+  t.q1 = wave == 0 ? lane & 15 : b - c * (c - 1) / 2;
+  t.dst[0] = t.dst[1] = 0;
 #pragma unroll
-      for (int h = 0; h < 4; ++h) r1[h] = __shfl(r2[h], P1, 64);
-      any |= on2;
-      // applied without branches: a pair that needs no rotation has the
-      // identity (cs 1, sn 0, ph 1), which leaves its entries exactly as
-      // they are
-      {
-        const double c = r2[0], sn = r2[1];
-        const double2 cph = make_double2(r2[2], -r2[3]);
-        const double2 x01 = cmul(b01, cph), x11 = cmul(b11, cph);
-        const double2 n00 = make_double2(c * b00.x - sn * x01.x, c * b00.y - sn * x01.y);
-        const double2 n01 = make_double2(sn * b00.x + c * x01.x, sn * b00.y + c * x01.y);
-        const double2 n10 = make_double2(c * b10.x - sn * x11.x, c * b10.y - sn * x11.y);
-        const double2 n11 = make_double2(sn * b10.x + c * x11.x, sn * b10.y + c * x11.y);
-        b00 = n00; b01 = n01; b10 = n10; b11 = n11;
-        const double2 y0 = cmul(w0q, cph), y1 = cmul(w1q, cph);
-        Ws[P1][p2] = make_double2(c * w0p.x - sn * y0.x, c * w0p.y - sn * y0.y);
-        Ws[P1][q2] = make_double2(sn * w0p.x + c * y0.x, sn * w0p.y + c * y0.y);
-        Ws[P1 + 16][p2] = make_double2(c * w1p.x - sn * y1.x, c * w1p.y - sn * y1.y);
-        Ws[P1 + 16][q2] = make_double2(sn * w1p.x + c * y1.x, sn * w1p.y + c * y1.y);
-      }
-      {
-        const double c = r1[0], sn = r1[1];
-        const double2 ph = make_double2(r1[2], r1[3]);
-        const double2 y10 = cmul(ph, b10), y11 = cmul(ph, b11);
-        const double2 n00 = make_double2(c * b00.x - sn * y10.x, c * b00.y - sn * y10.y);
-        const double2 n01 = make_double2(c * b01.x - sn * y11.x, c * b01.y - sn * y11.y);
-        const double2 n10 = make_double2(sn * b00.x + c * y10.x, sn * b00.y + c * y10.y);
-        const double2 n11 = make_double2(sn * b01.x + c * y11.x, sn * b01.y + c * y11.y);
-        b00 = n00; b01 = n01; b10 = n10; b11 = n11;
-      }
-      if (P1 == P2 && on2) {
-        b01 = make_double2(0.0, 0.0);
-        b10 = make_double2(0.0, 0.0);
-        b00.y = 0.0;
-        b11.y = 0.0;
-      }
-      const int nxt = cur ^ 1;
-      Gs[nxt][p1][p2] = b00; Gs[nxt][p1][q2] = b01;
-      Gs[nxt][q1][p2] = b10; Gs[nxt][q1][q2] = b11;
-      __syncthreads();
-      cur = nxt;
-    }
-    if (!__syncthreads_or(any)) break;
+  for (int e = 0; e < 4; ++e) {
+    bool conj = false;
+    const int at = gram_place(gram_next(2 * t.q1 + (e >> 1), PP),
+                              gram_next(2 * t.q2 + (e & 1), PP), PT, conj);
+    t.dst[e >> 1] |= ((unsigned)at | (conj ? 0x8000u : 0u)) << (16 * (e & 1));
+    // entries of a thread: the MFMA tile of its wavefront (one slice), or
+    // entry tid + 256 e of the summed partial Grams
+    const int i = slices == 1 ? 16 * (wave >> 1) + 4 * e + (lane >> 4) : (tid + JT * e) / JP;
+    const int j = slices == 1 ? 16 * (wave & 1) + (lane & 15) : (tid + JT * e) % JP;
+    bool cs = false;
+    const int place = gram_place(gram_pos(i, PP), gram_pos(j, PP), PT, cs);
+    t.store[e] = i > j ? -1 : place | (cs ? 1 << 30 : 0) | (i == j ? 1 << 29 : 0);
   }
+  return t;
+}
+
+// entry e of a thread's Gram entries (scaled by sc)
+__device__ __forceinline__ void pair_store(double2* Gp, const PairThread& t, int e, double2 v,
+                                           double sc) {
+  const int s = t.store[e];
+  if (s < 0) return;
+  const double y = (s & (1 << 29)) ? 0.0 : ((s & (1 << 30)) ? -v.y : v.y);
+  Gp[s & 0xffff] = make_double2(v.x * sc, y * sc);
+}
+
+// does some pair of the block pair need a rotation (the workgroup's answer)
+__device__ __forceinline__ bool pair_needs(const double2* Gp, const PairThread& t, double tol2,
+                                           double abs_tol2) {
+  const int b = gram_block(t.q1, t.q2);
+  const int b1 = gram_block(t.q1, t.q1), b2 = gram_block(t.q2, t.q2);
+  const double da1 = Gp[b1].x, db1 = Gp[3 * PT + b1].x;
+  const double da2 = Gp[b2].x, db2 = Gp[3 * PT + b2].x;
+  bool any = needs_rotation(da1, db2, cabs2(Gp[PT + b]), tol2, abs_tol2);
+  if (threadIdx.x >= 64) {
+    any |= needs_rotation(da1, da2, cabs2(Gp[b]), tol2, abs_tol2);
+    any |= needs_rotation(db1, da2, cabs2(Gp[2 * PT + b]), tol2, abs_tol2);
+    any |= needs_rotation(db1, db2, cabs2(Gp[3 * PT + b]), tol2, abs_tol2);
+  }
+  return __builtin_amdgcn_readfirstlane(__syncthreads_or((int)any)) != 0;
+}
+
+// lane move; a lane without a source keeps `old`
+template <int CTRL>
+__device__ __forceinline__ double dpp_keep_d(double old, double v) {
+  return __hiloint2double(
+      __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, 0xf, 0xf, false),
+      __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double2 dpp_row2(double2 v) {
+  return make_double2(dpp_d<CTRL>(v.x), dpp_d<CTRL>(v.y));
+}
+
+// The sweeps; W (row-major, by column) goes to Ws, whose memory is the second
+// buffer until then. rc and rs have two buffers of PP entries.
+__device__ __forceinline__ void pair_sweeps(double2* Gp, double* rc, double2* rs,
+                                            double2 (*Ws)[JP + 2], const PairThread& t,
+                                            double tol2, double abs_tol2, int inner_sweeps) {
+  static_assert(4 * PT <= JP * (JP + 2), "the second buffer fits into Ws");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q = lane & 15;
+  const bool first = q == 0, last = q == PP - 1;
+  const int rounds = inner_sweeps * (JP - 1);
+  double2* from = Gp;
+  double2* to = &Ws[0][0];
+  auto put = [&](unsigned place, double2 v) {   // place in the upper 16 bits
+    v.y = __hiloint2double(__double2hiint(v.y) ^ (int)(place & 0x80000000u),
+                           __double2loint(v.y));
+    to[(place >> 16) & 0x7fffu] = v;
+  };
+  if (wave == 0) {
+    // Pair q's next columns come from pairs q + 1 (its a) and q - 1 (its b); at
+    // the ends a_0 stays, b_0 was a_1, and a_last was b_last. Lane 0 has its two
+    // columns the other way round (its apq is the conjugate, its s -conj(s)):
+    // what enters at the ends of the lanes is then the value that a lane
+    // without a source keeps, but for one selection. Of the block (q1, q2) of
+    // those two pairs the entry (x, y) is wanted, x, y = b, a in the middle, a, a
+    // at the first and b, b at the last: with the columns' c it is rotated to
+    // c1 (c2 E_cc + z2 E_cs) + z1 (c2 E_sc + z2 E_ss), where E_c. is the column's
+    // own entry, E_s. the other column's, and z = -s (row) or -conj(s) (column)
+    // for an a, conj(s) (row) or s (column) for a b.
+    const int q1 = first ? 0 : last ? PP - 2 : q - 1, q2 = first ? 1 : last ? PP - 1 : q + 1;
+    const int row = first ? 0 : 1, col = last ? 1 : 0;
+    const int blk = gram_block(q1, q2);
+    const int cc = (2 * row + col) * PT + blk, cs = (2 * row + (col ^ 1)) * PT + blk;
+    const int sc = (2 * (row ^ 1) + col) * PT + blk;
+    const int ss = (2 * (row ^ 1) + (col ^ 1)) * PT + blk;
+    const double z1x = first ? -1.0 : 1.0, z2x = last ? 1.0 : -1.0, sx = first ? -1.0 : 1.0;
+    const unsigned dst = t.dst[0] ^ (first ? 0x80000000u : 0u);
+    const int dq = gram_block(q, q);
+    double app = Gp[(first ? 3 : 0) * PT + dq].x, aqq = Gp[(first ? 0 : 3) * PT + dq].x;
+    double c, shift;
+    double2 apq = Gp[PT + dq], s;
+    if (first) apq.y = -apq.y;
+    bool need = gram_rotation(true, app, aqq, apq, tol2, abs_tol2, c, s, shift);
+    rc[q] = c;       // (the four rows of lanes are alike)
+    rs[q] = make_double2(sx * s.x, s.y);
+    __syncthreads();
+    for (int round = 0; round < rounds; ++round) {
+      const double* const c_ = rc + (round & 1) * PP;
+      const double2* const s_ = rs + (round & 1) * PP;
+      const double2 ecc = from[cc], ecs = from[cs], esc = from[sc], ess = from[ss];
+      const double c1 = c_[q1], c2 = c_[q2];
+      const double2 s1 = s_[q1], s2 = s_[q2];
+      put(dst, need ? make_double2(0.0, 0.0) : apq);
+      const double na = app - shift, nb = aqq + shift;
+      const double x = first ? na : nb;
+      aqq = dpp_keep_d<kDppRowShr1>(nb, x);
+      app = dpp_keep_d<kDppRowShl1>(x, na);
+      const double2 z1 = make_double2(z1x * s1.x, -s1.y);
+      const double2 z2 = make_double2(z2x * s2.x, s2.y);
+      const double2 n0 = cadd(cscale(ecc, c2), cmul(z2, ecs));
+      const double2 n1 = cadd(cscale(esc, c2), cmul(z2, ess));
+      apq = cconj(cadd(cscale(n0, c1), cmul(z1, n1)));
+      need = gram_rotation(true, app, aqq, apq, tol2, abs_tol2, c, s, shift);
+      const int at = ((round + 1) & 1) * PP + q;
+      rc[at] = c;
+      rs[at] = make_double2(sx * s.x, s.y);
+      double2* const y = from;
+      from = to;
+      to = y;
+      __syncthreads();
+    }
+    __syncthreads();
+  } else {
+    // rows of W, four at a time: 0 to 23 wavefront 3, 24 to 27 wavefront 1, 28 to
+    // 31 wavefront 2
+    const int row0 = (wave == 3 ? 0 : 20 + 4 * wave) + (lane >> 4);
+    const int ca = q, cb = JP - 1 - q;    // (lane 0 the other way round, as above)
+    const double sx = first ? -1.0 : 1.0;
+    const bool own = tid - 64 < kPairOwners;
+    const int b = gram_block(t.q1, t.q2);
+    constexpr int kRows = 6;
+    double2 wa[kRows], wb[kRows];
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+      wa[h] = make_double2(row0 + 4 * h == ca ? 1.0 : 0.0, 0.0);
+      wb[h] = make_double2(row0 + 4 * h == cb ? 1.0 : 0.0, 0.0);
+    }
+    __syncthreads();
+    for (int round = 0; round < rounds; ++round) {
+      const double* const c_ = rc + (round & 1) * PP;
+      const double2* const s_ = rs + (round & 1) * PP;
+      const double c = c_[q];
+      const double2 s = make_double2(sx * s_[q].x, s_[q].y);
+      auto rows = [&](int h) __attribute__((always_inline)) {
+        const double2 ya = csub(cscale(wa[h], c), cmul(cconj(s), wb[h]));
+        const double2 yb = cadd(cmul(s, wa[h]), cscale(wb[h], c));
+        const double2 x = make_double2(first ? ya.x : yb.x, first ? ya.y : yb.y);
+        wb[h] = make_double2(dpp_keep_d<kDppRowShr1>(yb.x, x.x), dpp_keep_d<kDppRowShr1>(yb.y, x.y));
+        wa[h] = make_double2(dpp_keep_d<kDppRowShl1>(x.x, ya.x), dpp_keep_d<kDppRowShl1>(x.y, ya.y));
+      };
+      if (wave == 3) {
+#pragma unroll
+        for (int h = 1; h < kRows; ++h) rows(h);
+      } else if (own) {
+        const double2 b00 = from[b], b01 = from[PT + b];
+        const double2 b10 = from[2 * PT + b], b11 = from[3 * PT + b];
+        const double c1 = c_[t.q1], c2 = c_[t.q2];
+        const double2 s1 = s_[t.q1], s2 = s_[t.q2];
+        const double2 s1c = cconj(s1), s2c = cconj(s2);
+        const double2 n00 = csub(cscale(b00, c2), cmul(s2c, b01));
+        const double2 n01 = cadd(cmul(s2, b00), cscale(b01, c2));
+        const double2 n10 = csub(cscale(b10, c2), cmul(s2c, b11));
+        const double2 n11 = cadd(cmul(s2, b10), cscale(b11, c2));
+        put(t.dst[0] << 16, csub(cscale(n00, c1), cmul(s1, n10)));
+        put(t.dst[0], csub(cscale(n01, c1), cmul(s1, n11)));
+        put(t.dst[1] << 16, cadd(cmul(s1c, n00), cscale(n10, c1)));
+        put(t.dst[1], cadd(cmul(s1c, n01), cscale(n11, c1)));
+      }
+      rows(0);
+      double2* const y = from;
+      from = to;
+      to = y;
+      __syncthreads();
+    }
+    __syncthreads();   // (wavefront 0 has left the buffers too)
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+      if (h >= 1 && wave != 3) break;
+      Ws[row0 + 4 * h][ca] = wa[h];
+      Ws[row0 + 4 * h][cb] = wb[h];
+    }
+  }
+  __syncthreads();
+}
+
+// power of two that brings ||X||_F^2 to [1, 4) (1 where that is not a number)
+__device__ __forceinline__ double gram_scaling(double fro2) {
+  return (fro2 > 0.0 && fro2 < 1.7e308) ? ldexp(1.0, -2 * (ilogb(fro2) >> 1)) : 1.0;
 }
 
 // One 32-row chunk of the pair's 32 columns (rows r0.., below hi), four
@@ -679,14 +823,11 @@ __device__ __forceinline__ void put_chunk(double2 (*Xs)[JP + 1], const double2 (
 __device__ __forceinline__ void jacobi_body(const JacobiArgs& a, const int bid,
                                             const unsigned nblk) {
   __shared__ double2 Xs[JR][JP + 1];
-  // rows padded by two entries: the sub-steps' scattered 16-byte accesses
-  // conflict less in the LDS banks than with one
-  __shared__ double2 Gs[2][JP][JP + 2];
+  __shared__ double2 Gp[4 * PT];              // the pair's Gram matrix, by position
   __shared__ double2 Ws[JP][JP + 2];
-  // the pairs (p | q << 8, p < q) of every sub-step of the inner sweep
-  __shared__ int ptab[JP - 1][JB];
+  __shared__ double2 rot_s[2 * PP];
+  __shared__ double rot_c[2 * PP];
   __shared__ int cols[JP];
-  __shared__ int need;
   __shared__ bool skip_pair;
   __shared__ double red[JT];
 
@@ -696,11 +837,7 @@ __device__ __forceinline__ void jacobi_body(const JacobiArgs& a, const int bid,
   const int x_lo = min(a.m, slice * a.xrows_per), x_hi = min(a.m, x_lo + a.xrows_per);
   const int v_lo = min(a.n, slice * a.vrows_per), v_hi = min(a.n, v_lo + a.vrows_per);
   unsigned epoch = 0;
-  for (int e = tid; e < (JP - 1) * JB; e += JT) {
-    int p, q;
-    ordered_pair(e / JB, e % JB, p, q);
-    ptab[e / JB][e % JB] = p | (q << 8);
-  }
+  const PairThread pt = pair_thread(R);
 
   // V = identity, Frobenius norm of X
   for (long e = bid * (long)JT + tid; e < (long)a.n * a.n;
@@ -722,10 +859,11 @@ __device__ __forceinline__ void jacobi_body(const JacobiArgs& a, const int bid,
   }
   if (tid == 0) atomicAdd(a.fro2, red[0]);
   grid_barrier_all(a.bar, nblk, bid, epoch);
-  const double fro = sqrt(__hip_atomic_load(a.fro2, __ATOMIC_RELAXED,
-                                            __HIP_MEMORY_SCOPE_AGENT));
-  const double abs_tol = a.abs_tol_scale * fro;
-  const double tol2 = a.tol * a.tol, abs_tol2 = abs_tol * abs_tol;
+  // the pairs' Gram matrices are scaled with ||X||_F^2 (gram_scaling)
+  const double fro2 = ld_agent(a.fro2);
+  const double gsc = gram_scaling(fro2);
+  const double tol2 = a.tol * a.tol;
+  const double abs_tol2 = a.abs_tol_scale * a.abs_tol_scale * (fro2 * gsc);
   const int ti = tid >> 4, tj = tid & 15;        // 2x2 Gram blocking
   const int npairs = a.nb / 2;
   unsigned* pair_bar = a.bar + kBarrierWords;
@@ -762,7 +900,7 @@ __device__ __forceinline__ void jacobi_body(const JacobiArgs& a, const int bid,
       }
       __syncthreads();
       RTRACE(1);
-      if (skip_pair) {
+      if (__builtin_amdgcn_readfirstlane((int)skip_pair)) {
         // the pair barrier is kept in a skipped round: without it a slice
         // could finish the next round before a slower slice of its pair
         // finished this one, and the arrival count on pair_done, which
@@ -800,7 +938,13 @@ __device__ __forceinline__ void jacobi_body(const JacobiArgs& a, const int bid,
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
-          for (int v = 0; v < 2; ++v) Gs[0][ti + 16 * u][tj + 16 * v] = g[u][v];
+          for (int v = 0; v < 2; ++v) {
+            const int i = ti + 16 * u, j = tj + 16 * v;
+            bool conj;
+            const int at = gram_place(gram_pos(i, PP), gram_pos(j, PP), PT, conj);
+            const double y = i == j ? 0.0 : (conj ? -g[u][v].y : g[u][v].y);
+            if (i <= j) Gp[at] = make_double2(g[u][v].x * gsc, y * gsc);
+          }
       } else {
         // double-buffered by round parity (every round of a pair, skipped or
         // not, passes its pair barrier)
@@ -837,29 +981,10 @@ __device__ __forceinline__ void jacobi_body(const JacobiArgs& a, const int bid,
               if (sl0 + t < R) acc[q] = cadd(acc[q], v[t][q]);
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int e = tid + JT * q;
-          Gs[0][e / JP][e % JP] = acc[q];
-        }
-      }
-      for (int e = tid; e < JP * JP; e += JT)
-        Ws[e / JP][e % JP] = make_double2((e / JP) == (e % JP) ? 1.0 : 0.0, 0.0);
-      if (tid == 0) need = 0;
-      __syncthreads();
-      // ---- does the pair need a rotation? ----
-      {
-        int mine = 0;
-        for (int e = tid; e < JP * JP; e += JT) {
-          const int gi = e / JP, gj = e % JP;
-          if (gi < gj && cols[gi] >= 0 && cols[gj] >= 0) {
-            if (needs_rotation(Gs[0][gi][gi].x, Gs[0][gj][gj].x, cabs2(Gs[0][gi][gj]), tol2,
-                               abs_tol2))
-              mine = 1;
-          }
-        }
-        if (mine) need = 1;
+        for (int q = 0; q < 4; ++q) pair_store(Gp, pt, q, acc[q], gsc);
       }
       __syncthreads();
+      const bool need = pair_needs(Gp, pt, tol2, abs_tol2);
       PHASE(2);
       RTRACE(4);
       // record the outcome for later rounds: a rotated pair's blocks change,
@@ -874,8 +999,7 @@ __device__ __forceinline__ void jacobi_body(const JacobiArgs& a, const int bid,
         }
       }
       if (need) {
-        const unsigned vmask = pair_valid_mask(bi, bj, a.n);
-        pair_inner_sweeps(Gs, Ws, ptab, vmask, tol2, abs_tol2, a.inner_sweeps);
+        pair_sweeps(Gp, rot_c, rot_s, Ws, pt, tol2, abs_tol2, a.inner_sweeps);
         PHASE(3);
         RTRACE(5);
         // ---- X_pair <- X_pair Ws, V_pair <- V_pair Ws over this slice ----
@@ -961,7 +1085,9 @@ __device__ __forceinline__ void jacobi_body(const JacobiArgs& a, const int bid,
   if (bid == 0 && tid == 0) *a.info = converged ? sweep + 1 : -1;
 }
 
-__global__ void __launch_bounds__(JT)
+// Two workgroups a CU: the row slices of a pair are split over twice as many
+// (2652 x 2364: 265 ms; 451 ms with one).
+__global__ void __launch_bounds__(JT, 2)
 jacobi_kernel(JacobiArgs a) {
   jacobi_body(a, blockIdx.x, gridDim.x);
 }
@@ -969,7 +1095,7 @@ jacobi_kernel(JacobiArgs a) {
 // Several independent SVDs in one cooperative launch: workgroup b works on
 // problem block_prob[b] as its (b - starts[p])-th workgroup of
 // starts[p+1] - starts[p]; every problem has its own barrier counter.
-__global__ void __launch_bounds__(JT)
+__global__ void __launch_bounds__(JT, 2)
 jacobi_batch_kernel(const JacobiArgs* probs, const int* starts, const int* block_prob) {
   const int p = block_prob[blockIdx.x];
   const int s0 = starts[p];
@@ -992,11 +1118,11 @@ static_assert(kTileLd == JP + 1, "tile row stride");
 __device__ __forceinline__ void jacobi_tile_body(const JacobiArgs& a, const int bid,
                                                  const unsigned nblk) {
   extern __shared__ double2 tile[];
-  __shared__ double2 Gs[2][JP][JP + 2];
+  __shared__ double2 Gp[4 * PT];              // the pair's Gram matrix, by position
   __shared__ double2 Ws[JP][JP + 2];
-  __shared__ int ptab[JP - 1][JB];
+  __shared__ double2 rot_s[2 * PP];
+  __shared__ double rot_c[2 * PP];
   __shared__ int cols[JP];
-  __shared__ int need;
   __shared__ bool skip_pair;
   __shared__ double red[JT];
 
@@ -1017,11 +1143,7 @@ __device__ __forceinline__ void jacobi_tile_body(const JacobiArgs& a, const int 
   const __amdgpu_buffer_rsrc_t grs =
       agent_rsrc(a.gpart, (unsigned)min(2L * (a.nb / 2) * a.slices * (JP * JP) * 16, 0x7fffffffL));
   unsigned epoch = 0;
-  for (int e = tid; e < (JP - 1) * JB; e += JT) {
-    int p, q;
-    ordered_pair(e / JB, e % JB, p, q);
-    ptab[e / JB][e % JB] = p | (q << 8);
-  }
+  const PairThread pt = pair_thread(R);
 
   // V = identity, Frobenius norm of X
   for (long e = bid * (long)JT + tid; e < (long)a.n * a.n; e += (long)nblk * JT) {
@@ -1041,10 +1163,11 @@ __device__ __forceinline__ void jacobi_tile_body(const JacobiArgs& a, const int 
   }
   if (tid == 0) atomicAdd(a.fro2, red[0]);
   grid_barrier_all(a.bar, nblk, bid, epoch);
-  const double fro = sqrt(__hip_atomic_load(a.fro2, __ATOMIC_RELAXED,
-                                            __HIP_MEMORY_SCOPE_AGENT));
-  const double abs_tol = a.abs_tol_scale * fro;
-  const double tol2 = a.tol * a.tol, abs_tol2 = abs_tol * abs_tol;
+  // the pairs' Gram matrices are scaled with ||X||_F^2 (gram_scaling)
+  const double fro2 = ld_agent(a.fro2);
+  const double gsc = gram_scaling(fro2);
+  const double tol2 = a.tol * a.tol;
+  const double abs_tol2 = a.abs_tol_scale * a.abs_tol_scale * (fro2 * gsc);
   const int npairs = a.nb / 2;
   unsigned* pair_bar = a.bar + kBarrierWords;
   unsigned* pair_done = pair_bar + npairs;
@@ -1077,7 +1200,7 @@ __device__ __forceinline__ void jacobi_tile_body(const JacobiArgs& a, const int 
       }
       __syncthreads();
       RTRACE(1);
-      if (skip_pair) {
+      if (__builtin_amdgcn_readfirstlane((int)skip_pair)) {
         // the pair barrier is kept in a skipped round (see jacobi_body)
         if (R > 1) grid_barrier(pair_bar + pair, R, pair_epoch);
       } else {
@@ -1129,7 +1252,7 @@ __device__ __forceinline__ void jacobi_tile_body(const JacobiArgs& a, const int 
           for (int r = 0; r < 4; ++r) {
             const int gi = 16 * I + 4 * r + lk, gj = 16 * J + lr;
             const double2 g = make_double2(p1[r] - p2[r], p3[r] - p1[r] - p2[r]);
-            if (R == 1) Gs[0][gi][gj] = g;
+            if (R == 1) pair_store(Gp, pt, r, g, gsc);
             else st_agent16(grs, (unsigned)((mine - a.gpart) + gi * JP + gj) * 16u, g);
           }
         }
@@ -1162,29 +1285,10 @@ __device__ __forceinline__ void jacobi_tile_body(const JacobiArgs& a, const int 
                 if (sl0 + t < R) acc[q] = cadd(acc[q], v[t][q]);
           }
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int e = tid + JT * q;
-            Gs[0][e / JP][e % JP] = acc[q];
-          }
-        }
-        for (int e = tid; e < JP * JP; e += JT)
-          Ws[e / JP][e % JP] = make_double2((e / JP) == (e % JP) ? 1.0 : 0.0, 0.0);
-        if (tid == 0) need = 0;
-        __syncthreads();
-        // ---- does the pair need a rotation? ----
-        {
-          int mine = 0;
-          for (int e = tid; e < JP * JP; e += JT) {
-            const int gi = e / JP, gj = e % JP;
-            if (gi < gj && cols[gi] >= 0 && cols[gj] >= 0) {
-              if (needs_rotation(Gs[0][gi][gi].x, Gs[0][gj][gj].x, cabs2(Gs[0][gi][gj]), tol2,
-                                 abs_tol2))
-                mine = 1;
-            }
-          }
-          if (mine) need = 1;
+          for (int q = 0; q < 4; ++q) pair_store(Gp, pt, q, acc[q], gsc);
         }
         __syncthreads();
+        const bool need = pair_needs(Gp, pt, tol2, abs_tol2);
         RTRACE(4);
         // record the outcome for later rounds: a rotated pair's blocks change,
         // an unrotated pair is converged as long as they do not
@@ -1198,8 +1302,7 @@ __device__ __forceinline__ void jacobi_tile_body(const JacobiArgs& a, const int 
           }
         }
         if (need) {
-          pair_inner_sweeps(Gs, Ws, ptab, pair_valid_mask(bi, bj, a.n), tol2, abs_tol2,
-                            a.inner_sweeps);
+          pair_sweeps(Gp, rot_c, rot_s, Ws, pt, tol2, abs_tol2, a.inner_sweeps);
           RTRACE(5);
           // ---- tile <- tile W on the matrix cores: B = W (lane: k = 4 k4 +
           // lk, column lr of the 16-column half v), A = 16 tile rows ----
@@ -2030,29 +2133,6 @@ build_rh_batch_kernel(const RhArgs* pa) {
 // against 0.9 ms of jacobi_tile_kernel; 88 x 83 matrix in small_svd_kernel:
 // 0.82 ms against 1.83 ms with the one-sided sweeps in LDS, QR included.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int gram_block(int q1, int q2) { return q2 * (q2 + 1) / 2 + q1; }
-
-// position of column c in round 0 (P pairs) and a position's next one
-__device__ __forceinline__ int gram_pos(int c, int P) {
-  const int L = 2 * P - 1;
-  return c == L ? 0 : c == 0 ? 1 : c < P ? 2 * c : 2 * (L - c) + 1;
-}
-__device__ __forceinline__ int gram_next(int x, int P) {
-  if (x == 0 || P == 1) return x;
-  if (x == 2) return 1;
-  if ((x & 1) == 0) return x - 2;
-  return x == 2 * P - 1 ? x - 1 : x + 2;
-}
-
-// where the entry of positions (x, y) is kept (T: entries of a plane), and
-// whether conjugated
-__device__ __forceinline__ int gram_place(int x, int y, int T, bool& conj) {
-  const int qx = x >> 1, qy = y >> 1;
-  conj = qx > qy || (qx == qy && x > y);
-  if (conj) return (2 * (y & 1) + (x & 1)) * T + gram_block(qy, qx);
-  return (2 * (x & 1) + (y & 1)) * T + gram_block(qx, qy);
-}
-
 // 16 x 16 tile t of the upper triangle of Y^H Y (list (0,0), (0,1), (1,1),
 // (0,2), ...) by one wavefront, 3M on the FP64 matrix cores; Y is n x r with
 // leading dimension ld. Lane l gets rows 4 q + l / 16 of column l % 16.
@@ -2111,27 +2191,6 @@ __device__ __forceinline__ void gram_store(double2* G, int r, int t, const doubl
     const double im = i == j ? 0.0 : g[q].y;
     G[at] = make_double2(g[q].x, conj ? -im : im);
   }
-}
-
-// Rotation of the 2 x 2 block [[app, apq], [conj(apq), aqq]]: with
-// d = aqq - app and h = sqrt(d^2 + 4 |apq|^2), c = cos(theta) =
-// sqrt((h + |d|) / 2h) and s = sign(d) apq / (h c) (jacobi_rotation_fast's
-// formulas; the phase of apq stays in s, so its modulus is not needed, and G is
-// scaled, so the block is not). The identity where no rotation is needed.
-__device__ __forceinline__ void gram_rotation(bool valid, double app, double aqq, double2 apq,
-                                              double tol2, double abs_tol2, double& c,
-                                              double2& s) {
-  const double mag2 = cabs2(apq);
-  const bool need = valid & (mag2 > tol2 * fabs(app * aqq)) &
-                    (mag2 > abs_tol2 * fmax(fmax(app, aqq), 0.0)) & (mag2 > 0.0);
-  const double d = aqq - app;
-  const double h2 = need ? fma(d, d, 4.0 * mag2) : 1.0;
-  const double rh = rsqrt_nr(h2);
-  const double cos2 = fma(0.5 * fabs(d), rh, 0.5);
-  const double rc = rsqrt_nr(cos2);
-  const double f = copysign(rh * rc, d < 0.0 ? -1.0 : 1.0);
-  c = need ? cos2 * rc : 1.0;
-  s = make_double2(need ? apq.x * f : 0.0, need ? apq.y * f : 0.0);
 }
 
 // Two-sided Jacobi sweeps on G (rank r) in LDS; rc, rs: LDS scratch of 64
