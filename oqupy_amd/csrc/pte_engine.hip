@@ -117,6 +117,46 @@ static DTensor dupload(const std::vector<cplx>& h, int a, int b, int c, int e,
   return t;
 }
 
+// Entries from which the finite check of an input runs on the device: about
+// 30 us with its read-back, against 0.1 us per 16 x 64 entries read on the host.
+constexpr long kDeviceCheckMin = 1L << 14;
+
+// A matrix from the caller's memory, which the stream may read until it is
+// synchronised; non-finite values are an error. (The upload through a host copy
+// that was checked entry by entry cost more than the transfer: for the three
+// matrices of a 2652 x 2364 split and product about 100 ms of 497.)
+static DTensor dupload_checked(const double* data, int rows, int cols, hipStream_t s) {
+  const long count = 2L * rows * cols;
+  const bool on_device = (long)rows * cols >= kDeviceCheckMin;
+  int bad = 0;
+  if (!on_device) {
+    for (long i = 0; i < count; ++i) bad |= !std::isfinite(data[i]);
+    require(!bad, PTE_ERR_NUMERIC, "non-finite value in an input tensor");
+  }
+  DTensor t = dalloc(rows, cols, 1, 1, s);
+  try {
+    HIP_CHECK(hipMemcpyAsync(t.p, data, count * sizeof(double), hipMemcpyHostToDevice, s));
+    if (on_device) {
+      DTensor flag = dalloc(1, 1, 1, 1, s);
+      int* const flag_d = reinterpret_cast<int*>(flag.p);
+      hipError_t err = hipMemsetAsync(flag_d, 0, sizeof(int), s);
+      if (err == hipSuccess) {
+        finite_check_kernel<<<grid_for(count), 256, 0, s>>>(t.p, (long)rows * cols, flag_d);
+        err = hipMemcpyAsync(&bad, flag_d, sizeof(int), hipMemcpyDeviceToHost, s);
+      }
+      const hipError_t end = hipStreamSynchronize(s);
+      dfree(flag, s);
+      HIP_CHECK(err);
+      HIP_CHECK(end);
+      require(!bad, PTE_ERR_NUMERIC, "non-finite value in an input tensor");
+    }
+  } catch (...) {
+    dfree(t, s);
+    throw;
+  }
+  return t;
+}
+
 // An influence node [west][in][out][east]; middle nodes of the delta form
 // W[w,p,s,v] = delta(w,v) delta(p,s) I[w,p] keep only I (west-major).
 struct Node {
@@ -280,6 +320,8 @@ struct Workspace {
   unsigned* jskip = nullptr;   // converged-pair bookkeeping of the Jacobi
   size_t jskip_cap = 0;        // words
   int jskip_words = 0;         // words the last prepared Jacobi uses
+  char* fixed_d = nullptr;     // bar, flags, fro2, info_d, qr_cand and qr_rank_d
+  char* fixed_h = nullptr;     // info_h and qr_rank_h (pinned)
   int* flags = nullptr;
   double* fro2 = nullptr;
   SvdInfo* info_d = nullptr;
@@ -338,12 +380,10 @@ struct Workspace {
     log_shapes.push_back(k);
   }
 
-  void init(double eps, int cap) {
-    epsrel = eps;
-    chi_cap = cap;
+  // the stream alone: all that a contraction needs
+  void init_stream() {
     HIP_CHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     svd_stream = stream;
-    HIP_CHECK(hipEventCreateWithFlags(&ev_ready, hipEventDisableTiming));
     hipMemPool_t pool;
     int dev = 0;
     HIP_CHECK(hipGetDevice(&dev));
@@ -351,11 +391,46 @@ struct Workspace {
       uint64_t thr = ~0ull;
       (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &thr);
     }
-    HIP_CHECK(hipMalloc((void**)&bar, sizeof(unsigned) * kSyncWords));
-    HIP_CHECK(hipMalloc((void**)&flags, sizeof(int) * max_sweeps));
-    HIP_CHECK(hipMalloc((void**)&fro2, sizeof(double)));
-    HIP_CHECK(hipMalloc((void**)&info_d, sizeof(SvdInfo)));
-    HIP_CHECK(hipHostMalloc((void**)&info_h, sizeof(SvdInfo), hipHostMallocDefault));
+  }
+
+  // 256-byte aligned parts of one allocation (an allocation and its release are
+  // 10 to 15 us each, 50 in pinned memory)
+  struct Parts {
+    size_t size = 0;
+    size_t add(size_t bytes) {
+      const size_t at = size;
+      size += (bytes + 255) & ~(size_t)255;
+      return at;
+    }
+  };
+
+  void init(double eps, int cap) {
+    epsrel = eps;
+    chi_cap = cap;
+    init_stream();
+    HIP_CHECK(hipEventCreateWithFlags(&ev_ready, hipEventDisableTiming));
+    int dev = 0;
+    HIP_CHECK(hipGetDevice(&dev));
+    Parts parts;
+    const size_t at_bar = parts.add(sizeof(unsigned) * kSyncWords);
+    const size_t at_flags = parts.add(sizeof(int) * max_sweeps);
+    const size_t at_fro2 = parts.add(sizeof(double));
+    const size_t at_info = parts.add(sizeof(SvdInfo));
+    const size_t at_cand = parts.add(sizeof(QrcpCand) * 2 * 256);
+    const size_t at_rank = parts.add(sizeof(int));
+    HIP_CHECK(hipMalloc((void**)&fixed_d, parts.size));
+    bar = reinterpret_cast<unsigned*>(fixed_d + at_bar);
+    flags = reinterpret_cast<int*>(fixed_d + at_flags);
+    fro2 = reinterpret_cast<double*>(fixed_d + at_fro2);
+    info_d = reinterpret_cast<SvdInfo*>(fixed_d + at_info);
+    qr_cand = reinterpret_cast<QrcpCand*>(fixed_d + at_cand);
+    qr_rank_d = reinterpret_cast<int*>(fixed_d + at_rank);
+    Parts host;
+    const size_t at_hinfo = host.add(sizeof(SvdInfo));
+    const size_t at_hrank = host.add(sizeof(int));
+    HIP_CHECK(hipHostMalloc((void**)&fixed_h, host.size, hipHostMallocDefault));
+    info_h = reinterpret_cast<SvdInfo*>(fixed_h + at_hinfo);
+    qr_rank_h = reinterpret_cast<int*>(fixed_h + at_hrank);
     int per_cu = 0;
     HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &per_cu, reinterpret_cast<const void*>(jacobi_kernel), 256, 0));
@@ -366,9 +441,6 @@ struct Workspace {
     require(prop.sharedMemPerBlock >= kSmallLdsMax + 1024, PTE_ERR_DEVICE,
             "the engine needs 160 KiB of LDS per workgroup (gfx950)");
     init_tile_kernel();
-    HIP_CHECK(hipMalloc((void**)&qr_cand, sizeof(QrcpCand) * 2 * 256));
-    HIP_CHECK(hipMalloc((void**)&qr_rank_d, sizeof(int)));
-    HIP_CHECK(hipHostMalloc((void**)&qr_rank_h, sizeof(int), hipHostMallocDefault));
     require(max_coop_blocks > 0, PTE_ERR_DEVICE, "Jacobi kernel cannot be resident");
     HIP_CHECK(hipEventCreate(&ev0));
     HIP_CHECK(hipEventCreate(&ev1));
@@ -482,17 +554,12 @@ struct Workspace {
     carry.release(stream); carry2.release(stream); svh.release(stream);
     gpart.release(stream); Q.release(stream);
     (void)hipStreamSynchronize(stream);
-    (void)hipFree(qr_tau); (void)hipFree(qr_vscale); (void)hipFree(qr_beta);
-    (void)hipFree(qr_piv); (void)hipFree(qr_done); (void)hipFree(qr_cand);
-    (void)hipFree(qr_rank_d); (void)hipHostFree(qr_rank_h);
-    (void)hipFree(sigma); (void)hipFree(sorted); (void)hipFree(perm);
-    (void)hipFree(bar); (void)hipFree(jskip); (void)hipFree(flags); (void)hipFree(fro2);
-    (void)hipFree(info_d);
-    (void)hipHostFree(info_h);
-    (void)hipEventDestroy(ev0); (void)hipEventDestroy(ev1);
-    (void)hipEventDestroy(evj0); (void)hipEventDestroy(evj1);
-    (void)hipEventDestroy(evq0); (void)hipEventDestroy(evq1);
-    (void)hipEventDestroy(ev_ready);
+    // qr_tau and sigma are the first parts of their allocations
+    for (void* p : {(void*)qr_tau, (void*)sigma, (void*)jskip, (void*)fixed_d})
+      if (p) (void)hipFree(p);
+    if (fixed_h) (void)hipHostFree(fixed_h);
+    for (hipEvent_t ev : {ev0, ev1, evj0, evj1, evq0, evq1, ev_ready})
+      if (ev) (void)hipEventDestroy(ev);
     if (trace) std::fclose(trace);
     trace = nullptr;
     (void)hipStreamDestroy(stream);
@@ -504,11 +571,18 @@ struct Workspace {
     require(!external, PTE_ERR_CAPACITY, "matrix exceeds the allocation-free workspace");
     HIP_CHECK(hipStreamSynchronize(stream));
     HIP_CHECK(hipStreamSynchronize(svd_stream));
-    (void)hipFree(sigma); (void)hipFree(sorted); (void)hipFree(perm);
+    (void)hipFree(sigma);
+    sigma = nullptr;
+    nsv_cap = 0;
     size_t c = std::max<size_t>(n, 1024);
-    HIP_CHECK(hipMalloc((void**)&sigma, c * sizeof(double)));
-    HIP_CHECK(hipMalloc((void**)&sorted, c * sizeof(double)));
-    HIP_CHECK(hipMalloc((void**)&perm, c * sizeof(int)));
+    Parts parts;
+    parts.add(c * sizeof(double));
+    const size_t at_sorted = parts.add(c * sizeof(double));
+    const size_t at_perm = parts.add(c * sizeof(int));
+    HIP_CHECK(hipMalloc((void**)&sigma, parts.size));
+    char* const base = reinterpret_cast<char*>(sigma);
+    sorted = reinterpret_cast<double*>(base + at_sorted);
+    perm = reinterpret_cast<int*>(base + at_perm);
     nsv_cap = c;
   }
 
@@ -707,14 +781,22 @@ struct Workspace {
     require(!external, PTE_ERR_CAPACITY, "matrix exceeds the allocation-free workspace");
     HIP_CHECK(hipStreamSynchronize(stream));
     HIP_CHECK(hipStreamSynchronize(svd_stream));
-    (void)hipFree(qr_tau); (void)hipFree(qr_vscale); (void)hipFree(qr_beta);
-    (void)hipFree(qr_piv); (void)hipFree(qr_done);
+    (void)hipFree(qr_tau);
+    qr_tau = nullptr;
+    qr_cap = 0;
     const size_t c = std::max<size_t>(n, 1024);
-    HIP_CHECK(hipMalloc((void**)&qr_tau, c * sizeof(double2)));
-    HIP_CHECK(hipMalloc((void**)&qr_vscale, c * sizeof(double2)));
-    HIP_CHECK(hipMalloc((void**)&qr_beta, c * sizeof(double)));
-    HIP_CHECK(hipMalloc((void**)&qr_piv, c * sizeof(int)));
-    HIP_CHECK(hipMalloc((void**)&qr_done, c * sizeof(int)));
+    Parts parts;
+    parts.add(c * sizeof(double2));
+    const size_t at_vscale = parts.add(c * sizeof(double2));
+    const size_t at_beta = parts.add(c * sizeof(double));
+    const size_t at_piv = parts.add(c * sizeof(int));
+    const size_t at_done = parts.add(c * sizeof(int));
+    HIP_CHECK(hipMalloc((void**)&qr_tau, parts.size));
+    char* const base = reinterpret_cast<char*>(qr_tau);
+    qr_vscale = reinterpret_cast<double2*>(base + at_vscale);
+    qr_beta = reinterpret_cast<double*>(base + at_beta);
+    qr_piv = reinterpret_cast<int*>(base + at_piv);
+    qr_done = reinterpret_cast<int*>(base + at_done);
     qr_cap = c;
   }
 
@@ -3529,12 +3611,13 @@ int pte_contract(int precision, int m, int n, int k, const double* A, const doub
     require(precision == PTE_PRECISION_C128 || precision == PTE_PRECISION_C64, PTE_ERR_ARG,
             "unknown precision");
     Workspace ws;
-    ws.init(1e-7, 1);
+    ws.init_stream();
     ws.precision = precision;
+    DTensor da, db, dc;
     try {
-      DTensor da = dupload(to_cplx(A, (long)m * k), m, k, 1, 1, ws.stream);
-      DTensor db = dupload(to_cplx(B, (long)k * n), k, n, 1, 1, ws.stream);
-      DTensor dc = dalloc(m, n, 1, 1, ws.stream);
+      da = dupload_checked(A, m, k, ws.stream);
+      db = dupload_checked(B, k, n, ws.stream);
+      dc = dalloc(m, n, 1, 1, ws.stream);
       ws.contract(m, n, k, da.p, k, 1, db.p, n, 1, dc.p, n, 1);
       HIP_CHECK(hipGetLastError());
       HIP_CHECK(hipMemcpyAsync(C, dc.p, (size_t)m * n * sizeof(double2),
@@ -3544,6 +3627,9 @@ int pte_contract(int precision, int m, int n, int k, const double* A, const doub
       dfree(db, ws.stream);
       dfree(dc, ws.stream);
     } catch (...) {
+      dfree(da, ws.stream);
+      dfree(db, ws.stream);
+      dfree(dc, ws.stream);
       ws.destroy();
       throw;
     }
@@ -3561,8 +3647,7 @@ int pte_split_svd(int m, int n, const double* M, double epsrel, int chi_cap, dou
     ws.init(epsrel, chi_cap);
     try {
       const long cnt = (long)m * n;
-      std::vector<cplx> h = to_cplx(M, cnt);
-      DTensor dm = dupload(h, m, n, 1, 1, ws.stream);
+      DTensor dm = dupload_checked(M, m, n, ws.stream);
       int k;
       DevBuf u, svh;
       if (m <= kQrMaxRows) {

@@ -222,6 +222,8 @@ __global__ void rank_sort_kernel(const double* sigma, int n, int* perm, double* 
 __global__ void truncate_kernel(const double* sorted, int n, double epsrel, SvdInfo* info,
                                 int max_rank, const double* extra2);
 __global__ void emit_kernel(EmitArgs a);
+// *flag = 1 if a part of the `count` entries is not finite
+__global__ void finite_check_kernel(const double2* x, long count, int* flag);
 __global__ void conj_copy_kernel(const double2* src, long count, double2* dst);
 __global__ void conj_transpose_kernel(const double2* src, int R, int C, double2* dst);
 __global__ void transpose_kernel(const double2* src, int R, int C, double2* dst);

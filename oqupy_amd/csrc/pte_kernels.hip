@@ -3028,6 +3028,16 @@ apply_q_wave_kernel(ApplyQArgs a) {
   if (i1 < m) a.dst[(long)j * dj + (long)(i1 / a.B) * da + (long)(i1 % a.B) * db] = x1;
 }
 
+__global__ void __launch_bounds__(256)
+finite_check_kernel(const double2* x, long count, int* flag) {
+  bool bad = false;
+  for (long e = blockIdx.x * 256L + threadIdx.x; e < count; e += (long)gridDim.x * 256) {
+    const double2 v = x[e];
+    bad |= !(isfinite(v.x) && isfinite(v.y));
+  }
+  if (bad) *flag = 1;
+}
+
 // X (rows x cols, column-major, ld = rows) = conj(src) with src row-major
 // (cols x rows): X[r + c*rows] = conj(src[c*rows + r]) -- a plain conjugate
 __global__ void __launch_bounds__(256)
