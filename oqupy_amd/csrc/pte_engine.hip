@@ -1166,8 +1166,15 @@ struct Workspace {
     aq.B = B;
     aq.dj0 = dj0; aq.djk = djk; aq.da0 = da0; aq.dak = dak; aq.db0 = db0; aq.dbk = dbk;
     aq.dst = dst;
-    if (qr_m <= kApplyQWaveRows)
-      apply_q_wave_kernel<<<(k + 3) / 4, 256, 0, stream>>>(aq);
+    const int grid = (k + 3) / 4;
+    if (qr_m <= 128)
+      apply_q_wave_kernel<2><<<grid, 256, 0, stream>>>(aq);
+    else if (qr_m <= 256)
+      apply_q_wave_kernel<4><<<grid, 256, 0, stream>>>(aq);
+    else if (qr_m <= 512)
+      apply_q_wave_kernel<8><<<grid, 256, 0, stream>>>(aq);
+    else if (qr_m <= kApplyQWaveRows)
+      apply_q_wave_kernel<16><<<grid, 256, 0, stream>>>(aq);
     else
       apply_q_kernel<<<std::min(k, 1024), 256, (size_t)qr_m * sizeof(double2), stream>>>(aq);
   }

@@ -202,8 +202,9 @@ __global__ void gram_replay_kernel(GramReplayArgs a);
 __global__ void gram_replay_batch_kernel(const GramReplayArgs* probs);   // problem = blockIdx.y
 __global__ void gather_qr_rank_kernel(const QrcpArgs* probs, int n, int* out);
 __global__ void apply_q_kernel(ApplyQArgs a);
+template <int RP>
 __global__ void apply_q_wave_kernel(ApplyQArgs a);   // Q of at most kApplyQWaveRows rows
-constexpr int kApplyQWaveRows = 128;
+constexpr int kApplyQWaveRows = 1024;
 __global__ void zgemm_kernel(GemmArgs a);
 __global__ void zgemm_mfma_kernel(GemmArgs a);
 __global__ void cgemm_mfma_kernel(GemmArgs a);
