@@ -1,7 +1,7 @@
 """The Jacobi SVD on the Gram matrix (one workgroup) against LAPACK at the
 edges of its range: odd and even ranks, the 16-column tiles of the Gram
-matrix, the largest rank in the one-workgroup QR (96 columns) and after the
-grid's QR (126), the first rank beyond; repeated singular values, rank
+matrix, the largest rank in one workgroup (126 columns) and after the
+grid's QR, the first rank beyond; repeated singular values, rank
 deficiency, and values whose squares are near the ends of the range."""
 
 import numpy as np
