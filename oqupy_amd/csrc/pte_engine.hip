@@ -117,9 +117,11 @@ static DTensor dupload(const std::vector<cplx>& h, int a, int b, int c, int e,
   return t;
 }
 
-// Entries from which the finite check of an input runs on the device: about
-// 30 us with its read-back, against 0.1 us per 16 x 64 entries read on the host.
-constexpr long kDeviceCheckMin = 1L << 14;
+// Entries from which the finite check of an input runs on the device, where its
+// launch and read-back cost 25 to 40 us: a product of two matrices of 65536
+// entries each takes 500 us so and 433 checked on the host, of 262144 entries 1020
+// and 1070, of 1048576 entries 2780 and 3550.
+constexpr long kDeviceCheckMin = 1L << 17;
 
 // A matrix from the caller's memory, which the stream may read until it is
 // synchronised; non-finite values are an error. (The upload through a host copy
