@@ -330,6 +330,7 @@ struct Workspace {
   SvdInfo* info_h = nullptr;
   int max_sweeps = 80;
   int inner_sweeps = 1;      // tuning: PTE_JACOBI_INNER_SWEEPS
+  int gram_sweeps = kGramMaxSweeps;   // of a pass of the Gram Jacobi; tuning: PTE_GRAM_SWEEPS
   int jacobi_sync_words = kBarrierWords;   // words of `bar` the last prepared Jacobi uses
   int qr_blocks = 256;       // tuning: PTE_QR_BLOCKS (workgroups of the pivoted QR)
   int slice_rows = 64;       // tuning: PTE_JACOBI_SLICE_ROWS (min rows per slice)
@@ -608,11 +609,15 @@ struct Workspace {
         &per_cu, reinterpret_cast<const void*>(jacobi_tile_kernel), 256,
         tile_lds_bytes(kTileMaxRows)));
     tile_coop_blocks = per_cu * num_cus;
-    for (const void* f : {reinterpret_cast<const void*>(gram_svd_kernel),
-                          reinterpret_cast<const void*>(gram_svd_batch_kernel)})
+    for (const void* f : {reinterpret_cast<const void*>(gram_svd_kernel<kSmallThreads>),
+                          reinterpret_cast<const void*>(gram_svd_kernel<kGramThreads>),
+                          reinterpret_cast<const void*>(gram_svd_batch_kernel<kSmallThreads>),
+                          reinterpret_cast<const void*>(gram_svd_batch_kernel<kGramThreads>)})
       HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)gram_lds(kGramMaxRank)));
     if (const char* v = std::getenv("PTE_JACOBI_TILE")) tile_enabled = std::atoi(v) != 0;
+    if (const char* v = std::getenv("PTE_GRAM_SWEEPS"))
+      gram_sweeps = std::max(1, std::min(kGramMaxSweeps, std::atoi(v)));
     if (const char* v = std::getenv("PTE_JACOBI_TILE_ROWS"))
       tile_rows = std::max(32, std::min(kTileMaxRows, std::atoi(v)));
   }
@@ -959,9 +964,10 @@ struct Workspace {
     *logc = reinterpret_cast<double*>(gpart.p + rounds * 64);
   }
 
-  GramReplayArgs replay_args(int n, const double* logc, const double2* logs) const {
+  GramReplayArgs replay_args(const GramSvdArgs& ga, bool first) const {
     GramReplayArgs ra;
-    ra.Y = X.p; ra.n = n; ra.W = V.p; ra.info = info_d; ra.logc = logc; ra.logs = logs;
+    ra.Y = X.p; ra.n = ga.n; ra.first = first ? 1 : 0; ra.W = V.p; ra.info = info_d;
+    ra.logc = ga.logc; ra.logs = ga.logs;
     return ra;
   }
   static unsigned replay_grid(int n, int r) { return (unsigned)((n + r + 3) / 4); }
@@ -981,7 +987,7 @@ struct Workspace {
     sa.Y = X.p;
     sa.sigma = sigma; sa.perm = perm; sa.sorted = sorted; sa.info = info_d;
     sa.epsrel = epsrel; sa.max_rank = chi_cap;
-    sa.max_sweeps = std::min(max_sweeps, kGramMaxSweeps);
+    sa.max_sweeps = gram_sweeps;
     sa.copy = copy;
     sa.stop_rel = 0.0;
     sa.folded = nullptr;
@@ -990,10 +996,11 @@ struct Workspace {
     return sa;
   }
 
-  // the Jacobi of a rank above kGramSmallRank after small_svd_kernel's QR
+  // the passes after small_svd_kernel, from the first one on for ranks above
+  // kGramSmallRank (expect: kGramFresh)
   GramSvdArgs small_rest(const SmallSvdArgs& sa) const {
     GramSvdArgs ga;
-    ga.Y = sa.Y; ga.n = sa.n; ga.r = std::min(sa.m, sa.n); ga.pending = 1;
+    ga.Y = sa.Y; ga.n = sa.n; ga.r = std::min(sa.m, sa.n); ga.expect = kGramFresh;
     ga.sigma = sa.sigma; ga.perm = sa.perm; ga.sorted = sa.sorted; ga.info = sa.info;
     ga.epsrel = sa.epsrel; ga.max_rank = sa.max_rank; ga.max_sweeps = sa.max_sweeps;
     ga.copy = sa.copy;
@@ -1028,23 +1035,16 @@ struct Workspace {
     const bool timed = trace != nullptr;
     if (timed) mark(evj0);
     small_svd_kernel<<<1, kSmallThreads, small_lds(m, n), svd_stream>>>(sa);
-    if (std::min(m, n) > kGramSmallRank)
-      gram_svd_kernel<<<1, kGramThreads, gram_lds(std::min(m, n)), svd_stream>>>(
-          small_rest(sa));
-    gram_replay_kernel<<<replay_grid(n, std::min(m, n)), 256, 0, svd_stream>>>(
-        replay_args(n, sa.logc, sa.logs));
+    const GramSvdArgs ga = small_rest(sa);
+    if (ga.r > kGramSmallRank) gram_launch(ga);
+    const bool done = gram_complete(ga);
     if (timed) mark(evj1);
-    HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipMemcpyAsync(info_h, info_d, sizeof(SvdInfo), hipMemcpyDeviceToHost,
-                             svd_stream));
-    HIP_CHECK(hipStreamSynchronize(svd_stream));
-    if (info_h->sweeps < 0) {
-      // not converged within the log: Y is untouched, the blocked Jacobi
-      // takes it
+    if (!done) {
       small_state(m, n);
       trunc_extra2 = adaptive ? rank->out_d : nullptr;
       int k;
       try {
+        gram_rebuild();
         k = svd(n, qr_r);
       } catch (...) {
         trunc_extra2 = nullptr;
@@ -1053,7 +1053,41 @@ struct Workspace {
       trunc_extra2 = nullptr;
       return k;
     }
+    if (timed) HIP_CHECK(hipEventSynchronize(evj1));
     return small_finish(m, n, timed ? elapsed(evj0, evj1) : 0.f);
+  }
+
+  void gram_launch(const GramSvdArgs& ga) {
+    if (ga.r > kGramSmallRank)
+      gram_svd_kernel<kGramThreads><<<1, kGramThreads, gram_lds(ga.r), svd_stream>>>(ga);
+    else
+      gram_svd_kernel<kSmallThreads><<<1, kSmallThreads, gram_lds(ga.r), svd_stream>>>(ga);
+  }
+
+  // After the launch of the first pass: its replay, the check, and further passes
+  // while one rotated. Their number is known to the device alone, so all but the
+  // first check (enough but for a few matrices) wait for the summary, which is in
+  // info_h at the end. False: not converged, Y as the last pass left it.
+  bool gram_complete(GramSvdArgs ga) {
+    ga.expect = kGramRotated;
+    for (int pass = 2; pass <= kGramMaxPasses; ++pass) {
+      gram_replay_kernel<<<replay_grid(ga.n, ga.r), 256, 0, svd_stream>>>(
+          replay_args(ga, pass == 2));
+      gram_launch(ga);
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipMemcpyAsync(info_h, info_d, sizeof(SvdInfo), hipMemcpyDeviceToHost,
+                               svd_stream));
+      HIP_CHECK(hipStreamSynchronize(svd_stream));
+      if (info_h->state != kGramRotated) break;
+    }
+    return info_h->state == kGramDone;
+  }
+
+  // Y = R^H again, from the factors of the QR (for the blocked Jacobi)
+  void gram_rebuild() {
+    build_rh_kernel<<<grid_for((long)qr_n * qr_r), 256, 0, svd_stream>>>(
+        Q.p, qr_m, qr_n, qr_piv, qr_beta, qr_rank_d, X.p);
+    HIP_CHECK(hipGetLastError());
   }
 
   // Y of at most kGramMaxRank columns, from a pivoted QR (the method relies
@@ -1066,10 +1100,10 @@ struct Workspace {
     ensure_sv((size_t)r);
     V.ensure((size_t)r * r, svd_stream);
     GramSvdArgs ga;
-    ga.Y = X.p; ga.n = n; ga.r = r; ga.pending = 0;
+    ga.Y = X.p; ga.n = n; ga.r = r; ga.expect = 0;
     ga.sigma = sigma; ga.perm = perm; ga.sorted = sorted; ga.info = info_d;
     ga.epsrel = epsrel; ga.max_rank = chi_cap;
-    ga.max_sweeps = std::min(max_sweeps, kGramMaxSweeps);
+    ga.max_sweeps = gram_sweeps;
     ga.copy = copy;
     ga.extra2 = trunc_extra2;
     gram_log(r, &ga.logs, &ga.logc);
@@ -1081,16 +1115,14 @@ struct Workspace {
     GramSvdArgs ga = gram_prepare(n, r, nullptr);
     const bool timed = trace != nullptr;
     if (timed) mark(evj0);
-    gram_svd_kernel<<<1, kGramThreads, gram_lds(r), svd_stream>>>(ga);
-    gram_replay_kernel<<<replay_grid(n, r), 256, 0, svd_stream>>>(
-        replay_args(n, ga.logc, ga.logs));
+    gram_launch(ga);
+    const bool done = gram_complete(ga);
     if (timed) mark(evj1);
-    HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipMemcpyAsync(info_h, info_d, sizeof(SvdInfo), hipMemcpyDeviceToHost,
-                             svd_stream));
-    HIP_CHECK(hipStreamSynchronize(svd_stream));
-    // not converged within the log: Y is untouched
-    if (info_h->sweeps < 0) return svd(n, r);
+    if (!done) {
+      gram_rebuild();
+      return svd(n, r);
+    }
+    if (timed) HIP_CHECK(hipEventSynchronize(evj1));
     return jacobi_check(n, r, timed ? elapsed(evj0, evj1) : 0.f, true);
   }
 
@@ -1478,21 +1510,15 @@ struct Batcher {
   void run_small(std::vector<SvdRequest*>& rs, std::vector<SvdRequest*>* blocked) {
     ensure_gather(rs.size());
     std::vector<SmallSvdArgs> args;
-    std::vector<GramSvdArgs> rest;
-    std::vector<GramReplayArgs> reps;
+    std::vector<GramSvdArgs> grams, rest;
     std::vector<SvdRequest*> in;
-    size_t lds = 0, rest_lds = 0;
-    unsigned gx = 1;
+    size_t lds = 0;
     for (auto* r : rs) {
       try {
         args.push_back(r->ws->small_prepare(r->m, r->n, infos_d + in.size()));
-        reps.push_back(r->ws->replay_args(r->n, args.back().logc, args.back().logs));
+        grams.push_back(r->ws->small_rest(args.back()));
         lds = std::max(lds, Workspace::small_lds(r->m, r->n));
-        if (std::min(r->m, r->n) > kGramSmallRank) {
-          rest.push_back(r->ws->small_rest(args.back()));
-          rest_lds = std::max(rest_lds, Workspace::gram_lds(rest.back().r));
-        }
-        gx = std::max(gx, Workspace::replay_grid(r->n, std::min(r->m, r->n)));
+        if (grams.back().r > kGramSmallRank) rest.push_back(grams.back());
         in.push_back(r);
       } catch (...) {
         fail(r);
@@ -1502,40 +1528,70 @@ struct Batcher {
     for (auto& sa : args) sa.lds_bytes = (long)lds;
     Pack pk;
     const size_t oa = pk.add(args.data(), args.size() * sizeof(SmallSvdArgs));
-    const size_t orp = pk.add(reps.data(), reps.size() * sizeof(GramReplayArgs));
     const size_t ore = pk.add(rest.data(), rest.size() * sizeof(GramSvdArgs));
+    const GramSteps steps = gram_pack(pk, in, grams, true);
     char* base = upload(pk);
     HIP_CHECK(hipEventRecord(ev0, stream));
     small_svd_batch_kernel<<<(unsigned)in.size(), kSmallThreads, lds, stream>>>(
         reinterpret_cast<const SmallSvdArgs*>(base + oa));
-    if (!rest.empty())
-      gram_svd_batch_kernel<<<(unsigned)rest.size(), kGramThreads, rest_lds, stream>>>(
-          reinterpret_cast<const GramSvdArgs*>(base + ore));
-    gram_replay_batch_kernel<<<dim3(gx, (unsigned)in.size()), 256, 0, stream>>>(
-        reinterpret_cast<const GramReplayArgs*>(base + orp));
-    gather(in, [](SvdRequest* r, float ms) { return r->ws->small_finish(r->m, r->n, ms); },
-           [&](SvdRequest* r) {
-             r->ws->small_state(r->m, r->n);
-             r->jm = r->n;
-             r->jn = r->ws->qr_r;
-             blocked->push_back(r);
-           });
+    if (!rest.empty()) gram_launch(rest, base + ore);
+    gram_step(steps, grams, base);
+    gather(in, grams, [](SvdRequest* r, float ms) {
+      return r->ws->small_finish(r->m, r->n, ms);
+    }, [&](SvdRequest* r) {
+      r->ws->small_state(r->m, r->n);
+      r->ws->gram_rebuild();
+      r->jm = r->n;
+      r->jn = r->ws->qr_r;
+      blocked->push_back(r);
+    });
+  }
+
+  // a pass of each
+  void gram_launch(const std::vector<GramSvdArgs>& gs, const char* args) {
+    int rmax = 1;
+    for (const GramSvdArgs& ga : gs) rmax = std::max(rmax, ga.r);
+    const GramSvdArgs* const d = reinterpret_cast<const GramSvdArgs*>(args);
+    const size_t lds = Workspace::gram_lds(rmax);
+    if (rmax > kGramSmallRank)
+      gram_svd_batch_kernel<kGramThreads><<<(unsigned)gs.size(), kGramThreads, lds, stream>>>(d);
+    else
+      gram_svd_batch_kernel<kSmallThreads>
+          <<<(unsigned)gs.size(), kSmallThreads, lds, stream>>>(d);
+  }
+
+  // replays and the passes after them
+  struct GramSteps {
+    size_t replays = 0, passes = 0;   // places in the pack
+    unsigned grid = 1;
+  };
+  GramSteps gram_pack(Pack& pk, const std::vector<SvdRequest*>& in,
+                      std::vector<GramSvdArgs> gs, bool first) {
+    GramSteps st;
+    std::vector<GramReplayArgs> reps;
+    for (size_t i = 0; i < in.size(); ++i) {
+      gs[i].expect = kGramRotated;
+      reps.push_back(in[i]->ws->replay_args(gs[i], first));
+      st.grid = std::max(st.grid, Workspace::replay_grid(gs[i].n, gs[i].r));
+    }
+    st.replays = pk.add(reps.data(), reps.size() * sizeof(GramReplayArgs));
+    st.passes = pk.add(gs.data(), gs.size() * sizeof(GramSvdArgs));
+    return st;
+  }
+  void gram_step(const GramSteps& st, const std::vector<GramSvdArgs>& gs, char* base) {
+    gram_replay_batch_kernel<<<dim3(st.grid, (unsigned)gs.size()), 256, 0, stream>>>(
+        reinterpret_cast<const GramReplayArgs*>(base + st.replays));
+    gram_launch(gs, base + st.passes);
   }
 
   // Y of at most kGramMaxRank columns: as run_small, after run_qr
   void run_gram(std::vector<SvdRequest*>& rs, std::vector<SvdRequest*>* blocked) {
     ensure_gather(rs.size());
     std::vector<GramSvdArgs> args;
-    std::vector<GramReplayArgs> reps;
     std::vector<SvdRequest*> in;
-    size_t lds = 0;
-    unsigned gx = 1;
     for (auto* r : rs) {
       try {
         args.push_back(r->ws->gram_prepare(r->jm, r->jn, infos_d + in.size()));
-        reps.push_back(r->ws->replay_args(r->jm, args.back().logc, args.back().logs));
-        lds = std::max(lds, Workspace::gram_lds(r->jn));
-        gx = std::max(gx, Workspace::replay_grid(r->jm, r->jn));
         in.push_back(r);
       } catch (...) {
         fail(r);
@@ -1544,28 +1600,44 @@ struct Batcher {
     if (in.empty()) return;
     Pack pk;
     const size_t oa = pk.add(args.data(), args.size() * sizeof(GramSvdArgs));
-    const size_t orp = pk.add(reps.data(), reps.size() * sizeof(GramReplayArgs));
+    const GramSteps steps = gram_pack(pk, in, args, true);
     char* base = upload(pk);
     HIP_CHECK(hipEventRecord(ev0, stream));
-    gram_svd_batch_kernel<<<(unsigned)in.size(), kGramThreads, lds, stream>>>(
-        reinterpret_cast<const GramSvdArgs*>(base + oa));
-    gram_replay_batch_kernel<<<dim3(gx, (unsigned)in.size()), 256, 0, stream>>>(
-        reinterpret_cast<const GramReplayArgs*>(base + orp));
-    gather(in, [](SvdRequest* r, float ms) {
+    gram_launch(args, base + oa);
+    gram_step(steps, args, base);
+    gather(in, args, [](SvdRequest* r, float ms) {
       return r->ws->jacobi_check(r->jm, r->jn, ms, true);
-    }, [&](SvdRequest* r) { blocked->push_back(r); });
+    }, [&](SvdRequest* r) {
+      r->ws->gram_rebuild();
+      blocked->push_back(r);
+    });
   }
 
-  // after the launches of run_small / run_gram: summaries to the host, then
-  // `finish` per request, or `retry` where the Gram Jacobi did not converge
+  // after the launches of run_small / run_gram: summaries to the host, further
+  // passes of the requests whose check rotated, then `finish` per request, or
+  // `retry` where the Gram Jacobi did not converge
   template <class Finish, class Retry>
-  void gather(std::vector<SvdRequest*>& in, Finish finish, Retry retry) {
-    HIP_CHECK(hipEventRecord(ev1, stream));
-    HIP_CHECK(hipGetLastError());
+  void gather(const std::vector<SvdRequest*>& in, const std::vector<GramSvdArgs>& gs,
+              Finish finish, Retry retry) {
     n_launches += 1;
-    HIP_CHECK(hipMemcpyAsync(infos_h, infos_d, in.size() * sizeof(SvdInfo),
-                             hipMemcpyDeviceToHost, stream));
-    HIP_CHECK(hipStreamSynchronize(stream));
+    for (int pass = 2;; ++pass) {
+      HIP_CHECK(hipEventRecord(ev1, stream));
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipMemcpyAsync(infos_h, infos_d, in.size() * sizeof(SvdInfo),
+                               hipMemcpyDeviceToHost, stream));
+      HIP_CHECK(hipStreamSynchronize(stream));
+      std::vector<SvdRequest*> more;
+      std::vector<GramSvdArgs> more_gs;
+      for (size_t i = 0; i < in.size(); ++i)
+        if (infos_h[i].state == kGramRotated) {
+          more.push_back(in[i]);
+          more_gs.push_back(gs[i]);
+        }
+      if (more.empty() || pass == kGramMaxPasses) break;
+      Pack pk;
+      const GramSteps steps = gram_pack(pk, more, more_gs, false);
+      gram_step(steps, more_gs, upload(pk));
+    }
     float ms = 0.f;
     HIP_CHECK(hipEventElapsedTime(&ms, ev0, ev1));
     jac_ms_total += ms;
@@ -1573,7 +1645,7 @@ struct Batcher {
       SvdRequest* r = in[i];
       try {
         *r->ws->info_h = infos_h[i];
-        if (infos_h[i].sweeps < 0) retry(r);
+        if (infos_h[i].state != kGramDone) retry(r);
         else r->k = finish(r, ms);
       } catch (...) {
         fail(r);

@@ -37,7 +37,15 @@ struct SvdInfo {
   double s0;       // largest singular value
   double discarded;  // 2-norm of the discarded singular values
   int rounds;      // rotation rounds logged (Gram Jacobi)
-  int unused;
+  int state;       // of a Gram Jacobi (see GramState)
+};
+
+// States of a Gram Jacobi (gram_svd_kernel). While it is not done, SvdInfo's
+// `sweeps` counts the sweeps so far and `pad` is the rank.
+enum GramState {
+  kGramDone = 0,      // a freshly formed Gram matrix needed no rotation
+  kGramFresh = 1,     // Y is there, no pass was made
+  kGramRotated = 2    // a pass rotated: its log is to be replayed, then checked
 };
 
 struct JacobiArgs {
@@ -129,8 +137,8 @@ struct RhArgs {
 
 // One small truncated SVD (small_svd_kernel): the pivoted QR's outputs
 // (reflectors in A, tau, vscale, beta, piv, *qrank), Y = R^H in Y (n x r,
-// ld n), sigma, perm, sorted, info (info->pad = r) and the rotation log, from
-// which gram_replay_kernel forms Z = Y W in Y and W.
+// ld n), info (info->pad = r) and, of ranks up to kGramSmallRank, the first
+// pass of the Gram Jacobi with its rotation log.
 struct SmallSvdArgs {
   double2* A; int m, n;
   double2* tau; double2* vscale; double* beta; int* piv; int* qrank;
@@ -144,13 +152,15 @@ struct SmallSvdArgs {
   double* logc; double2* logs;
 };
 
-// Jacobi SVD of Y = R^H (n x r, ld n) of a pivoted QR on its Gram matrix, in
-// one workgroup (gram_svd_kernel): sigma, perm, sorted, info and the rotation
-// log (64 rotations per round). With `pending`, r is an upper bound: the rank
-// is info->pad, and there is nothing to do unless info->sweeps is 0.
+// One pass of the Jacobi SVD of Y (n x r, ld n; R^H of a pivoted QR, or that
+// times the rotations so far) on its Gram matrix, in one workgroup
+// (gram_svd_kernel): the rotation log (64 rotations per round), or, where none is
+// needed, sigma, perm, sorted and the final info. With `expect` (a GramState),
+// r is an upper bound: the rank is info->pad, and there is nothing to do unless
+// info->state is `expect`.
 struct GramSvdArgs {
   const double2* Y; int n, r;
-  int pending;
+  int expect;               // 0: the first pass, of rank r
   double* sigma; int* perm; double* sorted; SvdInfo* info;
   double epsrel; int max_rank; int max_sweeps;
   SvdInfo* copy;
@@ -158,17 +168,20 @@ struct GramSvdArgs {
   double* logc; double2* logs;
 };
 
-// Z = Y W in place and W (r x r, ld r, r = info->pad) from the rotation log;
-// nothing when info->sweeps < 0.
+// Y <- Y J in place and W <- W J (r x r, ld r, r = info->pad) with the rotations J
+// of the last pass from its log; `first` sets W = J (also where no rotation was
+// needed). Else nothing unless info->state is kGramRotated.
 struct GramReplayArgs {
   double2* Y; int n;
+  int first;
   double2* W;
   const SvdInfo* info;
   const double* logc; const double2* logs;
 };
 
 constexpr int kGramMaxRank = 126;           // G in LDS, two blocks of it per thread
-constexpr int kGramMaxSweeps = 20;          // sweeps the rotation log holds
+constexpr int kGramMaxSweeps = 20;          // sweeps of a pass, all in the rotation log
+constexpr int kGramMaxPasses = 6;           // passes, the last one rotating nothing
 constexpr int kSmallMaxCols = kGramMaxRank; // columns of M in small_svd_kernel
 constexpr int kSmallThreads = 512;          // its workgroup
 constexpr int kGramThreads = 1024;          // workgroup of gram_svd_kernel
@@ -196,7 +209,9 @@ __global__ void truncate_batch_kernel(const SvdPostArgs* pa, SvdInfo* out);
 __global__ void zero_items_kernel(const ZeroItem* items);
 __global__ void small_svd_kernel(SmallSvdArgs a);
 __global__ void small_svd_batch_kernel(const SmallSvdArgs* probs);
-__global__ void gram_svd_kernel(GramSvdArgs a);
+template <int NT>                           // kSmallThreads (ranks up to kGramSmallRank)
+__global__ void gram_svd_kernel(GramSvdArgs a);            // or kGramThreads
+template <int NT>
 __global__ void gram_svd_batch_kernel(const GramSvdArgs* probs);
 __global__ void gram_replay_kernel(GramReplayArgs a);
 __global__ void gram_replay_batch_kernel(const GramReplayArgs* probs);   // problem = blockIdx.y

@@ -2098,15 +2098,23 @@ build_rh_batch_kernel(const RhArgs* pa) {
 //
 // One-sided Jacobi rotates columns of Y, and of the accumulated W, and takes
 // three inner products of length n per pair and round to find each rotation.
-// Here the rotations are found on G = Y^H Y (computed once, on the FP64 matrix
+// Here a pass finds the rotations on G = Y^H Y (formed on the FP64 matrix
 // cores) by two-sided rotations in LDS: a pair's three entries are read, not
-// summed. The rows of R fall off with the pivots, G = D A D with D their norms
-// and A well conditioned, and Jacobi keeps the small entries of such a matrix
-// to high relative accuracy (Demmel and Veselic, 1992), so the singular values
-// are the square roots of the final diagonal and the rotations orthogonalise
-// Y itself to the stopping rule of jacobi_kernel; they are applied to the rows
-// of Y and of the identity afterwards, by as many wavefronts as there are rows
-// (gram_replay_kernel), from a log of every round's rotations.
+// summed. They are applied to the rows of Y and of W afterwards, by as many
+// wavefronts as there are rows (gram_replay_kernel), from a log of every round's
+// rotations. Then the next pass forms G anew, from the rotated Y. The SVD is done
+// when such a fresh G needs no rotation: that is the stopping rule of
+// jacobi_kernel on the inner products of Y's own columns, and the singular
+// values are their norms.
+//
+// The rows of R fall off with the pivots, G = D A D with D their norms. Where A
+// is well conditioned, Jacobi keeps the small entries of such a matrix to high
+// relative accuracy (Demmel and Veselic, 1992), and the second pass only checks.
+// A pivoted QR does not guarantee that: on Kahan's matrix of 100 columns (A of
+// condition 1e12) the roots of the first pass's diagonal are off by 2e-11 of the
+// largest. Its Y is nearly orthogonal all the same, so that one sweep of a second
+// pass settles the pairs that are left (2 to 7 of thousands, as of some matrices
+// with a flat spectrum), and its columns' norms are right to rounding.
 //
 // The order is the round-robin of P = ceil(r / 2) pairs: position 2q holds the
 // pair's first column a_q, position 2q + 1 its second, b_q; position 0 keeps
@@ -2124,7 +2132,7 @@ build_rh_batch_kernel(const RhArgs* pa) {
 // columns, with the packed triangle's indices computed every round, that
 // arithmetic alone took longer than the rotations: 1.5 us a round at r = 83.)
 // The padding column of an odd r is zero and stays so. A sweep starts with a
-// test of all pairs, so the last, idle sweep of the one-sided form is not run.
+// test of all pairs; a pass without a sweep is the check.
 // Rotation: (x_a, x_b) <- (c x_a - conj(s) x_b, s x_a + c x_b), s carrying the
 // phase of g_ab.
 // Bound by the chain of a round in one compute unit: LDS reads, about 60
@@ -2194,11 +2202,12 @@ __device__ __forceinline__ void gram_store(double2* G, int r, int t, const doubl
 }
 
 // Two-sided Jacobi sweeps on G (rank r) in LDS; rc, rs: LDS scratch of 64
-// rotations; NB: blocks per thread, at least T / NT. Returns the sweeps done.
+// rotations; NB: blocks per thread, at least T / NT. Returns the sweeps done: none if no
+// pair needs a rotation, max_sweeps also where some pair still does.
 template <int NT, int NB>
 __device__ __forceinline__ int gram_jacobi(double2* G, int r, double tol2, double abs_tol2,
                                            int max_sweeps, double* rc, double2* rs,
-                                           double* logc, double2* logs, bool& converged) {
+                                           double* logc, double2* logs) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int P = (r + 1) / 2, L = 2 * P - 1;
   const int T = P * (P + 1) / 2;
@@ -2233,7 +2242,6 @@ __device__ __forceinline__ int gram_jacobi(double2* G, int r, double tol2, doubl
                            __double2loint(v.y));
     G[(place >> 16) & 0x7fffu] = v;
   };
-  converged = false;
   int sweeps = 0;
   for (;;) {
     int mine = 0;
@@ -2251,11 +2259,7 @@ __device__ __forceinline__ int gram_jacobi(double2* G, int r, double tol2, doubl
       }
       if (any) mine = 1;
     }
-    if (!__syncthreads_or(mine)) {
-      converged = true;
-      break;
-    }
-    if (sweeps == max_sweeps) break;
+    if (!__syncthreads_or(mine) || sweeps == max_sweeps) break;
     for (int t = 0; t < L; ++t) {
       double2 b00[NB], b01[NB], b10[NB], b11[NB];
 #pragma unroll
@@ -2357,8 +2361,7 @@ __device__ __host__ constexpr int gram_entries(int r) {
 // thread of wavefront 0).
 template <int NT>
 __device__ __forceinline__ void gram_finish(const double2* G, int r, double epsrel,
-                                            int max_rank, double extra2, int sweeps,
-                                            int rounds, bool converged, int half,
+                                            int max_rank, double extra2, int sweeps, int half,
                                             double* s_sig,
                                             double* s_sorted, double* s_tail, double* sigma,
                                             int* perm, double* sorted, SvdInfo* info,
@@ -2411,22 +2414,22 @@ __device__ __forceinline__ void gram_finish(const double2* G, int r, double epsr
     SvdInfo inf;
     inf.rank = k;
     inf.overflow = k > max_rank ? 1 : 0;
-    inf.sweeps = converged ? sweeps + 1 : -1;
+    inf.sweeps = sweeps + 1;
     inf.pad = r;
     inf.s0 = s0;
     inf.discarded = sqrt(k < r ? s_tail[k] : extra2);
-    inf.rounds = rounds;
-    inf.unused = 0;
+    inf.rounds = 0;
+    inf.state = kGramDone;
     *info = inf;
     if (copy) *copy = inf;
   }
 }
 
-// Rest of the SVD after the Gram matrix: the whole workgroup of NT threads, NB
-// blocks of G per thread at most.
+// Rest of a pass after the Gram matrix, `before` sweeps after the start: the
+// whole workgroup of NT threads, NB blocks of G per thread at most.
 template <int NT, int NB, class Args>
 __device__ __forceinline__ void gram_run(const Args& a, double2* G, int n, int r,
-                                         double extra2) {
+                                         double extra2, int before) {
   double2* rs = G + gram_entries(r);
   double* rc = reinterpret_cast<double*>(rs + 64);
   double* s_sig = rc + 64;
@@ -2434,47 +2437,68 @@ __device__ __forceinline__ void gram_run(const Args& a, double2* G, int n, int r
   const double tr = gram_scale<NT>(G, r, &half);
   const double eps = 2.220446049250313e-16;
   const double tol = (n > 16 ? n : 16) * eps;
-  bool converged = false;
   const int sweeps = gram_jacobi<NT, NB>(G, r, tol * tol, eps * eps * tr, a.max_sweeps, rc, rs,
-                                         a.logc, a.logs, converged);
-  gram_finish<NT>(G, r, a.epsrel, a.max_rank, extra2, sweeps,
-                  sweeps * (max(2, r + (r & 1)) - 1), converged, half, s_sig, s_sig + r,
+                                         a.logc, a.logs);
+  if (sweeps > 0) {
+    if (threadIdx.x == 0) {
+      SvdInfo inf = {};
+      inf.sweeps = before + sweeps;
+      inf.pad = r;
+      inf.rounds = sweeps * (max(2, r + (r & 1)) - 1);
+      inf.state = kGramRotated;
+      *a.info = inf;
+      if (a.copy) *a.copy = inf;
+    }
+    return;
+  }
+  gram_finish<NT>(G, r, a.epsrel, a.max_rank, extra2, before, half, s_sig, s_sig + r,
                   s_sig + 2 * r, a.sigma, a.perm, a.sorted, a.info, a.copy);
 }
 
-// 1024 threads: at ranks above kGramSmallRank the rotations' FP64 issue and the
-// LDS traffic of G set the time of a round, not its barriers (112: 1.35 us a
+// 1024 threads at ranks above kGramSmallRank: there the rotations' FP64 issue and
+// the LDS traffic of G set the time of a round, not its barriers (112: 1.35 us a
 // round, 1.7 us with 512 threads; 74: 0.92 us and 0.96; 35: 0.68 us and 0.64).
+template <int NT>
 __device__ __forceinline__ void gram_svd_body(const GramSvdArgs& a) {
   extern __shared__ double2 lds_gram[];
-  // the rank and the matrix of the one-workgroup QR, if that left them here
-  if (a.info->sweeps != 0 && a.pending) return;
-  const int r = __builtin_amdgcn_readfirstlane(a.pending ? a.info->pad : a.r);
+  int rank = a.r, before = 0;
+  if (a.expect) {
+    const SvdInfo inf = *a.info;
+    if (inf.state != a.expect) return;
+    rank = inf.pad;
+    before = inf.sweeps;
+  }
+  const int r = __builtin_amdgcn_readfirstlane(rank);
   double2* G = lds_gram;
-  for (int e = threadIdx.x; e < gram_entries(r); e += kGramThreads)
-    G[e] = make_double2(0.0, 0.0);
+  for (int e = threadIdx.x; e < gram_entries(r); e += NT) G[e] = make_double2(0.0, 0.0);
   __syncthreads();
   const int nb = (r + 15) / 16;
-  for (int t = threadIdx.x >> 6; t < nb * (nb + 1) / 2; t += kGramThreads / 64) {
+  for (int t = threadIdx.x >> 6; t < nb * (nb + 1) / 2; t += NT / 64) {
     double2 g[4];
     gram_tile(a.Y, a.n, a.n, r, t, g);
     gram_store(G, r, t, g);
   }
   __syncthreads();
-  // 2016 blocks at rank 126
-  gram_run<kGramThreads, 2>(a, G, a.n, r, a.extra2 ? *a.extra2 : 0.0);
+  // 990 blocks at rank 88, 2016 at rank 126
+  gram_run<NT, 2>(a, G, a.n, r, a.extra2 ? *a.extra2 : 0.0, before);
 }
 
-__global__ void __launch_bounds__(kGramThreads)
+template <int NT>
+__global__ void __launch_bounds__(NT)
 gram_svd_kernel(GramSvdArgs a) {
-  gram_svd_body(a);
+  gram_svd_body<NT>(a);
 }
+template __global__ void gram_svd_kernel<kSmallThreads>(GramSvdArgs);
+template __global__ void gram_svd_kernel<kGramThreads>(GramSvdArgs);
 
-__global__ void __launch_bounds__(kGramThreads)
+template <int NT>
+__global__ void __launch_bounds__(NT)
 gram_svd_batch_kernel(const GramSvdArgs* probs) {
   const GramSvdArgs a = probs[blockIdx.x];
-  gram_svd_body(a);
+  gram_svd_body<NT>(a);
 }
+template __global__ void gram_svd_batch_kernel<kSmallThreads>(const GramSvdArgs*);
+template __global__ void gram_svd_batch_kernel<kGramThreads>(const GramSvdArgs*);
 
 // wavefront shifts by one lane: lane i reads lane i + 1 (down) or i - 1 (up)
 constexpr int kDppWaveShl1 = 0x130, kDppWaveShr1 = 0x138;
@@ -2483,8 +2507,8 @@ __device__ __forceinline__ double2 dpp_d2(double2 v) {
   return make_double2(dpp_d<CTRL>(v.x), dpp_d<CTRL>(v.y));
 }
 
-// Applies the logged rotations to the rows of Y (in place: Z = Y W) and of
-// the identity (W, r x r), one wavefront per row. Lane q holds the entries of
+// Applies the logged rotations to the rows of Y (in place) and of W (r x r, the
+// identity in the first pass), one wavefront per row. Lane q holds the entries of
 // the row in columns a_q and b_q; going to the next round of the round-robin
 // moves every a one lane down and every b one lane up (a_0 stays, b of the
 // last lane turns into its a, a_1 into b_0), so that a round is 12 FMAs and
@@ -2494,7 +2518,8 @@ __device__ __forceinline__ double2 dpp_d2(double2 v) {
 __device__ __forceinline__ void gram_replay_body(const GramReplayArgs& a, int row) {
   const SvdInfo inf = *a.info;
   const int r = inf.pad, n = a.n;
-  if (inf.sweeps < 0 || r < 1 || row >= n + r) return;
+  if (inf.state != kGramRotated && !(a.first && inf.state == kGramDone)) return;
+  if (r < 1 || row >= n + r) return;
   const int lane = threadIdx.x & 63;
   const int re = max(2, r + (r & 1)), P = re / 2, L = re - 1;
   const double2 zero = make_double2(0.0, 0.0);
@@ -2505,9 +2530,12 @@ __device__ __forceinline__ void gram_replay_body(const GramReplayArgs& a, int ro
   if (isy) {
     if (oa) xa = a.Y[row + (long)ca * n];
     if (ob) xb = a.Y[row + (long)cb * n];
-  } else {
+  } else if (a.first) {
     if (oa && ca == row - n) xa.x = 1.0;
     if (ob && cb == row - n) xb.x = 1.0;
+  } else {
+    if (oa) xa = a.W[row - n + (long)ca * r];
+    if (ob) xb = a.W[row - n + (long)cb * r];
   }
   const int rounds = inf.rounds;
   const int le = min(lane, P - 1);
@@ -2830,7 +2858,7 @@ __device__ __forceinline__ void small_svd_body(const SmallSvdArgs& a) {
       SvdInfo inf;
       inf.rank = 0; inf.overflow = 0; inf.sweeps = 1; inf.pad = 0;
       inf.s0 = 0.0; inf.discarded = 0.0;
-      inf.rounds = 0; inf.unused = 0;
+      inf.rounds = 0; inf.state = kGramDone;
       *a.info = inf;
       if (a.copy) *a.copy = inf;
     }
@@ -2853,6 +2881,7 @@ __device__ __forceinline__ void small_svd_body(const SmallSvdArgs& a) {
     if (tid == 0) {
       a.info->sweeps = 0;
       a.info->pad = r;
+      a.info->state = kGramFresh;
     }
     return;
   }
@@ -2885,8 +2914,8 @@ __device__ __forceinline__ void small_svd_body(const SmallSvdArgs& a) {
   }
   __syncthreads();
   // one block per thread up to rank 62 (496 blocks), two at 88 (990)
-  if (r <= 62) gram_run<NT, 1>(a, Gm, n, r, folded2);
-  else gram_run<NT, 2>(a, Gm, n, r, folded2);
+  if (r <= 62) gram_run<NT, 1>(a, Gm, n, r, folded2, 0);
+  else gram_run<NT, 2>(a, Gm, n, r, folded2, 0);
   PHASE(14);
 }
 
