@@ -1633,13 +1633,12 @@ __device__ __forceinline__ void qrcp_reduce(const QrcpCand* cand, int nblk, int 
   double sv = 0.0;
   unsigned key = 0, col = 0xfffffu;
   if ((int)threadIdx.x < nblk) {
-    // both words in one 16-byte load (each has its own tag)
-    const __amdgpu_buffer_rsrc_t rs = agent_rsrc(cand, (unsigned)nblk * 16u);
+    // atomic loads (each word has its own tag): the compiler may take a buffer load
+    // out of the loop
     unsigned long long w0, w1;
     for (;;) {
-      const double2 v = ld_agent16(rs, threadIdx.x * 16u);
-      w0 = (unsigned long long)__double_as_longlong(v.x);
-      w1 = (unsigned long long)__double_as_longlong(v.y);
+      w0 = ld_agent(&cand[threadIdx.x].w0);
+      w1 = ld_agent(&cand[threadIdx.x].w1);
       if ((w0 & kQrTagMask) == tag && (w1 & kQrTagMask) == tag) break;
       __builtin_amdgcn_s_sleep(1);
     }
