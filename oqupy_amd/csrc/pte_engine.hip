@@ -309,7 +309,8 @@ struct Workspace {
   int* qr_piv = nullptr;
   int* qr_done = nullptr;
   size_t qr_cap = 0;
-  QrcpCand* qr_cand = nullptr;
+  unsigned long long* qr_cand = nullptr;   // posts (kQrCandWords)
+  static constexpr size_t kQrCandWords = 2 * kQrPostWords * 256;
   int* qr_rank_d = nullptr;
   int* qr_rank_h = nullptr;
   int qr_m = 0, qr_n = 0, qr_r = 0;
@@ -419,14 +420,14 @@ struct Workspace {
     const size_t at_flags = parts.add(sizeof(int) * max_sweeps);
     const size_t at_fro2 = parts.add(sizeof(double));
     const size_t at_info = parts.add(sizeof(SvdInfo));
-    const size_t at_cand = parts.add(sizeof(QrcpCand) * 2 * 256);
+    const size_t at_cand = parts.add(sizeof(unsigned long long) * kQrCandWords);
     const size_t at_rank = parts.add(sizeof(int));
     HIP_CHECK(hipMalloc((void**)&fixed_d, parts.size));
     bar = reinterpret_cast<unsigned*>(fixed_d + at_bar);
     flags = reinterpret_cast<int*>(fixed_d + at_flags);
     fro2 = reinterpret_cast<double*>(fixed_d + at_fro2);
     info_d = reinterpret_cast<SvdInfo*>(fixed_d + at_info);
-    qr_cand = reinterpret_cast<QrcpCand*>(fixed_d + at_cand);
+    qr_cand = reinterpret_cast<unsigned long long*>(fixed_d + at_cand);
     qr_rank_d = reinterpret_cast<int*>(fixed_d + at_rank);
     Parts host;
     const size_t at_hinfo = host.add(sizeof(SvdInfo));
@@ -507,7 +508,8 @@ struct Workspace {
     flags = reinterpret_cast<int*>(take(sizeof(int) * max_sweeps));
     fro2 = reinterpret_cast<double*>(take(sizeof(double)));
     info_d = reinterpret_cast<SvdInfo*>(take(sizeof(SvdInfo)));
-    qr_cand = reinterpret_cast<QrcpCand*>(take(sizeof(QrcpCand) * 2 * 256));
+    qr_cand = reinterpret_cast<unsigned long long*>(
+        take(sizeof(unsigned long long) * kQrCandWords));
     qr_rank_d = reinterpret_cast<int*>(take(sizeof(int)));
     qr_tau = reinterpret_cast<double2*>(take(sizeof(double2) * big));
     qr_vscale = reinterpret_cast<double2*>(take(sizeof(double2) * big));
@@ -900,6 +902,10 @@ struct Workspace {
     return k;
   }
 
+  static size_t qr_cand_bytes(int nblk) {
+    return sizeof(unsigned long long) * 2 * kQrPostWords * nblk;
+  }
+
   // one launch of the pivoted QR of Q (m x n): capped at *max_steps when
   // given, resumed after `start` steps when start > 0 (stop threshold
   // drop_abs2 on the squared residual). Returns the steps taken in total;
@@ -914,7 +920,7 @@ struct Workspace {
     qa.out = rank ? rank->out_d : nullptr;
     qa.mark_rel = rank ? rank->theta * epsrel : 0.0;
     qa.stop_at_mark = stop_at_mark ? 1 : 0;
-    HIP_CHECK(hipMemsetAsync(qr_cand, 0, sizeof(QrcpCand) * 2 * nblk, svd_stream));
+    HIP_CHECK(hipMemsetAsync(qr_cand, 0, qr_cand_bytes(nblk), svd_stream));
     void* kargs[] = {&qa};
     mark(evq0);
     HIP_CHECK(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(qrcp_kernel),
@@ -1680,7 +1686,7 @@ struct Batcher {
           const int g = alloc[i - ch.first];
           args.push_back(r->ws->qr_prepare(r->m, r->n, g));
           zeros.push_back(ZeroItem{reinterpret_cast<unsigned*>(r->ws->qr_cand),
-                                   (int)(2 * g * sizeof(QrcpCand) / sizeof(unsigned)), 0});
+                                   (int)(Workspace::qr_cand_bytes(g) / sizeof(unsigned)), 0});
           grids.push_back(g);
           in.push_back(r);
         } catch (...) {

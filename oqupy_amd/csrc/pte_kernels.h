@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "pte_post.h"
+
 namespace pte {
 
 enum NodeKind { NODE_DENSE = 0, NODE_DELTA = 1 };
@@ -81,19 +83,15 @@ struct EmitArgs {
   double2* dst;
 };
 
-// Pivoted QR of a column-major matrix (see qrcp_kernel): a workgroup's post of
-// one step (see qrcp_post).
-struct QrcpCand {
-  unsigned long long w0, w1;
-};
-
+// Pivoted QR of a column-major matrix (see qrcp_kernel).
 struct QrcpArgs {
   double2* A; int m, n; long lda;
   double drop;                // stop when the residual norm <= drop * ||A||_F
   double2* tau; double2* vscale; double* beta;
   int* piv;                   // [n] physical column of each step, then the rest
   int* done;                  // [n] scratch
-  QrcpCand* cand;             // [2 * gridDim.x] posts, zeroed before the launch
+  unsigned long long* cand;   // posts, zeroed before the launch: [2][gridDim.x][2] words
+                              // 0 and 1, then [2][gridDim.x] words 2
   int* rank;                  // steps taken
   const int* max_steps;       // optional cap on the steps (device int)
   double* out;                // optional: [0] squared residual norm at the stop,

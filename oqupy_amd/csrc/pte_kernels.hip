@@ -1576,7 +1576,7 @@ emit_kernel(EmitArgs a) {
 // step's reflector from the pivot column itself, so workgroups wait for each
 // other once per step: each posts its candidate (largest residual norm) and
 // every one waits for all posts of the step and reduces them identically.
-// A post is two 8-byte words that each carry the step's tag, so reading the
+// A post is of 8-byte words that each carry the step's tag, so reading the
 // posts is the waiting: no arrival counter stands between them (two dependent
 // atomics and a separate read of the candidates less). A step at 380 x 108 takes
 // 7.0 us on 27 workgroups (8.8 with the counters; 1.5 forming the reflector, 1.3
@@ -1591,17 +1591,10 @@ __device__ __forceinline__ void better(double& v, int& c, double ov, int oc) {
   if (oc >= 0 && (c < 0 || ov > v || (ov == v && oc < c))) { v = ov; c = oc; }
 }
 
-constexpr unsigned long long kQrTagMask = 0xfffull;
-__device__ __forceinline__ unsigned long long qrcp_tag(int j) {
-  return (unsigned long long)(1 + j % 4095);
-}
-
-// Posts the workgroup's candidate of step j: word 0 holds the upper word of the
-// largest residual norm, its column (20 bits; all ones: none) and the tag, word
-// 1 the sum of the squared residual norms with the tag in its lowest 12 bits.
-// Every wavefront waits for its own column stores first.
-__device__ __forceinline__ void qrcp_post(QrcpCand* dst, int j, double wmax, int wcol,
-                                          double wsum, double* cw_max, int* cw_col,
+// Posts the workgroup's candidate of step j (see QrcpPost; wcol: number of the
+// column among its own). Every wavefront waits for its own column stores first.
+__device__ __forceinline__ void qrcp_post(const QrcpArgs& a, int blk, int nblk, int j, double wmax,
+                                          int wcol, double wsum, double* cw_max, int* cw_col,
                                           double* cw_sum) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (lane == 0) { cw_max[wave] = wmax; cw_col[wave] = wcol; cw_sum[wave] = wsum; }
@@ -1614,55 +1607,94 @@ __device__ __forceinline__ void qrcp_post(QrcpCand* dst, int j, double wmax, int
       sm += cw_sum[w];
       better(v, c, cw_max[w], cw_col[w]);
     }
+    QrcpPost post;
+    post.norm = c >= 0 ? (unsigned long long)__double_as_longlong(v) : 0ull;
+    post.sum = (unsigned long long)__double_as_longlong(sm);
+    post.local = c >= 0 ? (unsigned)c : kQrNoColumn;
     const unsigned long long tag = qrcp_tag(j);
-    const unsigned long long key = c >= 0 ? (unsigned)__double2hiint(v) : 0u;
-    const unsigned long long col = c >= 0 ? (unsigned)c : 0xfffffu;
-    st_agent(&dst->w1, ((unsigned long long)__double_as_longlong(sm) & ~kQrTagMask) | tag);
-    st_agent(&dst->w0, (key << 32) | (col << 12) | tag);
+    const long at = (long)(j & 1) * nblk + blk;
+    st_agent(a.cand + 2 * at, qrcp_word(post, 0, tag));
+    st_agent(a.cand + 2 * at + 1, qrcp_word(post, 1, tag));
+    st_agent(a.cand + 4 * nblk + at, qrcp_word(post, 2, tag));
   }
 }
 
 // Waits for the posts of step j and reduces them: the column of the largest
-// norm (by the upper word, ties to the smaller column; -1: none) and the
-// residual total, the same bits in every thread of the grid.
-__device__ __forceinline__ void qrcp_reduce(const QrcpCand* cand, int nblk, int j,
+// norm (ties to the smaller column; -1: none) and the residual total, the same
+// bits in every thread of the grid. The waits poll by atomic loads (the compiler
+// may take a buffer load out of the loop).
+__device__ __forceinline__ void qrcp_reduce(const QrcpArgs& a, int nblk, int j,
                                             double (*slot)[4], unsigned (*slotk)[4],
-                                            unsigned (*slotc)[4], int& parity, int* bestc,
-                                            double* total) {
+                                            unsigned (*slotc)[4], int (*slotn)[4], int& parity,
+                                            int* bestc, double* total) {
   const unsigned long long tag = qrcp_tag(j);
-  double sv = 0.0;
-  unsigned key = 0, col = 0xfffffu;
+  const long at = (long)(j & 1) * nblk + threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr unsigned kNone = ~0u;
+  // a workgroup without columns left has norm 0
+  QrcpPost post{0ull, 0ull, kQrNoColumn};
   if ((int)threadIdx.x < nblk) {
-    // atomic loads (each word has its own tag): the compiler may take a buffer load
-    // out of the loop
     unsigned long long w0, w1;
     for (;;) {
-      w0 = ld_agent(&cand[threadIdx.x].w0);
-      w1 = ld_agent(&cand[threadIdx.x].w1);
-      if ((w0 & kQrTagMask) == tag && (w1 & kQrTagMask) == tag) break;
+      w0 = ld_agent(a.cand + 2 * at);
+      w1 = ld_agent(a.cand + 2 * at + 1);
+      if (qrcp_tagged(w0, tag) && qrcp_tagged(w1, tag)) break;
       __builtin_amdgcn_s_sleep(1);
     }
-    key = (unsigned)(w0 >> 32);
-    col = (unsigned)(w0 >> 12) & 0xfffffu;
-    sv = __longlong_as_double((long long)(w1 & ~kQrTagMask));
+    post = qrcp_unpack(w0, w1);
   }
-  // a workgroup without columns left has key 0 and the largest column number
+  const unsigned key = (unsigned)(post.norm >> 32);
+  const unsigned col = post.local == kQrNoColumn ? kNone : threadIdx.x + post.local * nblk;
   const unsigned wkey = wave_max(key);
-  const unsigned wcol = wave_min(key == wkey ? col : 0xfffffu);
-  if ((threadIdx.x & 63) == 0) {
-    slotk[parity][threadIdx.x >> 6] = wkey;
-    slotc[parity][threadIdx.x >> 6] = wcol;
+  const unsigned wcol = wave_min(key == wkey ? col : kNone);
+  const int tied = __popcll(__ballot(key == wkey && col != kNone));
+  if (lane == 0) {
+    slotk[parity][wave] = wkey;
+    slotc[parity][wave] = wcol;
+    slotn[parity][wave] = tied;
   }
   // block_sum256 synchronises before reading, which also publishes the slots
-  *total = block_sum256(sv, slot, parity);
+  *total = block_sum256(__longlong_as_double((long long)post.sum), slot, parity);
   const int par = parity ^ 1;
-  unsigned k = slotk[par][0], c = slotc[par][0];
+  unsigned k = 0, c = kNone;
+  int count = 0;
 #pragma unroll
-  for (int w = 1; w < 4; ++w) {
+  for (int w = 0; w < 4; ++w) {
     const unsigned ok = slotk[par][w], oc = slotc[par][w];
-    if (ok > k || (ok == k && oc < c)) { k = ok; c = oc; }
+    const int on = slotn[par][w];
+    if (on > 0 && (count == 0 || ok > k)) { k = ok; c = oc; count = on; }
+    else if (on > 0 && ok == k) { c = min(c, oc); count += on; }
   }
-  *bestc = __builtin_amdgcn_readfirstlane(c == 0xfffffu ? -1 : (int)c);
+  if (__builtin_amdgcn_readfirstlane(count) > 1) {
+    // upper halves tie: the lower ones of the tied workgroups
+    unsigned low = 0;
+    const bool mine = key == k && col != kNone;
+    if (mine) {
+      unsigned long long w2;
+      for (;;) {
+        w2 = ld_agent(a.cand + 4 * nblk + at);
+        if (qrcp_tagged(w2, tag)) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+      low = qrcp_norm_low(w2);
+    }
+    const unsigned wlow = wave_max(low);
+    const unsigned wc = wave_min(mine && low == wlow ? col : kNone);
+    __syncthreads();   // the slots above are read
+    if (lane == 0) {
+      slotk[par][wave] = wlow;
+      slotc[par][wave] = wc;
+    }
+    __syncthreads();
+    k = 0;
+    c = kNone;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const unsigned ok = slotk[par][w], oc = slotc[par][w];
+      if (oc != kNone && (c == kNone || ok > k || (ok == k && oc < c))) { k = ok; c = oc; }
+    }
+  }
+  *bestc = __builtin_amdgcn_readfirstlane((int)c);
 }
 
 // loads of the pivoted QR issued together (per thread), and the rows of a
@@ -1675,6 +1707,7 @@ __device__ __forceinline__ void qrcp_body(const QrcpArgs& a, const int blk, cons
   extern __shared__ double2 vcol[];            // reflector of the step (m)
   __shared__ double slot[2][4];
   __shared__ unsigned slotk[2][4], slotc[2][4];
+  __shared__ int slotn[2][4];
   __shared__ double vn1[kQrcpMaxLocal], vn2[kQrcpMaxLocal];
   __shared__ int done[kQrcpMaxLocal];
   __shared__ double cw_max[4], cw_sum[4];
@@ -1736,12 +1769,12 @@ __device__ __forceinline__ void qrcp_body(const QrcpArgs& a, const int blk, cons
       if (j0 == 0) st_agent(a.done + c, 0);
     }
     wsum += nrm * nrm;
-    better(wmax, wcol, nrm, c);
+    better(wmax, wcol, nrm, q);   // (the workgroup's columns ascend with q)
   }
-  qrcp_post(a.cand + (j0 & 1) * nblk + blk, j0, wmax, wcol, wsum, cw_max, cw_col, cw_sum);
+  qrcp_post(a, blk, nblk, j0, wmax, wcol, wsum, cw_max, cw_col, cw_sum);
   double total;
   int p;
-  qrcp_reduce(a.cand + (j0 & 1) * nblk, nblk, j0, slot, slotk, slotc, parity, &p, &total);
+  qrcp_reduce(a, nblk, j0, slot, slotk, slotc, slotn, parity, &p, &total);
   const double total0 = total;
   const double drop2 = j0 > 0 ? a.drop_abs2 : a.drop * a.drop * total;
   const double tol3z = 1.4901161193847656e-08;   // sqrt(eps), zlaqp2
@@ -1919,7 +1952,7 @@ __device__ __forceinline__ void qrcp_body(const QrcpArgs& a, const int blk, cons
           }
         }
         wsum += nv * nv;
-        better(wmax, wcol, nv, c);
+        better(wmax, wcol, nv, q);
         continue;
       }
       // rows j .. j + 64 kQrCache - 1 stay in registers between the dot
@@ -2006,13 +2039,13 @@ __device__ __forceinline__ void qrcp_body(const QrcpArgs& a, const int blk, cons
         }
       }
       wsum += nv * nv;
-      better(wmax, wcol, nv, c);
+      better(wmax, wcol, nv, q);
     }
     PHASE(9);
     ++j;
-    qrcp_post(a.cand + (j & 1) * nblk + blk, j, wmax, wcol, wsum, cw_max, cw_col, cw_sum);
+    qrcp_post(a, blk, nblk, j, wmax, wcol, wsum, cw_max, cw_col, cw_sum);
     PHASE(10);
-    qrcp_reduce(a.cand + (j & 1) * nblk, nblk, j, slot, slotk, slotc, parity, &p, &total);
+    qrcp_reduce(a, nblk, j, slot, slotk, slotc, slotn, parity, &p, &total);
     PHASE(12);
     if (a.mark_rel > 0.0) {
       if (j == 1) {
