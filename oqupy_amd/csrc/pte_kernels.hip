@@ -2632,8 +2632,7 @@ gram_replay_batch_kernel(const GramReplayArgs* probs) {
 // reflectors (zlarfg) and the eps-rank stop are qrcp_kernel's; the residual
 // norms are summed anew in every step (two FMAs a row, in place of the
 // downdate's square root and division and of a pass over the pivot column), and
-// the pivot is the first column whose squared norm has the largest upper word
-// (within 1e-6 of the largest). A step:
+// the pivot is the first column with the largest one. A step:
 //   (1) each group has the norm, first entry and reflector scalars of its
 //       remaining rows; each wavefront posts its largest column to LDS; barrier;
 //   (2) every wavefront picks the winner of the posts; the winner's group
@@ -2656,14 +2655,22 @@ gram_replay_batch_kernel(const GramReplayArgs* probs) {
 struct SmallCand {
   double2 tau, scale;
   double sum, beta;
-  unsigned key;      // upper word of the squared norm
+  double norm2;      // squared norm
   int col;
-  int pad[2];
+  int pad;
 };
 constexpr int kSmallWaves = kSmallThreads / 64;
 static_assert(kSmallWaves == 8, "the posts are reduced over groups of 8 lanes");
 static_assert(64 * kSmallRows * 16 + kSmallWaves * (int)sizeof(SmallCand) +
                   2 * 128 * (int)sizeof(int) <= (int)kSmallQrLds, "LDS of the QR");
+
+__device__ __forceinline__ double larger(double a, double b) { return b > a ? b : a; }
+template <int HALF>
+__device__ __forceinline__ double swap_larger(double v) {
+  double lo, hi;
+  swap_d<HALF>(v, lo, hi);
+  return larger(lo, hi);
+}
 
 // 1/x and 1/sqrt(x): refined estimates where they are safe, else the division
 __device__ __forceinline__ double rcp_safe(double x) {
@@ -2720,15 +2727,13 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
     group_sum4(tail, ax, ay, z, G);
     const double norm2 = alive ? tail + fma(ax, ax, ay * ay) : 0.0;
     // largest column of the wavefront: its norms are the same bits in all lanes
-    // of a group, so the first lane with the largest key is lane 0 of a group
-    unsigned key = (unsigned)__double2hiint(norm2);
-    const unsigned mykey = key;
-    double sv = norm2;
-    if (G <= 4) { key = max(key, (unsigned)dpp_i<kDppHalfMirror>((int)key)); sv += dpp_d<kDppHalfMirror>(sv); }
-    if (G <= 8) { key = max(key, (unsigned)dpp_i<kDppMirror>((int)key)); sv += dpp_d<kDppMirror>(sv); }
-    if (G <= 16) { key = swap_max<16>(key); sv = swap_sum<16>(sv); }
-    if (G <= 32) { key = swap_max<32>(key); sv = swap_sum<32>(sv); }
-    const unsigned long long at = __ballot(alive && mykey == key);
+    // of a group, so the first lane with the largest one is lane 0 of a group
+    double big = norm2, sv = norm2;
+    if (G <= 4) { big = larger(big, dpp_d<kDppHalfMirror>(big)); sv += dpp_d<kDppHalfMirror>(sv); }
+    if (G <= 8) { big = larger(big, dpp_d<kDppMirror>(big)); sv += dpp_d<kDppMirror>(sv); }
+    if (G <= 16) { big = swap_larger<16>(big); sv = swap_sum<16>(sv); }
+    if (G <= 32) { big = swap_larger<32>(big); sv = swap_sum<32>(sv); }
+    const unsigned long long at = __ballot(alive && norm2 == big);
     double beta = ax;
     double2 tau = make_double2(0.0, 0.0), scale = make_double2(0.0, 0.0);
     if (tail != 0.0 || ay != 0.0) {
@@ -2746,7 +2751,7 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
       cd->scale = scale;
       cd->sum = sv;
       cd->beta = beta;
-      cd->key = key;
+      cd->norm2 = big;
       cd->col = at ? myc : -1;
     }
   };
@@ -2762,16 +2767,15 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
     // wavefront, whose columns are the smaller ones
     const SmallCand* cl = cand + (lane & (kSmallWaves - 1));
     const int mcol = cl->col;
-    unsigned key = cl->key;
-    double total = cl->sum;
-    const unsigned mykey = key;
-    key = max(key, (unsigned)dpp_i<kDppXor1>((int)key));
+    const double wnorm2 = cl->norm2;
+    double total = cl->sum, big = wnorm2;
+    big = larger(big, dpp_d<kDppXor1>(big));
     total += dpp_d<kDppXor1>(total);
-    key = max(key, (unsigned)dpp_i<kDppXor2>((int)key));
+    big = larger(big, dpp_d<kDppXor2>(big));
     total += dpp_d<kDppXor2>(total);
-    key = max(key, (unsigned)dpp_i<kDppHalfMirror>((int)key));
+    big = larger(big, dpp_d<kDppHalfMirror>(big));
     total += dpp_d<kDppHalfMirror>(total);
-    const unsigned long long at = __ballot(mcol >= 0 && mykey == key);
+    const unsigned long long at = __ballot(mcol >= 0 && wnorm2 == big);
     const int ws = at ? __ffsll(at) - 1 : 0;          // wavefront of the winner
     const int p = at ? __builtin_amdgcn_readlane(mcol, ws) : -1;
     // residual test; an adaptive stop (stop_rel > 0) ends at a residual of

@@ -13,8 +13,9 @@ from oqupy_amd.backends import engine
 
 pytestmark = pytest.mark.gpu
 
-# the grid's QR, from two workgroups on
-SHAPES = [(2600, 8), (700, 30), (200, 100), (140, 130), (1100, 200)]
+# one workgroup with 64 to 4 lanes a column; the grid's QR from two workgroups on
+SHAPES = [(2, 2), (9, 8), (40, 16), (30, 32), (90, 64), (128, 126),
+          (2600, 8), (700, 30), (200, 100), (140, 130), (1100, 200)]
 
 
 @pytest.mark.parametrize("m,n", SHAPES)
