@@ -482,17 +482,12 @@ __device__ __forceinline__ bool needs_rotation(double app, double aqq, double ma
          mag2 > 0.0;
 }
 
-// 1/sqrt(x) and 1/x for normal positive x: the hardware estimates (measured
-// relative error 2^-24) refined by one cubic step to full double precision.
+// 1/sqrt(x) for normal positive x: the hardware estimate (measured relative
+// error 2^-24) refined by one cubic step to full double precision.
 __device__ __forceinline__ double rsqrt_nr(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-x * y, y, 1.0);
   return fma(y * e, fma(0.375, e, 0.5), y);
-}
-__device__ __forceinline__ double rcp_nr(double x) {
-  const double y = __builtin_amdgcn_rcp(x);
-  const double e = fma(-x, y, 1.0);
-  return fma(fma(e, e, e), y, y);
 }
 
 // Rotation of the 2 x 2 block [[app, apq], [conj(apq), aqq]]: with
@@ -2672,14 +2667,6 @@ __device__ __forceinline__ double swap_larger(double v) {
   return larger(lo, hi);
 }
 
-// 1/x and 1/sqrt(x): refined estimates where they are safe, else the division
-__device__ __forceinline__ double rcp_safe(double x) {
-  return (x > 1e-290 && x < 1e290) ? rcp_nr(x) : 1.0 / x;
-}
-__device__ __forceinline__ double rsqrt_safe(double x) {
-  return (x > 1e-290 && x < 1e290) ? rsqrt_nr(x) : 1.0 / sqrt(x);
-}
-
 template <int RP>
 __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, double2* vcol,
                                         SmallCand* cand, int* s_piv, int* s_done,
@@ -2737,13 +2724,11 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
     double beta = ax;
     double2 tau = make_double2(0.0, 0.0), scale = make_double2(0.0, 0.0);
     if (tail != 0.0 || ay != 0.0) {
-      const double inv = rsqrt_safe(norm2);
-      const double ib = -copysign(inv, ax);        // 1 / beta
-      beta = -copysign(norm2 * inv, ax);
+      beta = -copysign(sqrt(norm2), ax);
       const double dr = ax - beta;
-      const double id = rcp_safe(fma(dr, dr, ay * ay));
-      scale = make_double2(dr * id, -ay * id);
-      tau = make_double2(-dr * ib, -ay * ib);
+      const double den = fma(dr, dr, ay * ay);
+      scale = make_double2(dr / den, -ay / den);
+      tau = make_double2(-dr / beta, -ay / beta);
     }
     if (lane == (at ? __ffsll(at) - 1 : 0)) {
       SmallCand* cd = cand + wave;
