@@ -955,8 +955,9 @@ struct Workspace {
     const size_t y = (size_t)(n | 1) * r * 16;
     return std::max({kSmallQrLds, y <= kSmallLdsMax ? y : 0, gram_lds(r)});
   }
-  // M fits the registers of one workgroup: 2.8 us a step at 88 x 83 and 6.1 at
-  // 128 x 126, where qrcp_kernel takes 7 to 9 us, so the limit is what fits.
+  // M fits the registers of one workgroup (kSmallRows). At the limit the whole SVD
+  // takes 2.35 ms here at 152 x 126 (2.75 by qrcp_kernel at 153 rows), 0.76 at
+  // 304 x 64 (0.91 at 305), 0.32 at 608 x 32 (0.40) and 0.095 at 2432 x 8 (0.20).
   bool small_ok(int m, int n) const {
     return small_enabled && n <= kSmallMaxCols && m <= kSmallRows * small_lanes(n);
   }

@@ -184,7 +184,7 @@ constexpr int kSmallMaxCols = kGramMaxRank; // columns of M in small_svd_kernel
 constexpr int kSmallThreads = 512;          // its workgroup
 constexpr int kGramThreads = 1024;          // workgroup of gram_svd_kernel
 constexpr int kGramSmallRank = 88;          // ranks small_svd_kernel finishes itself
-constexpr int kSmallRows = 40;              // rows of M a lane holds at most
+constexpr int kSmallRows = 38;              // rows of M a lane holds at most (no scratch)
 constexpr size_t kSmallQrLds = 64 * kSmallRows * 16 + 2048;   // LDS of its QR
 // lanes per column of small_svd_kernel's QR
 __host__ __device__ constexpr int small_lanes(int n) {

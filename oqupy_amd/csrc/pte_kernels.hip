@@ -2652,7 +2652,11 @@ gram_replay_batch_kernel(const GramReplayArgs* probs) {
 // [u][64 lanes]. (Skipping the finished rows took 1550 instructions a step at
 // 12 rows a lane, two thirds of them branches, masks and register copies.) The
 // reflector is used unscaled, its scale (vscale, as in the factors of
-// qrcp_kernel) folded into the scalars.
+// qrcp_kernel) folded into the scalars. All of it fits 256 VGPRs up to 38 rows a
+// lane, with no scratch, as the reflector's rows are read eight at a time and the
+// scalars of the whole factorisation lie in LDS (with 40 rows, and a branch after
+// those reads, which let the compiler gather them all before it, 448 bytes a lane
+// were spilled and a step at 160 x 126 took 12 us).
 // 512 threads: a workgroup barrier costs 86 cycles with 8 wavefronts, 326 with
 // 16 and 11 with 4, and 256 threads would not hold M.
 // Bound by the chain of a step (two barriers, two passes through LDS, the
@@ -2669,7 +2673,8 @@ struct SmallCand {
 constexpr int kSmallWaves = kSmallThreads / 64;
 static_assert(kSmallWaves == 8, "the posts are reduced over groups of 8 lanes");
 static_assert(64 * kSmallRows * 16 + kSmallWaves * (int)sizeof(SmallCand) +
-                  2 * 128 * (int)sizeof(int) <= (int)kSmallQrLds, "LDS of the QR");
+                  2 * 128 * (int)sizeof(int) + 2 * (int)sizeof(double) <=
+                  (int)kSmallQrLds, "LDS of the QR");
 
 __device__ __forceinline__ double larger(double a, double b) { return b > a ? b : a; }
 template <int HALF>
@@ -2682,7 +2687,7 @@ __device__ __forceinline__ double swap_larger(double v) {
 template <int RP>
 __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, double2* vcol,
                                         SmallCand* cand, int* s_piv, int* s_done,
-                                        double& folded2) {
+                                        double* s_stop, double& folded2) {
   // up to 24 rows the reflector's rows stay in registers between the inner
   // product and the update, else they are read again
   constexpr bool kKeep = RP <= 24;
@@ -2692,7 +2697,6 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
   const double eps = 2.220446049250313e-16;
   const int kmax = min(m, n);
   bool alive = myc < n;
-  int myt = -1;                       // step at which the own column was pivoted
   double2 col[RP];
 #pragma unroll
   for (int u = 0; u < RP; ++u) {
@@ -2754,8 +2758,8 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
   };
   post(0);
   SEG_INIT();
-  double drop2 = 0.0, stop2 = -1.0;
-  folded2 = 0.0;
+  bool folded = false;
+  double total;
   int j = 0;
   for (;;) {
     __syncthreads();
@@ -2765,7 +2769,8 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
     const SmallCand* cl = cand + (lane & (kSmallWaves - 1));
     const int mcol = cl->col;
     const double wnorm2 = cl->norm2;
-    double total = cl->sum, big = wnorm2;
+    total = cl->sum;
+    double big = wnorm2;
     big = larger(big, dpp_d<kDppXor1>(big));
     total += dpp_d<kDppXor1>(total);
     big = larger(big, dpp_d<kDppXor2>(big));
@@ -2777,10 +2782,12 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
     const int p = at ? __builtin_amdgcn_readlane(mcol, ws) : -1;
     // residual test; an adaptive stop (stop_rel > 0) ends at a residual of
     // stop_rel * |beta_0| and counts it in the cut
-    if (j == 0) drop2 = eps * eps * total;
+    // (both thresholds are kept in LDS, from step 0 on)
+    const double drop2 = j == 0 ? eps * eps * total : s_stop[0];
     bool go = j < kmax && p >= 0 && total > drop2;
-    if (a.stop_rel > 0.0 && j >= 1 && total <= stop2) {
-      folded2 = (p >= 0 && j < kmax) ? total : 0.0;
+    folded = a.stop_rel > 0.0 && j >= 1 && total <= s_stop[1];
+    if (folded) {
+      folded = p >= 0 && j < kmax;
       go = false;
     }
     // (the same in every lane; said so, so that the loop, its step and all that
@@ -2788,15 +2795,17 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
     if (!__builtin_amdgcn_readfirstlane((int)go)) break;
     const SmallCand* cw = cand + ws;
     const double2 tau = cw->tau, scale = cw->scale;
-    if (j == 0) stop2 = (a.stop_rel * cw->beta) * (a.stop_rel * cw->beta);
+    if (j == 0 && tid == 0) {
+      s_stop[0] = drop2;
+      s_stop[1] = (a.stop_rel * cw->beta) * (a.stop_rel * cw->beta);
+    }
     if (alive && myc == p) {
 #pragma unroll
       for (int u = 0; u < RP; ++u) vcol[64 * u + g] = col[u];
       alive = false;
-      myt = j;
       if (g == 0) {
         s_piv[j] = p;
-        s_done[p] = 1;
+        s_done[p] = j + 1;
         a.tau[j] = tau;
         a.vscale[j] = scale;
         a.beta[j] = cw->beta;
@@ -2822,6 +2831,7 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
       const double2 tw = cmulc(tau, w);
       const double2 sv2 = cmul(scale, tw);
       SEG(3);
+      if (g == (j & (G - 1))) a.A[j + (long)myc * m] = csub(cj, tw);
       if (!kKeep) asm volatile("" ::: "memory");
 #pragma unroll
       for (int u = 0; u < RP; ++u) {
@@ -2831,15 +2841,16 @@ __device__ __forceinline__ int small_qr(const SmallSvdArgs& a, const int lg, dou
         cfma(col[u], make_double2(-v.x, -v.y), sv2);
         if (!kKeep && u % 8 == 7) __builtin_amdgcn_sched_barrier(0);
       }
-      if (g == (j & (G - 1))) a.A[j + (long)myc * m] = csub(cj, tw);
     }
     ++j;
     SEG(4);
     post(j);
     SEG(5);
   }
+  folded2 = folded ? total : 0.0;
   SEG_FLUSH(0, 6);
   // reflectors to global memory (apply_q_kernel reads them)
+  const int myt = myc < n ? s_done[myc] - 1 : -1;    // step that took the own column
   if (myt >= 0) {
     // (opaque copy: the indices and masks of the loads above would otherwise be
     // kept in registers through the loop for reuse here)
@@ -2874,16 +2885,17 @@ __device__ __forceinline__ void small_svd_body(const SmallSvdArgs& a) {
   SmallCand* cand = reinterpret_cast<SmallCand*>(vcol + 64 * kSmallRows);
   int* s_piv = reinterpret_cast<int*>(cand + kSmallWaves);
   int* s_done = s_piv + 128;
+  double* s_stop = reinterpret_cast<double*>(s_done + 128);
   PHASE_INIT();
   const int lg = __builtin_amdgcn_readfirstlane(31 - __clz(small_lanes(n)));
   const int rows = (m + (1 << lg) - 1) >> lg;
   double folded2;
-  const int steps = rows <= 4 ? small_qr<4>(a, lg, vcol, cand, s_piv, s_done, folded2)
-                : rows <= 8  ? small_qr<8>(a, lg, vcol, cand, s_piv, s_done, folded2)
-                : rows <= 16 ? small_qr<16>(a, lg, vcol, cand, s_piv, s_done, folded2)
-                : rows <= 24 ? small_qr<24>(a, lg, vcol, cand, s_piv, s_done, folded2)
-                : rows <= 32 ? small_qr<32>(a, lg, vcol, cand, s_piv, s_done, folded2)
-                             : small_qr<kSmallRows>(a, lg, vcol, cand, s_piv, s_done, folded2);
+  const int steps = rows <= 4 ? small_qr<4>(a, lg, vcol, cand, s_piv, s_done, s_stop, folded2)
+                : rows <= 8  ? small_qr<8>(a, lg, vcol, cand, s_piv, s_done, s_stop, folded2)
+                : rows <= 16 ? small_qr<16>(a, lg, vcol, cand, s_piv, s_done, s_stop, folded2)
+                : rows <= 24 ? small_qr<24>(a, lg, vcol, cand, s_piv, s_done, s_stop, folded2)
+                : rows <= 32 ? small_qr<32>(a, lg, vcol, cand, s_piv, s_done, s_stop, folded2)
+                             : small_qr<kSmallRows>(a, lg, vcol, cand, s_piv, s_done, s_stop, folded2);
   PHASE(13);
   const int r = __builtin_amdgcn_readfirstlane(steps);
   if (r == 0) {
