@@ -912,7 +912,7 @@ struct Workspace {
   // the stop summary goes to rank->out_h when the learned form is on.
   int qrcp_run(int m, int n, const int* max_steps, int start, double drop_abs2, float* ms,
                bool stop_at_mark = false) {
-    const int nblk = qr_natural_grid(n);
+    const int nblk = qr_natural_grid(m, n);
     QrcpArgs qa = qr_prepare(m, n, nblk);
     qa.max_steps = max_steps;
     qa.start = start;
@@ -1137,9 +1137,14 @@ struct Workspace {
   // workgroup per CU: every workgroup reads all posts of a step, and a
   // wavefront's only column stays in its registers. A step at 380 x 108 takes
   // 7.0 us with the 27 workgroups of four columns, 7.6 with 108 of one and 9.2
-  // with 14 of eight.
-  int qr_natural_grid(int n) const {
-    return std::max(1, std::min({(n + 3) / 4, qr_blocks, num_cus}));
+  // with 14 of eight. Far beyond the 1024 rows that the registers hold a column is
+  // read and written every step, by its wavefront alone, and the posts weigh less:
+  // there a column to a workgroup, while there are compute units for all (4000 x
+  // 100: 2.35 ms, 2.44 with four to a workgroup; 8000 x 64 2.80 and 3.01; 9216 x 128
+  // 6.35 and 6.81; but 2652 x 200 3.60 and 3.52, 4000 x 600 15.1 and 14.8).
+  int qr_natural_grid(int m, int n) const {
+    const int cols = m >= 3000 && n <= num_cus ? 1 : 4;
+    return std::max(1, std::min({(n + cols - 1) / cols, qr_blocks, num_cus}));
   }
   static int qr_min_grid(int n) { return std::max(1, (n + kQrcpMaxLocal - 1) / kQrcpMaxLocal); }
 
@@ -1673,7 +1678,7 @@ struct Batcher {
     for (auto& ch : chunks(qrs, cap, ming)) {
       std::vector<int> nat, mn;
       for (size_t i = ch.first; i < ch.second; ++i) {
-        nat.push_back(qrs[i]->ws->qr_natural_grid(qrs[i]->n));
+        nat.push_back(qrs[i]->ws->qr_natural_grid(qrs[i]->m, qrs[i]->n));
         mn.push_back(Workspace::qr_min_grid(qrs[i]->n));
       }
       const std::vector<int> alloc = allocate(nat, mn, cap);
