@@ -878,7 +878,7 @@ struct Workspace {
     trunc_extra2 = folded ? rank->out_d : nullptr;
     int k;
     try {
-      k = gram_ok(r) ? svd_gram(n, r) : svd(n, r);
+      k = gram_ok(n, r) ? svd_gram(n, r) : svd(n, r);
     } catch (...) {
       trunc_extra2 = nullptr;
       throw;
@@ -1097,11 +1097,18 @@ struct Workspace {
     HIP_CHECK(hipGetLastError());
   }
 
-  // Y of at most kGramMaxRank columns, from a pivoted QR (the method relies
-  // on its graded rows); beyond, G does not fit one workgroup. Both sides at
-  // ranks 64 to 126 of the TEMPO and PT-TEMPO runs: 0.41 ms on average here,
-  // 0.9 ms in the blocked Jacobi.
-  bool gram_ok(int r) const { return small_enabled && r <= kGramMaxRank; }
+  // After the grid's QR: the Gram Jacobi, whose single workgroup forms G, against
+  // the blocked Jacobi on the whole card. Both sides in ms, Y of n rows and rank r:
+  //   r    n = 130        300        600        1024       2048
+  //   24   0.13 0.21  0.14 0.21  0.15 0.21  0.21 0.22  0.28 0.27
+  //   64   0.43 0.57  0.46 0.52  0.58 0.60  0.70 0.59  1.03 0.69
+  //   96   0.88 0.97  0.83 1.00  1.06 1.00  1.33 1.04  1.96 1.30
+  //   112  1.16 1.45  1.26 1.42  1.40 1.54  1.75 1.60  3.54 1.95
+  //   126  1.64 1.45  1.76 1.46  2.14 1.56  2.57 1.63  3.38 1.97
+  // (the blocked one without its four clearing and three finishing launches).
+  bool gram_ok(int n, int r) const {
+    return small_enabled && r <= kGramGridRank && n <= kGramGridRows;
+  }
 
   GramSvdArgs gram_prepare(int n, int r, SvdInfo* copy) {
     ensure_sv((size_t)r);
@@ -1289,7 +1296,7 @@ struct Workspace {
 // arrive serves all requests at once on the batch stream: one launch for the
 // SVDs done by one workgroup each (small_svd_batch_kernel), one cooperative
 // launch of qrcp_batch_kernel for the pivoted QRs of the others, one launch
-// for the Gram Jacobi of those of rank up to kGramMaxRank and one of
+// for the Gram Jacobi of those within its range (gram_ok) and one of
 // jacobi_batch_kernel for the rest, each workgroup of a cooperative launch
 // working on one request with that request's own barrier counter. Requests that do not fit
 // the co-resident grid together go into several launches.
@@ -1596,7 +1603,7 @@ struct Batcher {
     gram_launch(gs, base + st.passes);
   }
 
-  // Y of at most kGramMaxRank columns: as run_small, after run_qr
+  // Y in the range of gram_ok: as run_small, after run_qr
   void run_gram(std::vector<SvdRequest*>& rs, std::vector<SvdRequest*>* blocked) {
     ensure_gather(rs.size());
     std::vector<GramSvdArgs> args;
@@ -1867,7 +1874,7 @@ struct Batcher {
     if (!qrs.empty()) run_qr(qrs);
     for (auto* r : batch) {
       if (r->failed || (r->qr && r->ws->small_ok(r->m, r->n))) continue;
-      if (r->qr && r->ws->gram_ok(r->jn)) gr.push_back(r);
+      if (r->qr && r->ws->gram_ok(r->jm, r->jn)) gr.push_back(r);
       else jr.push_back(r);
     }
     if (!gr.empty()) run_gram(gr, &jr);

@@ -180,6 +180,8 @@ struct GramReplayArgs {
 constexpr int kGramMaxRank = 126;           // G in LDS, two blocks of it per thread
 constexpr int kGramMaxSweeps = 20;          // sweeps of a pass, all in the rotation log
 constexpr int kGramMaxPasses = 6;           // passes, the last one rotating nothing
+constexpr int kGramGridRank = 112;          // after the grid's QR: largest rank
+constexpr int kGramGridRows = 512;          // and rows of Y (see gram_ok)
 constexpr int kSmallMaxCols = kGramMaxRank; // columns of M in small_svd_kernel
 constexpr int kSmallThreads = 512;          // its workgroup
 constexpr int kGramThreads = 1024;          // workgroup of gram_svd_kernel

@@ -1,5 +1,6 @@
 """Truncated SVDs on both sides of the lines between the kernels' ranges (needs
-a GPU), against LAPACK: the workgroups of the grid's QR for tall matrices."""
+a GPU), against LAPACK: the workgroups of the grid's QR for tall matrices, and
+the Jacobi that follows it."""
 
 import numpy as np
 import pytest
@@ -13,13 +14,17 @@ EPSREL = 1e-9
 # a column to a workgroup from 3000 rows on, up to as many columns as compute units
 TALL = [(2999, 9), (3000, 9), (3000, 1), (3000, 256), (3000, 257), (9216, 3)]
 
+# ranks up to 112 of Y = R^H with up to 512 rows by the Gram Jacobi, others blocked
+JACOBI = [(112, 512), (113, 512), (112, 513), (400, 112), (400, 113), (3, 512), (3, 513),
+          (1, 513), (126, 2000)]
+
 
 def _unitary(rng, m, r):
     a = rng.normal(size=(m, r)) + 1j * rng.normal(size=(m, r))
     return np.linalg.qr(a)[0]
 
 
-@pytest.mark.parametrize("m,n", TALL)
+@pytest.mark.parametrize("m,n", TALL + JACOBI)
 def test_routes(m, n):
     print(f"[gpu-case] svd route {m}x{n}", flush=True)
     rng = np.random.default_rng([m, n])
