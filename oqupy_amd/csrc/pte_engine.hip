@@ -809,6 +809,15 @@ struct Workspace {
     qr_cap = c;
   }
 
+  // The one-workgroup SVD neither caps nor records, so the forms that predict a
+  // rank, and the log of any form, leave it the matrices of up to 96 columns and
+  // 159 KiB (their histories have always begun beyond that) and take the
+  // grid's QR beyond.
+  bool rank_keeps(int m, int n) const {
+    return (rank->mode != 3 || rank->rec_cap > 0) &&
+           (n > 96 || (size_t)m * n * 16 + (size_t)n * 64 > kSmallLdsMax);
+  }
+
   // Truncated SVD of M (m x n, column-major in Q, ld = m, m <= kQrMaxRows):
   // pivoted QR  M P = Q R  (stopped once the unfactored block is below
   // eps * ||M||_F, r steps), then the Jacobi SVD of Y = R^H (n x r) in X,
@@ -827,8 +836,9 @@ struct Workspace {
   // (mode 3 stops there without a prediction).
   int svd_qrcp(int m, int n, int key = -1) {
     if (batcher) return batched_svd(true, m, n);
-    if (small_ok(m, n)) {
-      const bool adaptive = rank != nullptr && key >= 0 && rank->mode == 3;
+    const bool learn = rank != nullptr && key >= 0;
+    if (small_ok(m, n) && !(learn && rank_keeps(m, n))) {
+      const bool adaptive = learn && rank->mode == 3;
       const int k = svd_small(m, n, adaptive);
       if (adaptive) {
         rank->svds += 1;
@@ -837,7 +847,6 @@ struct Workspace {
       }
       return k;
     }
-    const bool learn = rank != nullptr && key >= 0;
     const bool capped = learn && rank->mode > 0;
     const RankQuery q = learn ? rank->query(key, m, n, (float)epsrel) : RankQuery();
     if (capped && rank->mode != 3) {
