@@ -726,8 +726,9 @@ struct Workspace {
   }
 
   // after synchronisation: checks, statistics, kept rank
-  // `small`: the SVD ran in small_svd_kernel (its time is kept apart from
-  // the Jacobi kernel's statistics)
+  // `small`: the Jacobi ran in one workgroup, in small_svd_kernel or after the
+  // grid's QR in gram_svd_kernel (its time is kept apart from the Jacobi kernel's
+  // statistics)
   int jacobi_check(int m, int n, float ms, bool small = false) {
     require(info_h->sweeps > 0, PTE_ERR_NUMERIC,
             "Jacobi SVD did not converge (" + std::to_string(m) + "x" +

@@ -185,7 +185,10 @@ constexpr int kGramGridRows = 512;          // and rows of Y (see gram_ok)
 constexpr int kSmallMaxCols = kGramMaxRank; // columns of M in small_svd_kernel
 constexpr int kSmallThreads = 512;          // its workgroup
 constexpr int kGramThreads = 1024;          // workgroup of gram_svd_kernel
-constexpr int kGramSmallRank = 88;          // ranks small_svd_kernel finishes itself
+// Ranks whose first pass small_svd_kernel does itself: two blocks of G a thread hold
+// no more. (A round takes 0.64 us with its 512 threads at rank 35, 0.68 with 1024;
+// 0.96 and 0.92 at rank 74, where another launch would cost more than that gives.)
+constexpr int kGramSmallRank = 88;
 constexpr int kSmallRows = 38;              // rows of M a lane holds at most (no scratch)
 constexpr size_t kSmallQrLds = 64 * kSmallRows * 16 + 2048;   // LDS of its QR
 // lanes per column of small_svd_kernel's QR

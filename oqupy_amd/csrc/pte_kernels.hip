@@ -5,8 +5,12 @@
 //  * mpo_apply_kernel  applies one influence node W[w,p,s,v] to the GEMM result
 //                      G[(l,p),(x,v)] and writes the SVD input matrix or a site
 //  * jacobi_kernel     blocked one-sided Jacobi SVD (Hestenes) of a column-major
-//                      matrix, one workgroup per block pair and round, grid
-//                      barriers between rounds (cooperative launch)
+//                      matrix, one workgroup per row slice of a block pair and
+//                      round; a pair waits for its two blocks' last rotation, the
+//                      grid only between sweeps (cooperative launch)
+//  * small_svd_kernel / gram_svd_kernel / gram_replay_kernel
+//                      SVDs of ranks up to 126 by a Jacobi on the Gram matrix in
+//                      one workgroup
 //  * column_norm_kernel / rank_sort_kernel / truncate_kernel
 //                      singular values, descending order, epsrel cut
 //  * emit kernels      new sites, carries and S V^H rows from the Jacobi output
@@ -648,11 +652,6 @@ __device__ __forceinline__ double dpp_keep_d(double old, double v) {
       __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, 0xf, 0xf, false),
       __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, 0xf, 0xf, false));
 }
-template <int CTRL>
-__device__ __forceinline__ double2 dpp_row2(double2 v) {
-  return make_double2(dpp_d<CTRL>(v.x), dpp_d<CTRL>(v.y));
-}
-
 // The sweeps; W (row-major, by column) goes to Ws, whose memory is the second
 // buffer until then. rc and rs have two buffers of PP entries.
 __device__ __forceinline__ void pair_sweeps(double2* Gp, double* rc, double2* rs,
@@ -964,7 +963,7 @@ __device__ __forceinline__ void jacobi_body(const JacobiArgs& a, const int bid,
         PHASE(1);
         RTRACE(3);
         // identical summation order (slice 0, 1, ...) in every workgroup of
-        // the pair; loads of eight slices are in flight together
+        // the pair; loads of kJacobiSumBatch slices are in flight together
         constexpr int SB = kJacobiSumBatch;
         double2 acc[4];
 #pragma unroll
