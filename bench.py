@@ -43,9 +43,9 @@ PHASE_STEPS = {"c2": 40, "c3": 0, "c5": 0}
 # what the counters read for a plain copy (keyed by config, precision, rank
 # form, phase steps, warm-up, timed steps)
 TRAFFIC = {
-    # FETCH_SIZE 2720739.2 KiB x 2.000 + WRITE_SIZE 2205739.9 KiB x 1.000 per
-    # Jacobi dispatch, mean over the window's 3286 dispatches
-    ("c2", "c128", "exact", 40, 5, 20): 7830751514,
+    # FETCH_SIZE 2308486.1 KiB x 2.000 + WRITE_SIZE 1868655.3 KiB x 1.000 per
+    # Jacobi dispatch, mean over the window's 3900 dispatches
+    ("c2", "c128", "exact", 40, 5, 20): 6641282549,
 }
 TRAFFIC_SOURCE = "profiles/hbm_traffic_svd_kernels_pt_tempo_dkmax200_steps47-66.md"
 

@@ -1582,9 +1582,9 @@ emit_kernel(EmitArgs a) {
 // A post is of 8-byte words that each carry the step's tag, so reading the
 // posts is the waiting: no arrival counter stands between them (two dependent
 // atomics and a separate read of the candidates less). A step at 380 x 108 takes
-// 7.0 us on 27 workgroups (8.8 with the counters; 1.5 forming the reflector, 1.3
+// 7.2 us on 27 workgroups (8.8 with the counters; 1.5 forming the reflector, 1.3
 // updating the columns, 2.3 until their stores are acknowledged, 1.7 waiting for
-// the posts), at 996 x 860 8.8 us on 215 (10.1). The posts are double-buffered by step parity: a workgroup
+// the posts), at 996 x 860 9.0 us on 215 (9.9). The posts are double-buffered by step parity: a workgroup
 // posts step j + 2 after reading all posts of step j + 1, which were made after
 // their workgroups had read step j's. They are zeroed before the launch (no
 // step has tag 0).
@@ -2172,9 +2172,9 @@ build_rh_batch_kernel(const RhArgs* pa) {
 // phase of g_ab.
 // Bound by the chain of a round in one compute unit: LDS reads, about 60
 // dependent FP64 operations of a rotation, the blocks' 48 each, LDS writes.
-// Y of 100 columns on average (TEMPO, bonds of about a hundred): 0.41 ms
-// against 0.9 ms of jacobi_tile_kernel; 88 x 83 matrix in small_svd_kernel:
-// 0.82 ms against 1.83 ms with the one-sided sweeps in LDS, QR included.
+// 88 x 83 matrix in small_svd_kernel, QR included: 0.78 ms, the replay 0.06, the
+// check 0.025, against 1.83 ms with one-sided sweeps in LDS. (Against
+// jacobi_tile_kernel after the grid's QR: the host's rule has both sides.)
 // ---------------------------------------------------------------------------
 // 16 x 16 tile t of the upper triangle of Y^H Y (list (0,0), (0,1), (1,1),
 // (0,2), ...) by one wavefront, 3M on the FP64 matrix cores; Y is n x r with
